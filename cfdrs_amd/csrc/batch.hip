@@ -12,10 +12,15 @@
 // ticket per item, exits when the queue is drained).  A system with more
 // than wave_max_rows rows is one item for the whole 256-thread block; smaller
 // systems are grouped four to an item, one per wavefront, and reduce with
-// shuffles only.  Each team keeps the shared vectors of its system (x, p) in
-// LDS and each lane its rows' share of r, z, q and the FP32 correction in
-// registers, so during the iterations global memory serves only the matrix
-// and three per-row inputs.
+// shuffles only.
+//
+// Two kernels share that scheme.  A system whose rows couple to at most
+// kRegOff other nodes (channel junctions of up to four channels) is solved by
+// k_batch_reg: the lane that owns a row keeps its matrix entries, x, r and p
+// in registers, so an iteration touches LDS for the gathers of p and for the
+// reductions only.  Any other system, and the restarted refinement, goes to
+// k_batch: x and p in LDS, r, z and q in registers, the matrix and three
+// per-row inputs read from memory in every iteration.
 #include <algorithm>
 #include <cmath>
 #include <numeric>
@@ -475,8 +480,440 @@ __global__ __launch_bounds__(kBlock) void k_batch(BArgs A) {
   }
 }
 
+// ---- register-resident systems ---------------------------------------------------
+// Bound: the dependent chain of an iteration (one LDS gather pass, two
+// reductions, three barriers), not bytes.  Read from memory, the matrix cost
+// a chain of L2 round trips per product: 8.8 us per iteration of a 2,000-row
+// system with two such systems per CU.  A lane's 8 rows of at most 4
+// off-diagonal entries are 64 + 16 VGPRs of FP64 values and 16 of packed LDS
+// offsets; with x, r, p and the Jacobi factors they fit the 256 VGPRs of two
+// wavefronts per SIMD, the residency k_batch had.  The row count per lane R is
+// a template argument picked per system, so a small system neither loops
+// over nor holds rows it does not have, and all gathers of a product are
+// issued together.  Whole calls, against k_batch on the same systems: 4,096
+// networks of 50-2,000 nodes 26.4 -> 8.0 ms, forward and adjoint of 600
+// networks of 30-700 nodes 6.35 -> 2.58 ms.
+constexpr int kRegOff = 4;  // off-diagonal entries per row
+
+// Team sums with one barrier each: the two reductions of an iteration use
+// different LDS slots, and at least one other barrier lies between two uses
+// of the same slots.
+template <class Team>
+__device__ __forceinline__ double reg_sum(double v, double *sh) {
+  v = wave_sum(v);
+  if constexpr (Team::size == kBlock) {
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = sh[0] + sh[1] + sh[2] + sh[3];
+  }
+  return v;
+}
+template <class Team>
+__device__ __forceinline__ void reg_sum2(double &a, double &b, double *sh) {
+  a = wave_sum(a);
+  b = wave_sum(b);
+  if constexpr (Team::size == kBlock) {
+    if ((threadIdx.x & 63) == 0) {
+      sh[4 + (threadIdx.x >> 6)] = a;
+      sh[8 + (threadIdx.x >> 6)] = b;
+    }
+    __syncthreads();
+    a = sh[4] + sh[5] + sh[6] + sh[7];
+    b = sh[8] + sh[9] + sh[10] + sh[11];
+  }
+}
+
+// The lane's R rows (tl, tl + size, ...): diagonal, off-diagonal entries in
+// column order with the LDS byte offsets of their columns (two 16-bit offsets
+// per register), Jacobi factors.  Rows past the system's end are zero rows,
+// and absent entries are zeros at the row's own column.
+template <class Team, int R, typename T>
+struct RegRows {
+  T d[R], a[R][kRegOff], jd[R];
+  unsigned c[R][kRegOff / 2];
+  __device__ __forceinline__ void load(const BArgs &A, const T *vals, const T *jdv, int r0, int n, int tl) {
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const int i = tl + j * Team::size;
+      const bool own = i < n;
+      const int row = r0 + (own ? i : 0);
+      const int kb = A.rp[row], len = own ? A.rp[row + 1] - kb : 0;
+      T v[kRegOff + 1];
+      int col[kRegOff + 1];
+      int dpos = kRegOff + 1;
+#pragma unroll
+      for (int k = 0; k <= kRegOff; ++k) {
+        const bool ok = k < len;
+        const int e = ok ? kb + k : kb;
+        v[k] = ok ? vals[e] : T(0);
+        col[k] = ok ? A.ci[e] - r0 : (own ? i : 0);
+        if (ok && col[k] == i) dpos = k;
+      }
+      d[j] = T(0);
+#pragma unroll
+      for (int k = 0; k <= kRegOff; ++k)
+        if (dpos == k) d[j] = v[k];
+      unsigned o[kRegOff];
+#pragma unroll
+      for (int k = 0; k < kRegOff; ++k) {
+        a[j][k] = dpos > k ? v[k] : v[k + 1];
+        o[k] = (unsigned)((dpos > k ? col[k] : col[k + 1]) * (int)sizeof(T));
+      }
+#pragma unroll
+      for (int k = 0; k < kRegOff / 2; ++k) c[j][k] = o[2 * k] | o[2 * k + 1] << 16;
+      jd[j] = own ? jdv[row] : T(0);
+      // one row's loads at a time: all rows in flight would spill
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  // q = A v over the lane's rows: v in LDS, the lane's own entries of v in own
+  __device__ __forceinline__ void product(const T *v, const T (&own)[R], T (&q)[R]) const {
+    const char *base = reinterpret_cast<const char *>(v);
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      T g[kRegOff];
+#pragma unroll
+      for (int k = 0; k < kRegOff; ++k)
+        g[k] = *reinterpret_cast<const T *>(base + ((k & 1) ? c[j][k / 2] >> 16 : c[j][k / 2] & 0xffffu));
+      T s = d[j] * own[j];
+#pragma unroll
+      for (int k = 0; k < kRegOff; ++k) s += a[j][k] * g[k];
+      q[j] = s;
+    }
+  }
+};
+
+// Jacobi-PCG in FP64 with the matrix in registers: the recurrence of team_cg
+// and the FP64 branch of solve_system.  Where the Jacobi and equilibration
+// factors of every row are equal (the diagonal is the row's largest entry, as
+// in every network Laplacian), the equilibrated residual is z = D^-1 r.
+template <class Team, int R>
+__device__ __forceinline__ void reg_solve64(const BArgs &A, int r0, int n, int tl, double *ps, double *sh, double thr2,
+                                            double &rn0, double &rr, int &iters, int &term) {
+  RegRows<Team, R, double> M;
+  M.load(A, A.v64, A.jd64, r0, n, tl);
+  double x[R], r[R], p[R], q[R];
+  bool same = true;
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const int i = tl + j * Team::size;
+    x[j] = i < n ? A.x[r0 + i] : 0.0;
+    if (i < n) same = same && A.eq[r0 + i] == M.jd[j];
+  }
+  if constexpr (Team::size == kBlock) same = __syncthreads_and(same ? 1 : 0) != 0;
+  else same = __all(same ? 1 : 0) != 0;
+  iters = 0;
+  for (bool first = true;; first = false) {
+    // r = b - A x and its equilibrated norm, x gathered through ps
+    Team::sync();  // every lane is done with the previous contents of ps
+#pragma unroll
+    for (int j = 0; j < R; ++j) ps[tl + j * Team::size] = x[j];
+    Team::sync();
+    M.product(ps, x, q);
+    double acc = 0.0;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const int i = tl + j * Team::size;
+      r[j] = i < n ? A.b[r0 + i] - q[j] : 0.0;
+      const double e = (i < n ? A.eq[r0 + i] : 0.0) * r[j];
+      acc += e * e;
+    }
+    rr = reg_sum<Team>(acc, sh);
+    if (first) {
+      rn0 = sqrt(rr);
+      term = CFDLA_TERM_INITIAL_RESIDUAL;
+      if (rr <= thr2) break;
+    } else {
+      if (rr <= thr2) {
+        term = CFDLA_TERM_CONVERGED;
+        break;
+      }
+      if (term != CFDLA_TERM_CONVERGED) break;
+      if (iters >= A.max_it) {
+        term = CFDLA_TERM_MAX_ITERATIONS;
+        break;
+      }
+    }
+    // start (or restart) the recurrence from the explicit residual
+    Team::sync();  // every lane has read x from ps
+    double rz = 0.0;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      p[j] = M.jd[j] * r[j];
+      ps[tl + j * Team::size] = p[j];
+      rz += r[j] * p[j];
+    }
+    rz = reg_sum<Team>(rz, sh);
+    Team::sync();
+    term = CFDLA_TERM_MAX_ITERATIONS;
+    while (iters < A.max_it) {
+      M.product(ps, p, q);
+      double pq = 0.0;
+#pragma unroll
+      for (int j = 0; j < R; ++j) pq += p[j] * q[j];
+      pq = reg_sum<Team>(pq, sh);
+      if (!(pq > 0.0) || !isfinite(pq)) {
+        term = CFDLA_TERM_NONPOSITIVE_CURVATURE;
+        break;
+      }
+      const double alpha = rz / pq;
+      double en = 0.0, rzn = 0.0;
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        x[j] += alpha * p[j];
+        r[j] = r[j] - alpha * q[j];
+        q[j] = M.jd[j] * r[j];  // z
+        en += q[j] * q[j];
+        rzn += r[j] * q[j];
+      }
+      if (!same) {  // the equilibration factors differ from the Jacobi ones
+        en = 0.0;
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+          const int i = tl + j * Team::size;
+          const double e = (i < n ? A.eq[r0 + i] : 0.0) * r[j];
+          en += e * e;
+        }
+      }
+      reg_sum2<Team>(en, rzn, sh);
+      ++iters;
+      if (en <= thr2) {
+        term = CFDLA_TERM_CONVERGED;
+        break;
+      }
+      if (rzn == 0.0 || !isfinite(rzn)) {
+        term = CFDLA_TERM_BREAKDOWN;
+        break;
+      }
+      const double beta = rzn / rz;
+      rz = rzn;
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        p[j] = q[j] + beta * p[j];
+        ps[tl + j * Team::size] = p[j];
+      }
+      Team::sync();
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const int i = tl + j * Team::size;
+    if (i < n) A.x[r0 + i] = x[j];
+  }
+}
+
+// FP32 Jacobi-PCG with reliable FP64 residual replacement, the matrix's FP32
+// values in registers: the recurrence of team_cg_reliable.  The FP64 residual
+// of a replacement reads the FP64 matrix from memory.
+template <class Team, int R>
+__device__ __forceinline__ void reg_solve32(const BArgs &A, int r0, int n, int tl, double *psd, double *sh,
+                                            double thr2, double &rn0, double &rr, int &iters, int &nrep, int &term) {
+  float *ps = reinterpret_cast<float *>(psd);
+  RegRows<Team, R, float> M;
+  M.load(A, A.v32, A.jd32, r0, n, tl);
+  double x[R], r64[R], eq[R];
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const int i = tl + j * Team::size;
+    x[j] = i < n ? A.x[r0 + i] : 0.0;
+    eq[j] = i < n ? A.eq[r0 + i] : 0.0;
+  }
+  enum { kStart, kReplace, kCurvature, kBreakdown, kLimit } why = kStart;
+  float r[R], p[R], q[R], d[R];
+#pragma unroll
+  for (int j = 0; j < R; ++j) d[j] = 0.0f;
+  double sc = 1.0, sc2 = 1.0, thr2s = thr2, ref = 0.0, rz = 0.0, en = 0.0;
+  double d2 = A.delta * A.delta;
+  iters = 0;
+  nrep = -1;  // the initial residual is not a replacement
+  for (;;) {
+    // x += d / sc, d = 0, then the FP64 residual
+    Team::sync();
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      if (why != kStart) x[j] += (double)d[j] / sc;
+      d[j] = 0.0f;
+      psd[tl + j * Team::size] = x[j];
+    }
+    Team::sync();
+    double acc = 0.0;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const int i = tl + j * Team::size;
+      r64[j] = 0.0;
+      if (i < n) {
+        double s = 0.0;
+        for (int k = A.rp[r0 + i]; k < A.rp[r0 + i + 1]; ++k) s += A.v64[k] * psd[A.ci[k] - r0];
+        r64[j] = A.b[r0 + i] - s;
+      }
+      const double e = eq[j] * r64[j];
+      acc += e * e;
+    }
+    rr = reg_sum<Team>(acc, sh);
+    ++nrep;
+    bool restart = false;
+    if (why == kStart) {
+      rn0 = sqrt(rr);
+      term = CFDLA_TERM_INITIAL_RESIDUAL;
+      if (rr <= thr2) break;
+      sc = 1.0 / sqrt(rr);
+      sc2 = sc * sc;
+      thr2s = thr2 * sc2;
+    } else if (why == kReplace) {
+      if (rr <= thr2 || !isfinite(rr)) {
+        term = rr <= thr2 ? CFDLA_TERM_CONVERGED : CFDLA_TERM_BREAKDOWN;
+        break;
+      }
+      restart = rr * sc2 > 4.0 * en;
+      if (restart) d2 = fmin(0.25, d2 * 100.0);
+    } else {
+      term = why == kCurvature ? CFDLA_TERM_NONPOSITIVE_CURVATURE
+             : why == kBreakdown ? CFDLA_TERM_BREAKDOWN
+             : rr <= thr2 ? CFDLA_TERM_CONVERGED : CFDLA_TERM_MAX_ITERATIONS;
+      break;
+    }
+    ref = rr * sc2;
+    // r32 = sc r64, z = D^-1 r32; the direction goes on, or starts again
+    Team::sync();  // every lane has read x from ps, and sh is free
+    double rzn = 0.0;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      r[j] = (float)(r64[j] * sc);
+      q[j] = M.jd[j] * r[j];
+      rzn += (double)r[j] * (double)q[j];
+    }
+    rzn = reg_sum<Team>(rzn, sh);
+    if (why == kReplace && (rzn == 0.0 || !isfinite(rzn))) {
+      why = kBreakdown;
+      continue;
+    }
+    const float b0 = why == kStart || restart ? 0.0f : (float)(rzn / rz);
+    rz = rzn;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      p[j] = why == kStart ? q[j] : q[j] + b0 * p[j];
+      ps[tl + j * Team::size] = p[j];
+    }
+    Team::sync();
+    while (true) {
+      if (iters >= A.max_it) {
+        why = kLimit;
+        break;
+      }
+      M.product(ps, p, q);
+      double pq = 0.0;
+#pragma unroll
+      for (int j = 0; j < R; ++j) pq += (double)p[j] * (double)q[j];
+      pq = reg_sum<Team>(pq, sh);
+      if (!(pq > 0.0) || !isfinite(pq)) {
+        why = kCurvature;
+        break;
+      }
+      const double alpha = rz / pq;
+      en = 0.0;
+      rzn = 0.0;
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        d[j] += (float)alpha * p[j];
+        r[j] = r[j] - (float)alpha * q[j];
+        q[j] = M.jd[j] * r[j];
+        const double e = eq[j] * (double)r[j];
+        en += e * e;
+        rzn += (double)r[j] * (double)q[j];
+      }
+      reg_sum2<Team>(en, rzn, sh);
+      ++iters;
+      if (en <= thr2s || en <= d2 * ref) {
+        why = kReplace;
+        break;
+      }
+      if (rzn == 0.0 || !isfinite(rzn)) {
+        why = kBreakdown;
+        break;
+      }
+      const double beta = rzn / rz;
+      rz = rzn;
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        p[j] = q[j] + (float)beta * p[j];
+        ps[tl + j * Team::size] = p[j];
+      }
+      Team::sync();
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const int i = tl + j * Team::size;
+    if (i < n) A.x[r0 + i] = x[j];
+  }
+}
+
+template <class Team, bool F32>
+__device__ __forceinline__ void solve_system_reg(const BArgs &A, int sys, int tl, double *ps, double *sh) {
+  const int r0 = A.sys_row[sys], n = A.sys_row[sys + 1] - r0;
+  double bb = 0.0;
+  for (int i = tl; i < n; i += Team::size) {
+    const double e = A.eq[r0 + i] * A.b[r0 + i];
+    bb += e * e;
+  }
+  bb = reg_sum<Team>(bb, sh);
+  const double thr = fmax(A.tol_abs, A.tol_rel * sqrt(bb));
+  const double thr2 = thr * thr;
+  double rn0 = 0.0, rr = 0.0;
+  int iters = 0, outer = 0, term = 0;
+  // rows per lane: the same for the whole team
+  const int rows = __builtin_amdgcn_readfirstlane((n + Team::size - 1) / Team::size);
+#define CFDLA_REG(R)                                                                           \
+  do {                                                                                         \
+    if constexpr (F32) reg_solve32<Team, R>(A, r0, n, tl, ps, sh, thr2, rn0, rr, iters, outer, term); \
+    else reg_solve64<Team, R>(A, r0, n, tl, ps, sh, thr2, rn0, rr, iters, term);               \
+  } while (0)
+  if (rows <= 1) CFDLA_REG(1);
+  else if (rows == 2) CFDLA_REG(2);
+  else if (rows <= 4) CFDLA_REG(4);
+  else if (rows <= 6) CFDLA_REG(6);
+  else CFDLA_REG(kRowsPerLane);
+#undef CFDLA_REG
+  if (tl == 0) {
+    BatchReport rep;
+    rep.iterations = iters;
+    rep.outer = outer;
+    rep.rn0 = rn0;
+    rep.rn = sqrt(rr);
+    rep.thr = thr;
+    rep.term = term;
+    rep.pad = F32 ? 1 : 0;  // the report's precision: 0 FP64, 1 FP32-refined
+    A.rep[sys] = rep;
+  }
+}
+
+// 2 wavefronts per SIMD: 256 VGPRs per lane
+template <bool F32>
+__global__ __launch_bounds__(kBlock, 2) void k_batch_reg(BArgs A) {
+  __shared__ double ps[kMaxBatchRows];
+  __shared__ double sh[12];
+  __shared__ int item_sh;
+  const int total = A.n_block_items + A.n_wave_items;
+  while (true) {
+    if (threadIdx.x == 0) item_sh = (int)atomicAdd(A.queue, 1u);
+    __syncthreads();
+    const int item = item_sh;
+    __syncthreads();
+    if (item >= total) break;  // queue drained: every block leaves
+    if (item < A.n_block_items) {
+      solve_system_reg<BlockTeam, F32>(A, A.items[item], threadIdx.x, ps, sh);
+    } else {
+      const int w = threadIdx.x >> 6;
+      const int k = (item - A.n_block_items) * (kBlock / 64) + w;
+      if (k < A.n_wave_sys)
+        solve_system_reg<WaveTeam, F32>(A, A.items[A.n_block_items + k], threadIdx.x & 63, ps + w * kWaveSlice, sh);
+    }
+    __syncthreads();
+  }
+}
+
 __global__ void k_reset_queue(unsigned *q) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *q = 0u;
+  if (threadIdx.x < 2 && blockIdx.x == 0) q[threadIdx.x] = 0u;
 }
 
 }  // namespace
@@ -496,24 +933,41 @@ void BatchSolver::build(const NetworkInput &in) {
   for (int64_t s = 0; s < nsys; ++s)
     CFDLA_REQUIRE(in.node_off[s + 1] - in.node_off[s] <= kMaxBatchRows, CFDLA_ERR_CONFIG,
                   "batched networks are limited to 2048 nodes each; solve larger ones with cfdla_solve");
+  // systems every row of which has at most kRegOff off-diagonal entries
+  fits_reg.assign((size_t)nsys, 1);
+  for (int64_t s = 0; s < nsys; ++s)
+    for (int64_t i = sys_row[(size_t)s]; i < sys_row[(size_t)s + 1] && fits_reg[(size_t)s]; ++i) {
+      int64_t off = 0;
+      for (int64_t k = host.rp[(size_t)i]; k < host.rp[(size_t)i + 1]; ++k) off += host.ci[(size_t)k] != i;
+      if (off > kRegOff) fits_reg[(size_t)s] = 0;
+    }
   on_device = false;
 }
 
 void BatchSolver::make_items() {
   const int wm = std::min(std::max(sched.wave_max_rows, 0), kWaveSlice);
-  std::vector<int32_t> big, small;
-  for (int64_t s = 0; s < nsys; ++s) (sys_row[s + 1] - sys_row[s] > wm ? big : small).push_back((int32_t)s);
   auto by_size = [&](int32_t a, int32_t b) {
     const int na = sys_row[a + 1] - sys_row[a], nb = sys_row[b + 1] - sys_row[b];
     return na != nb ? na > nb : a < b;
   };
-  std::sort(big.begin(), big.end(), by_size);
-  std::sort(small.begin(), small.end(), by_size);
-  std::vector<int32_t> items(big);
-  items.insert(items.end(), small.begin(), small.end());
-  n_block_items = (int)big.size();
-  n_wave_sys = (int)small.size();
-  n_wave_items = (n_wave_sys + kBlock / 64 - 1) / (kBlock / 64);
+  // all systems for k_batch, then those that fit k_batch_reg and the others
+  std::vector<int32_t> items;
+  for (int list = 0; list < 3; ++list) {
+    std::vector<int32_t> big, small;
+    for (int64_t s = 0; s < nsys; ++s) {
+      if (list > 0 && (fits_reg[(size_t)s] != 0) != (list == 1)) continue;
+      (sys_row[s + 1] - sys_row[s] > wm ? big : small).push_back((int32_t)s);
+    }
+    std::sort(big.begin(), big.end(), by_size);
+    std::sort(small.begin(), small.end(), by_size);
+    BatchItems &l = lists[list];
+    l.first = (int)items.size();
+    l.n_block_items = (int)big.size();
+    l.n_wave_sys = (int)small.size();
+    l.n_wave_items = (l.n_wave_sys + kBlock / 64 - 1) / (kBlock / 64);
+    items.insert(items.end(), big.begin(), big.end());
+    items.insert(items.end(), small.begin(), small.end());
+  }
   if (items.empty()) items.push_back(0);
   d_items.upload(items.data(), items.size());
   sync_stream();
@@ -548,7 +1002,7 @@ void BatchSolver::upload() {
   d_eq.upload(eq.data(), N);
   d_jd32.upload(jd32.data(), N);
   d_rep.ensure((size_t)std::max<int64_t>(1, nsys));
-  d_queue.ensure(1);
+  d_queue.ensure(2);
   d_slot_off.upload(plan.slot_off.data(), plan.slot_off.size());
   d_slot_src.upload(plan.slot_src.data(), std::max<size_t>(1, plan.slot_src.size()));
   d_rhs_off.upload(plan.rhs_off.data(), plan.rhs_off.size());
@@ -565,7 +1019,7 @@ void BatchSolver::upload() {
 
 namespace {
 // ---- scratch of the allocation-free batched solve ---------------------------
-// One 256-byte slot for the work-queue counter, then report staging for at
+// One 256-byte slot for the two work-queue counters, then report staging for at
 // most kNoAllocMaxSystems systems: 256 + 16384 x 48 bytes (768.25 KiB), held
 // by every GPU the library runs on until the process ends.  Host code reaches
 // it only through the address hipGetSymbolAddress returns for the current
@@ -611,11 +1065,6 @@ void BatchSolver::launch(double *x, const cfdla_solver_config &cfg, const double
   a.jd32 = d_jd32.p;
   a.x = x;
   a.rep = rep;
-  a.items = d_items.p;
-  a.queue = queue;
-  a.n_block_items = n_block_items;
-  a.n_wave_items = n_wave_items;
-  a.n_wave_sys = n_wave_sys;
   a.tol_abs = cfg.tol_abs;
   a.tol_rel = cfg.tol_rel;
   a.inner_tol = cfg.inner_tol > 0.0 ? cfg.inner_tol : 1e-5;
@@ -628,7 +1077,24 @@ void BatchSolver::launch(double *x, const cfdla_solver_config &cfg, const double
   a.delta = cfg.reliable_delta > 0.0 ? cfg.reliable_delta : 1e-1;
   const int grid = std::max(1, sched.blocks_per_cu) * num_cus();
   hipLaunchKernelGGL(k_reset_queue, dim3(1), dim3(64), 0, stream(), queue);
-  hipLaunchKernelGGL(k_batch, dim3(grid), dim3(kBlock), 0, stream(), a);
+  auto run = [&](int list, int slot) {
+    const BatchItems &l = lists[list];
+    if (l.n_block_items + l.n_wave_items == 0) return;
+    a.items = d_items.p + l.first;
+    a.queue = queue + slot;
+    a.n_block_items = l.n_block_items;
+    a.n_wave_items = l.n_wave_items;
+    a.n_wave_sys = l.n_wave_sys;
+    if (list != 1) hipLaunchKernelGGL(k_batch, dim3(grid), dim3(kBlock), 0, stream(), a);
+    else if (a.refined) hipLaunchKernelGGL((k_batch_reg<true>), dim3(grid), dim3(kBlock), 0, stream(), a);
+    else hipLaunchKernelGGL((k_batch_reg<false>), dim3(grid), dim3(kBlock), 0, stream(), a);
+  };
+  if (a.refined && !a.reliable) {
+    run(0, 0);  // restarted refinement
+  } else {
+    run(1, 0);
+    run(2, 1);
+  }
   CFDLA_HIP(hipGetLastError());
 }
 
@@ -656,7 +1122,7 @@ void BatchSolver::solve_noalloc(double *x, const cfdla_solver_config &cfg, Batch
   CFDLA_REQUIRE(p != nullptr, CFDLA_ERR_DEVICE, "allocation-free solve scratch not resolved on this device");
   unsigned *queue = static_cast<unsigned *>(p);
   BatchReport *rep = reinterpret_cast<BatchReport *>(static_cast<unsigned char *>(p) + kNoAllocQueueBytes);
-  launch(x, cfg, rhs_dev, queue, rep);  // k_reset_queue clears the counter the previous call left
+  launch(x, cfg, rhs_dev, queue, rep);  // k_reset_queue clears the counters the previous call left
   if (reports) {
     CFDLA_HIP(hipMemcpyAsync(reports, rep, (size_t)nsys * sizeof(BatchReport), hipMemcpyDeviceToHost, stream()));
   }

@@ -79,6 +79,11 @@ struct BatchReport {
   int32_t term, pad;  // pad: the precision the solve ran in (cfdla_report.precision)
 };
 
+// One queue of a batch: positions in d_items, the block-team systems first.
+struct BatchItems {
+  int first = 0, n_block_items = 0, n_wave_items = 0, n_wave_sys = 0;
+};
+
 struct BatchSolver {
   int64_t nsys = 0, nrows = 0;
   HostCsr host;
@@ -100,7 +105,8 @@ struct BatchSolver {
   DevBuf<double> d_dirval, d_neumann;
   bool device_newer = false;  // values / rhs were re-formed on the device since the last host assembly
   DevBuf<unsigned> d_queue;
-  int n_block_items = 0, n_wave_items = 0, n_wave_sys = 0;
+  std::vector<uint8_t> fits_reg;  // per system: solved with its matrix in registers
+  BatchItems lists[3];            // all systems; those of fits_reg; the others
   void build(const NetworkInput &in);
   void upload();
   void make_items();
