@@ -906,6 +906,7 @@ void AmgPrecond::upload() {
   const size_t L = host.levels.size();
   lv.clear();
   lv.resize(L);
+  std::vector<std::vector<int32_t>> gs_order(L), gs_off(L);
   for (size_t l = 0; l < L; ++l) {
     HostLevel &h = host.levels[l];
     DevLevel &d = lv[l];
@@ -919,6 +920,8 @@ void AmgPrecond::upload() {
       std::vector<int32_t> colour, order;
       greedy_colouring(h.A, colour, d.gs_off, order);
       d.gs_perm.upload(order.data(), std::max<size_t>(1, order.size()));
+      gs_order[l] = std::move(order);
+      gs_off[l] = d.gs_off;
     }
     size_t n = (size_t)h.A.n;
     if (l > 0) {
@@ -936,6 +939,11 @@ void AmgPrecond::upload() {
                   "AMG coarsest level too large for the dense direct solve; raise max_levels");
     std::vector<double> inv = dense_inverse(host.levels.back().A);
     coarse_inv.upload(inv.data(), inv.size());
+  }
+  tail = GsTail{};
+  if (cfg.smoother != 2) {
+    const int first = gs_tail_first(host, gs_order, gs_off, cfg.coarse_solver == 1);
+    if (first >= 0) tail.build(host, first, gs_order, gs_off);
   }
   sync_stream();
   on_device = true;
@@ -1072,6 +1080,7 @@ void AmgPrecond::update_values_device(const double *fine_values) {
     refresh_level(c.A, host.levels[l + 1].A, true);
   }
   if (fused.level >= 0) refresh_fused_device();
+  if (tail.level >= 0) tail.refresh(lv);
   if (cfg.coarse_solver == 1) {
     const DevCsr &cA = lv.back().A;
     dense_inverse_device(coarse_n, cA.rp.p, cA.ci.p, cA.v64.p, coarse_inv.p);
@@ -1120,7 +1129,10 @@ void AmgPrecond::vcycle_gs(int l, const T *b, T *x, Scal *s, bool chk, int dot_o
   RedWs &ws = ctx().ws;
   const int n = L.A.n;
   const bool coarsest = (size_t)l + 1 == lv.size();
-  if (coarsest && cfg.coarse_solver == 1) {
+  if (l == tail.level) {
+    gs_tail<T>(tail, b, x, cfg.relaxation_factor, cfg.pre_smooth_iterations, cfg.post_smooth_iterations,
+               cfg.smoother == 1, cfg.coarse_solver == 1 ? coarse_inv.p : nullptr, s, chk);
+  } else if (coarsest && cfg.coarse_solver == 1) {
     dense_gemv<T>(n, coarse_inv.p, b, x, s, chk);
   } else {
     // amg.rs:423-503 from the zero guess (amg.rs:553): pre-smoothing, and on

@@ -126,6 +126,61 @@ struct FusedOp {
   bool plans = false;
 };
 
+// The small levels of a Gauss-Seidel hierarchy, run by one workgroup
+// (gs_tail.hip): per level the rows grouped by colour (position order) with
+// their off-diagonal entries, the diagonal in position order, P, and R with
+// its rows in the coarse level's position order.  Rows are padded in groups
+// of 4 to the longest of their colour (of P, of R).
+struct TailLevelDev {
+  int n, nc, slots, pw, rw;
+  int meta;                        // the level's first colour in the meta data
+  int iv, id, ib, ix, icol, irow;  // inner levels: places in LDS
+  const uint16_t *row, *col, *pcol, *rcol;
+  const double *v64, *d64, *p64, *r64;
+  const float *v32, *d32, *p32, *r32;
+  double *b64, *x64;  // right-hand side (position order) and iterate
+  float *b32, *x32;
+};
+struct TailLevel {
+  int slots = 0;
+  DevBuf<int32_t> src, dsrc;  // CSR slot of every entry and diagonal (-1: none)
+  DevBuf<uint16_t> row, col, pcol, rcol;
+  DevBuf<double> v64, d64, p64, r64, b64, x64;
+  DevBuf<float> v32, d32, p32, r32, b32, x32;
+};
+// Colours of all tail levels together (their meta data is held in LDS), and
+// the LDS left beside it.
+constexpr int kTailColours = 192;
+constexpr int kTailLds = 160 * 1024 - kTailColours * 16;
+// Rows of a tail level: two FP64 vectors in LDS, each with a zero behind it.
+constexpr int kTailRows = kTailLds / 16 - 1;
+// Entries per colour up to which one workgroup's sweep beats a launch per
+// colour: 0.5 us and 0.125 us per 1,000 entries (2.9 us for 19,000 of a
+// 7,680-row level) against 4.7 us per k_gs_colour launch.
+constexpr int64_t kTailNnzPerColour = 32000;
+// Rows of a dense coarsest level that one workgroup multiplies in a few us.
+constexpr int kTailDenseRows = 256;
+struct GsTail {
+  int level = -1;  // first level of the tail (-1: none)
+  int cap = 0;     // the most rows of its levels
+  int inner = 0;   // first level (of lv) with its entries in LDS
+  int icap = 0, itotal = 0, lds_vals = 0, lds_words = 0, ncolours = 0;
+  std::vector<TailLevel> lv;
+  DevBuf<TailLevelDev> d_desc;
+  DevBuf<int32_t> d_meta;  // 4 per colour: first position, rows, first slot, slots per row
+  void build(const HostHierarchy &h, int first, const std::vector<std::vector<int32_t>> &order,
+             const std::vector<std::vector<int32_t>> &off);
+  // entries and diagonals from the levels' device values
+  void refresh(const std::vector<DevLevel> &dev);
+};
+int gs_tail_first(const HostHierarchy &h, const std::vector<std::vector<int32_t>> &order,
+                  const std::vector<std::vector<int32_t>> &off, bool direct);
+// x = V-cycle(b) over the tail's levels; inv: dense inverse of the coarsest
+// level, or null for the reference's sweeps there.
+template <typename T>
+void gs_tail(const GsTail &t, const T *b, T *x, double omega, int pre, int post, bool symmetric, const double *inv,
+             Scal *s, bool check_done);
+
 // C = A B on the device (galerkin.hip), bit-identical to csr_multiply: C's
 // row pointers, columns and values, and the per-slot plan of the product.
 // A is nr rows (int32 CSR), B has ncols columns.
@@ -148,6 +203,7 @@ struct AmgPrecond : Precond {
   // from zero, residual and restriction as one product when the smoother is
   // Jacobi with two pre-sweeps (level -1: none).
   FusedOp fused;
+  GsTail tail;  // the small levels of a Gauss-Seidel hierarchy
   bool build_fused(size_t l);
   void refresh_fused_device();
   // AlgebraicMultigrid::recompute (amg.rs:179-214) on the device from
