@@ -17,6 +17,7 @@
 // b % 8), so the x gathers of neighbouring rows hit the L2 of the XCD that
 // owns them.
 #include "epilogue.hpp"
+#include "finalize.hpp"
 #include "internal.hpp"
 #include "reduce.hpp"
 
@@ -32,32 +33,43 @@ __device__ __forceinline__ void keep_direction(int n, const T *__restrict__ p, T
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) pn[i] = p[i];
 }
 
-template <typename T, int EPI, bool DOT, bool SYM, int ND>
+// CONS: the reduction before this product is still pending (finalize.hpp).
+// Every load of the block's tile is issued, then the block sums the partials
+// and advances the scalars while they are in flight; one tile per block.
+template <typename T, int EPI, bool DOT, bool SYM, int ND, bool CONS>
 __global__ __launch_bounds__(kBlock) void k_dia(int n, DiaDesc dd, const T *__restrict__ dv,
                                                 const T *__restrict__ x, const T *__restrict__ b,
                                                 const T *__restrict__ dinv, T omega, T *y, const T *dotw, Scal *s,
-                                                int check_done, double *partials, T *y2) {
-  if (check_done && s->done) {
-    if constexpr (EPI == EPI_DIR) keep_direction(n, x, y2);
-    return;
+                                                int check_done, double *partials, T *y2, Pend pd) {
+  if constexpr (!CONS) {
+    if (check_done && s->done) {
+      if constexpr (EPI == EPI_DIR) keep_direction(n, x, y2);
+      return;
+    }
+    if constexpr (EPI == EPI_DIR) omega = (T)s->beta;
   }
-  if constexpr (EPI == EPI_DIR) omega = (T)s->beta;
   // entries per row in column order: SYM lower k = ND-1..1, main, upper k = 1..ND-1
   constexpr int NS = SYM ? 2 * ND - 1 : ND;
   const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3, per = gridDim.x >> 3;
   const int tiles = (n + kBlock - 1) / kBlock;
   const int chunk = (tiles + 7) >> 3;
   const int t1 = min(tiles, xcd * chunk + chunk);
-  double dacc = 0.0;
+  double dacc[EPI == EPI_DOT2 ? 2 : 1] = {};
   for (int t = xcd * chunk + local; t < t1; t += per) {
-    const int row = t * kBlock + (int)threadIdx.x;
-    if (row >= n) continue;
-    const EpiIn<T> e = epi_load<T, EPI, DOT>(row, x, b, dinv, omega, y, dotw);
+    const int mine = t * kBlock + (int)threadIdx.x;
+    const bool live = mine < n;
+    if constexpr (!CONS) {
+      if (!live) continue;
+    }
+    const int row = CONS && !live ? n - 1 : mine;
+    EpiIn<T> e = epi_load<T, EPI, DOT>(row, x, b, dinv, omega, y, dotw);
+    T ou = T(0), ow = T(0);  // the row's own direction operands
+    if constexpr (CONS && EPI == EPI_DIR) gather_raw<T, EPI>(row, x, b, dinv, ou, ow);
     // Branch-free: every value and gather load is issued before the sums;
     // an out-of-range column re-reads row's own slot and is masked.
     int c[NS];
     bool ok[NS];
-    T v[NS], xv[NS];
+    T v[NS], gu[NS], gw[NS];
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
       const bool lower = SYM && j < ND - 1;
@@ -68,16 +80,30 @@ __global__ __launch_bounds__(kBlock) void k_dia(int n, DiaDesc dd, const T *__re
       v[j] = dv[k * n + (lower && ok[j] ? col : row)];
     }
 #pragma unroll
-    for (int j = 0; j < NS; ++j) xv[j] = gather<T, EPI>(c[j], x, b, dinv, omega);
+    for (int j = 0; j < NS; ++j) gather_raw<T, EPI>(c[j], x, b, dinv, gu[j], gw[j]);
+    if constexpr (CONS) {
+      __shared__ Scal sc;
+      consume(pd, sc);
+      if (check_done && sc.done) {
+        if constexpr (EPI == EPI_DIR) keep_direction(n, x, y2);
+        return;
+      }
+      if constexpr (EPI == EPI_DIR) {
+        omega = (T)sc.beta;
+        e.x = gather_combine<T, EPI>(ou, ow, omega);
+      }
+    }
     T sum = T(0);
 #pragma unroll
-    for (int j = 0; j < NS; ++j) sum += (ok[j] && v[j] != T(0)) ? v[j] * xv[j] : T(0);
-    epi_store<T, EPI, DOT>(e, row, sum, omega, y, dotw, dacc, y2);
+    for (int j = 0; j < NS; ++j)
+      sum += (ok[j] && v[j] != T(0)) ? v[j] * gather_combine<T, EPI>(gu[j], gw[j], omega) : T(0);
+    if (live) {
+      epi_store<T, EPI, DOT>(e, row, sum, omega, y, dotw, dacc[0], y2);
+      if constexpr (EPI == EPI_DOT2) dacc[1] += (double)sum * (double)sum;
+    }
+    if constexpr (CONS) break;
   }
-  if constexpr (DOT) {
-    double d1[1] = {dacc};
-    block_partials<1>(d1, partials);
-  }
+  if constexpr (DOT) block_partials<EPI == EPI_DOT2 ? 2 : 1>(dacc, partials);
 }
 
 // ---- R rows per lane, 16-byte loads ------------------------------------------
@@ -100,47 +126,44 @@ __device__ __forceinline__ void ldv(const T *p, T (&o)[R]) {
   for (int r = 0; r < R; ++r) o[r] = v[r];
 }
 
-// gathered operands at the R aligned columns c..c+R-1
+// loaded operands of the gathers at the R aligned columns c..c+R-1 (gather_raw)
 template <typename T, int EPI, int R>
 __device__ __forceinline__ void gatherv(int c, const T *__restrict__ x, const T *__restrict__ b,
-                                        const T *__restrict__ dinv, T omega, T (&o)[R]) {
+                                        const T *__restrict__ dinv, T (&u)[R], T (&w)[R]) {
   if constexpr (EPI == EPI_JACOBI0) {
-    T dd[R], bb[R];
-    ldv<T, R>(dinv + c, dd);
-    ldv<T, R>(b + c, bb);
-#pragma unroll
-    for (int r = 0; r < R; ++r) o[r] = omega * dd[r] * bb[r];
-  } else if constexpr (EPI == EPI_DIR) {
-    T pp[R], zz[R];
-    ldv<T, R>(x + c, pp);
-    ldv<T, R>(b + c, zz);
-#pragma unroll
-    for (int r = 0; r < R; ++r) o[r] = cg_dir(omega, pp[r], zz[r]);
+    ldv<T, R>(dinv + c, u);
+    ldv<T, R>(b + c, w);
   } else {
-    ldv<T, R>(x + c, o);
+    ldv<T, R>(x + c, u);
+    if constexpr (EPI == EPI_DIR) ldv<T, R>(b + c, w);
   }
 }
 
-template <typename T, int EPI, bool DOT, int ND, int R>
+template <typename T, int EPI, bool DOT, int ND, int R, bool CONS>
 __global__ __launch_bounds__(kBlock) void k_dia_vec(int n, DiaDesc dd, const T *__restrict__ dv,
                                                     const T *__restrict__ x, const T *__restrict__ b,
                                                     const T *__restrict__ dinv, T omega, T *y, const T *dotw,
-                                                    Scal *s, int check_done, double *partials, T *y2) {
-  if (check_done && s->done) {
-    if constexpr (EPI == EPI_DIR) keep_direction(n, x, y2);
-    return;
+                                                    Scal *s, int check_done, double *partials, T *y2, Pend pd) {
+  if constexpr (!CONS) {
+    if (check_done && s->done) {
+      if constexpr (EPI == EPI_DIR) keep_direction(n, x, y2);
+      return;
+    }
+    if constexpr (EPI == EPI_DIR) omega = (T)s->beta;
   }
-  if constexpr (EPI == EPI_DIR) omega = (T)s->beta;
   const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3, per = gridDim.x >> 3;
   const int groups = n / R;
   const int tiles = (groups + kBlock - 1) / kBlock;
   const int chunk = (tiles + 7) >> 3;
   const int t1 = min(tiles, xcd * chunk + chunk);
-  double dacc = 0.0;
+  double dacc[EPI == EPI_DOT2 ? 2 : 1] = {};
   for (int t = xcd * chunk + local; t < t1; t += per) {
     const int g = t * kBlock + (int)threadIdx.x;
-    if (g >= groups) continue;
-    const int row = g * R;
+    const bool live = g < groups;
+    if constexpr (!CONS) {
+      if (!live) continue;
+    }
+    const int row = (CONS && !live ? groups - 1 : g) * R;
     // epilogue operands, then every entry and gather load before the sums
     EpiIn<T> e[R];
     {
@@ -171,15 +194,12 @@ __global__ __launch_bounds__(kBlock) void k_dia_vec(int n, DiaDesc dd, const T *
       }
     }
     // main diagonal and the operand at the lane's own columns
-    T vm[R], xm[R];
+    // (loads only; the gathered operands are combined below, once omega is known)
+    T vm[R], mu[R], mw[R];
     ldv<T, R>(dv + row, vm);
-    gatherv<T, EPI, R>(row, x, b, dinv, omega, xm);
-    if constexpr (EPI == EPI_DIR) {
-#pragma unroll
-      for (int r = 0; r < R; ++r) e[r].x = xm[r];  // the direction at the lane's own rows
-    }
+    gatherv<T, EPI, R>(row, x, b, dinv, mu, mw);
     // off-diagonals: lower (column row + r - off) and upper (row + r + off)
-    T vl[ND][R], xl[ND][R], vu[ND][R], xu[ND][R];
+    T vl[ND][R], lu[ND][R], lw[ND][R], vu[ND][R], uu[ND][R], uw[ND][R];
     bool okl[ND][R], oku[ND][R];
 #pragma unroll
     for (int k = 1; k < ND; ++k) {
@@ -190,22 +210,20 @@ __global__ __launch_bounds__(kBlock) void k_dia_vec(int n, DiaDesc dd, const T *
         // inner neighbours come from the lane's own vectors
         const bool okf = row > 0, okb = row + R < n;
         const T vfirst = dk[okf ? row - 1 : row];
-        const T xfirst = gather<T, EPI>(okf ? row - 1 : row, x, b, dinv, omega);
-        const T xlast = gather<T, EPI>(okb ? row + R : row, x, b, dinv, omega);
+        gather_raw<T, EPI>(okf ? row - 1 : row, x, b, dinv, lu[k][0], lw[k][0]);
+        gather_raw<T, EPI>(okb ? row + R : row, x, b, dinv, uu[k][R - 1], uw[k][R - 1]);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
           vl[k][r] = r == 0 ? vfirst : vu[k][r - 1];
-          xl[k][r] = r == 0 ? xfirst : xm[r - 1];
           okl[k][r] = r > 0 || okf;
-          xu[k][r] = r == R - 1 ? xlast : xm[r + 1];
           oku[k][r] = r < R - 1 || okb;
         }
       } else {
         // whole vectors are in or out of range (row, off and n are multiples of R)
         const bool okL = row - off >= 0, okU = row + off < n;
         ldv<T, R>(dk + (okL ? row - off : row), vl[k]);
-        gatherv<T, EPI, R>(okL ? row - off : row, x, b, dinv, omega, xl[k]);
-        gatherv<T, EPI, R>(okU ? row + off : row, x, b, dinv, omega, xu[k]);
+        gatherv<T, EPI, R>(okL ? row - off : row, x, b, dinv, lu[k], lw[k]);
+        gatherv<T, EPI, R>(okU ? row + off : row, x, b, dinv, uu[k], uw[k]);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
           okl[k][r] = okL;
@@ -213,6 +231,28 @@ __global__ __launch_bounds__(kBlock) void k_dia_vec(int n, DiaDesc dd, const T *
         }
       }
     }
+    if constexpr (CONS) {
+      __shared__ Scal sc;
+      consume(pd, sc);
+      if (check_done && sc.done) {
+        if constexpr (EPI == EPI_DIR) keep_direction(n, x, y2);
+        return;
+      }
+      if constexpr (EPI == EPI_DIR) omega = (T)sc.beta;
+    }
+    T xm[R], xl[ND][R], xu[ND][R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      xm[r] = gather_combine<T, EPI>(mu[r], mw[r], omega);
+      if constexpr (EPI == EPI_DIR) e[r].x = xm[r];  // the direction at the lane's own rows
+    }
+#pragma unroll
+    for (int k = 1; k < ND; ++k)
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        xl[k][r] = k == 1 && r > 0 ? xm[r - 1] : gather_combine<T, EPI>(lu[k][r], lw[k][r], omega);
+        xu[k][r] = k == 1 && r < R - 1 ? xm[r + 1] : gather_combine<T, EPI>(uu[k][r], uw[k][r], omega);
+      }
     T out[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -226,8 +266,14 @@ __global__ __launch_bounds__(kBlock) void k_dia_vec(int n, DiaDesc dd, const T *
       for (int k = 1; k < ND; ++k)
         sum += (oku[k][r] && vu[k][r] != T(0)) ? vu[k][r] * xu[k][r] : T(0);
       out[r] = epi_out<T, EPI>(e[r], sum, omega);
-      if constexpr (DOT) dacc += (double)(EPI == EPI_DIR ? e[r].x : (dotw == y ? out[r] : e[r].w)) * (double)out[r];
+      if constexpr (DOT) {
+        if (live) {
+          dacc[0] += (double)(EPI == EPI_DIR ? e[r].x : (dotw == y ? out[r] : e[r].w)) * (double)out[r];
+          if constexpr (EPI == EPI_DOT2) dacc[1] += (double)out[r] * (double)out[r];
+        }
+      }
     }
+    if (CONS && !live) break;
     vec_t<T, R> ov;
 #pragma unroll
     for (int r = 0; r < R; ++r) ov[r] = out[r];
@@ -238,25 +284,54 @@ __global__ __launch_bounds__(kBlock) void k_dia_vec(int n, DiaDesc dd, const T *
       for (int r = 0; r < R; ++r) pv[r] = e[r].x;
       *reinterpret_cast<vec_t<T, R> *>(y2 + row) = pv;
     }
+    if constexpr (CONS) break;
   }
-  if constexpr (DOT) {
-    double d1[1] = {dacc};
-    block_partials<1>(d1, partials);
-  }
+  if constexpr (DOT) block_partials<EPI == EPI_DOT2 ? 2 : 1>(dacc, partials);
 }
+
+// Products that follow a reduction within an iteration take it along while it
+// is pending: the CG direction, the first product of a V-cycle, BiCGSTAB's
+// second product.
+template <int EPI>
+constexpr bool consumes() { return EPI == EPI_DIR || EPI == EPI_JACOBI0 || EPI == EPI_DOT2; }
 
 template <typename T, int EPI, bool DOT, bool SYM, int ND>
 void launch_shape(const DevCsr &A, int blocks, const T *x, const T *b, const T *dinv, double omega, T *y,
                   const T *dotw, Scal *s, bool check_done, RedWs &ws, T *y2) {
-  hipLaunchKernelGGL((k_dia<T, EPI, DOT, SYM, ND>), dim3(blocks), dim3(kBlock), 0, stream(), A.n, A.dia_desc,
-                     A.dia_vals<T>(), x, b, dinv, (T)omega, y, dotw, s, check_done ? 1 : 0, ws.partials.p, y2);
+  double *part = DOT ? nullptr : ws.partials.p;
+  if constexpr (consumes<EPI>()) {
+    if (pending_on(s) && blocks <= kConsumeBlocks) {
+      const Pend pd = take_pending(s);
+      if (DOT) part = ws.next();
+      hipLaunchKernelGGL((k_dia<T, EPI, DOT, SYM, ND, true>), dim3(blocks), dim3(kBlock), 0, stream(), A.n, A.dia_desc,
+                         A.dia_vals<T>(), x, b, dinv, (T)omega, y, dotw, pd.out, check_done ? 1 : 0, part, y2, pd);
+      return;
+    }
+  }
+  s = settled_scal(s);
+  if (DOT) part = ws.next();
+  hipLaunchKernelGGL((k_dia<T, EPI, DOT, SYM, ND, false>), dim3(blocks), dim3(kBlock), 0, stream(), A.n, A.dia_desc,
+                     A.dia_vals<T>(), x, b, dinv, (T)omega, y, dotw, s, check_done ? 1 : 0, part, y2, Pend{});
 }
 
 template <typename T, int EPI, bool DOT, int ND, int R>
 void launch_vec(const DevCsr &A, const T *x, const T *b, const T *dinv, double omega, T *y, const T *dotw,
                 Scal *s, bool check_done, RedWs &ws, int blocks, T *y2) {
-  hipLaunchKernelGGL((k_dia_vec<T, EPI, DOT, ND, R>), dim3(blocks), dim3(kBlock), 0, stream(), A.n, A.dia_desc,
-                     A.dia_vals<T>(), x, b, dinv, (T)omega, y, dotw, s, check_done ? 1 : 0, ws.partials.p, y2);
+  double *part = DOT ? nullptr : ws.partials.p;
+  if constexpr (consumes<EPI>()) {
+    if (pending_on(s) && blocks <= kConsumeBlocks) {
+      const Pend pd = take_pending(s);
+      if (DOT) part = ws.next();
+      hipLaunchKernelGGL((k_dia_vec<T, EPI, DOT, ND, R, true>), dim3(blocks), dim3(kBlock), 0, stream(), A.n,
+                         A.dia_desc, A.dia_vals<T>(), x, b, dinv, (T)omega, y, dotw, pd.out, check_done ? 1 : 0, part,
+                         y2, pd);
+      return;
+    }
+  }
+  s = settled_scal(s);
+  if (DOT) part = ws.next();
+  hipLaunchKernelGGL((k_dia_vec<T, EPI, DOT, ND, R, false>), dim3(blocks), dim3(kBlock), 0, stream(), A.n, A.dia_desc,
+                     A.dia_vals<T>(), x, b, dinv, (T)omega, y, dotw, s, check_done ? 1 : 0, part, y2, Pend{});
 }
 
 bool aligned(const void *p, size_t bytes) { return (reinterpret_cast<uintptr_t>(p) & (bytes - 1)) == 0; }
@@ -309,7 +384,7 @@ void launch_dia(const DevCsr &A, const T *x, const T *b, const T *dinv, double o
         case 3: launch_vec<T, EPI, DOT, 3, R>(A, x, b, dinv, omega, y, dotw, s, check_done, ws, vblocks, y2); break;
         default: launch_vec<T, EPI, DOT, 4, R>(A, x, b, dinv, omega, y, dotw, s, check_done, ws, vblocks, y2); break;
       }
-      if (DOT) finish(1, s, op, vblocks, ws, check_done);
+      if (DOT) finish(EPI == EPI_DOT2 ? 2 : 1, s, op, vblocks, ws, check_done);
       return;
     }
   }
@@ -333,7 +408,7 @@ void launch_dia(const DevCsr &A, const T *x, const T *b, const T *dinv, double o
     }
   }
 #undef CFDLA_DIA
-  if (DOT) finish(1, s, op, blocks, ws, check_done);
+  if (DOT) finish(EPI == EPI_DOT2 ? 2 : 1, s, op, blocks, ws, check_done);
 }
 
 #define CFDLA_DIA_INST(T, E)                                                                                   \
@@ -348,7 +423,9 @@ void launch_dia(const DevCsr &A, const T *x, const T *b, const T *dinv, double o
   CFDLA_DIA_INST(T, EPI_ADD)     \
   CFDLA_DIA_INST(T, EPI_JACOBI0) \
   template void launch_dia<T, EPI_DIR, true>(const DevCsr &, const T *, const T *, const T *, double, T *, const T *, \
-                                             Scal *, bool, int, RedWs &, T *);
+                                             Scal *, bool, int, RedWs &, T *);                                   \
+  template void launch_dia<T, EPI_DOT2, true>(const DevCsr &, const T *, const T *, const T *, double, T *, const T *, \
+                                              Scal *, bool, int, RedWs &, T *);
 CFDLA_DIA_ALL(double)
 CFDLA_DIA_ALL(float)
 

@@ -48,7 +48,7 @@ __device__ __forceinline__ EpiIn<T> epi_load(int row, const T *__restrict__ x, c
 // The value an epilogue writes for row sum `sum`.
 template <typename T, int EPI>
 __device__ __forceinline__ T epi_out(const EpiIn<T> &e, T sum, T omega) {
-  if constexpr (EPI == EPI_Y || EPI == EPI_RJ0 || EPI == EPI_DIR) return sum;
+  if constexpr (EPI == EPI_Y || EPI == EPI_RJ0 || EPI == EPI_DIR || EPI == EPI_DOT2) return sum;
   else if constexpr (EPI == EPI_RESID) return e.b - sum;
   else if constexpr (EPI == EPI_JACOBI || EPI == EPI_JACOBI0) return e.x + omega * e.d * (e.b - sum);
   else return e.y + sum;
@@ -76,6 +76,27 @@ __device__ __forceinline__ T gather(int c, const T *__restrict__ x, const T *__r
   if constexpr (EPI == EPI_JACOBI0) return omega * dinv[c] * b[c];
   else if constexpr (EPI == EPI_DIR) return cg_dir(omega, x[c], b[c]);
   else return x[c];
+}
+
+// The same in two steps, for a kernel that learns omega after its loads: the
+// loaded operands (u, and w where the epilogue combines two) and their
+// combination.
+template <typename T, int EPI>
+__device__ __forceinline__ void gather_raw(int c, const T *__restrict__ x, const T *__restrict__ b,
+                                           const T *__restrict__ dinv, T &u, T &w) {
+  if constexpr (EPI == EPI_JACOBI0) {
+    u = dinv[c];
+    w = b[c];
+  } else {
+    u = x[c];
+    w = EPI == EPI_DIR ? b[c] : T(0);
+  }
+}
+template <typename T, int EPI>
+__device__ __forceinline__ T gather_combine(T u, T w, T omega) {
+  if constexpr (EPI == EPI_JACOBI0) return omega * u * w;
+  else if constexpr (EPI == EPI_DIR) return cg_dir(omega, u, w);
+  else return u;
 }
 
 

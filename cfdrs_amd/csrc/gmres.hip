@@ -255,6 +255,9 @@ SolveOut gmres(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int64_
   const int nb = std::min(kMdotBlocks, blocks_for(n, kBlock * 4));
   int64_t enq = 0;
   while (true) {
+    // the residual's read left no reduction pending, and the cycle's kernels
+    // start none: the scalars stay where they are until its end
+    s = settled_scal(s);
     hipLaunchKernelGGL((k_gm_restart<T>), dim3(eb), dim3(kBlock), 0, stream(), n, r, beta, V, s, L);
     int steps = (int)std::min<int64_t>(m, max_it - enq);
     for (int j = 0; j < steps; ++j) {

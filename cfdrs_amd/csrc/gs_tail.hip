@@ -586,6 +586,7 @@ void gs_tail(const GsTail &t, const T *b, T *x, double omega, int pre, int post,
   // larger levels' two vectors
   const size_t bytes = std::max((size_t)t.lds_vals * sizeof(T),
                                 (2 * ((size_t)t.icap + 1) + t.itotal) * sizeof(T) + (size_t)t.lds_words * sizeof(uint16_t));
+  s = settled_scal(s);
   hipLaunchKernelGGL((k_gs_tail<T>), dim3(1), dim3(kTailThreads), bytes, stream(), t.d_desc.p, (int)t.lv.size(),
                      t.inner, t.cap, t.icap, t.itotal, reinterpret_cast<const int4 *>(t.d_meta.p), t.ncolours, b, x,
                      (T)omega, pre, post, symmetric ? 1 : 0, inv, s, check_done ? 1 : 0);

@@ -289,18 +289,42 @@ struct Scal {
   int32_t pad;
 };
 
-// Per-stream reduction workspace: block partials and an arrival counter that
-// the last block resets, so the workspace needs no clearing between kernels.
+// Reduction workspace: two sets of block partials used in turn, so a kernel
+// that still sums one reduction's partials can write its own.
 struct RedWs {
   DevBuf<double> partials;
-  DevBuf<unsigned> counter;
+  int cur = 0;
   void init();
+  double *current() const;  // the set the latest reducing kernel writes
+  double *next() {          // the set for the next reducing kernel
+    cur ^= 1;
+    return current();
+  }
 };
 
 constexpr int kBlock = 256;
 constexpr int kMaxBlocks = 8192;  // capacity of the block partials (grid of any reducing kernel)
 constexpr int kGridCap = 2048;    // grid of the grid-stride vector and row-block kernels
 constexpr int kMaxRed = 8;
+inline double *RedWs::current() const { return partials.p + (size_t)cur * kMaxRed * kMaxBlocks; }
+
+// A reduction whose partials are written and whose finalize op has not run:
+// the next kernel that depends on it sums them itself (finalize.hpp).
+// Up to kConsumeBlocks partials: 4 loads per thread of every consuming block.
+constexpr int kConsumeBlocks = 1024;
+struct Pend {
+  int nblocks;  // 0: nothing pending
+  int nv, op, check_done;
+  const double *partials;
+  const Scal *in;
+  Scal *out;
+};
+constexpr int kScalSlots = 4;  // solve slots; slot i's twin is slot i + kScalSlots
+Scal *live_scal(Scal *s);
+void flush_pending();
+Scal *settled_scal(Scal *s);
+Pend take_pending(Scal *s);
+bool pending_on(Scal *s);  // take_pending(s) would return a reduction
 
 enum FinalizeOp : int {
   OP_NONE = 0,
@@ -321,7 +345,7 @@ enum FinalizeOp : int {
   OP_BI_RR_RHO = 14,   // BiCGSTAB: OP_BI_RR on red0, then (still running) OP_BI_RHO on red1 = rhat . r
 };
 
-enum Epi : int { EPI_Y = 0, EPI_RESID = 1, EPI_JACOBI = 2, EPI_ADD = 3, EPI_JACOBI0 = 4, EPI_RJ0 = 5, EPI_DIR = 6 };
+enum Epi : int { EPI_Y = 0, EPI_RESID = 1, EPI_JACOBI = 2, EPI_ADD = 3, EPI_JACOBI0 = 4, EPI_RJ0 = 5, EPI_DIR = 6, EPI_DOT2 = 7 };
 
 // ---- kernel launchers (kernels.hip) -------------------------------------
 // Diagonal-format product with epilogue (dia.hip); A.dia must hold and the
@@ -330,8 +354,9 @@ bool dia_supported(const DiaDesc &d);
 template <typename T, int EPI, bool DOT>
 void launch_dia(const DevCsr &A, const T *x, const T *b, const T *dinv, double omega, T *y, const T *dotw,
                 Scal *s, bool check_done, int op, RedWs &ws, T *y2 = nullptr);
-// Single-block kernel that sums the block partials of a reducing kernel and
-// runs the finalize op (kernels.hip).
+// Leaves the reduction whose partials (ws.current()) a kernel has just written
+// pending, or runs its finalize op in a single-block kernel when it has too
+// many partials (kernels.hip).
 void finish(int nv, Scal *s, int op, int nblocks, RedWs &ws, bool check_done);
 int xcd_grid(int units, int units_per_block, int cap = kGridCap);
 
@@ -390,6 +415,7 @@ void dense_inverse_device(int n, const int32_t *rp, const int32_t *ci, const dou
 //               fly at every gathered column, as k_cg_direction forms it
 //               (x = the previous direction, b = z, beta = s->beta; omega
 //               unused); y = A p, y2 = p, and the dot reduces p . y
+//   EPI_DOT2    y = A x and the two dots dotw . y and y . y
 // When dot_op != OP_NONE, also reduces sum_i dotw_i * y_i (dotw defaults to
 // x when null) and runs dot_op.  Skipped entirely when *s->done != 0 and
 // check_done is set.
@@ -443,10 +469,12 @@ template <typename T>
 void dense_gemv(int n, const double *ainv, const T *b, T *x, Scal *s, bool check_done, int parts = 1);
 
 // BiCGSTAB vector kernels
+// p = r + beta (p - omega v); with jd also ph = jd .* p (the Jacobi preconditioner)
 template <typename T>
-void bicg_p_update(int n, const T *r, const T *v, T *p, Scal *s);  // p = r + beta (p - omega v)
+void bicg_p_update(int n, const T *r, const T *v, T *p, Scal *s, const T *jd = nullptr, T *ph = nullptr);
+// s = r - alpha v; ||s||^2; with jd also sh = jd .* s
 template <typename T>
-void bicg_s_update(int n, const T *r, const T *v, T *sv, Scal *s, RedWs &ws);  // s = r - alpha v; ||s||^2
+void bicg_s_update(int n, const T *r, const T *v, T *sv, Scal *s, RedWs &ws, const T *jd = nullptr, T *sh = nullptr);
 // x += alpha ph + omega sh; r = s - omega t; ||r||^2 -> OP_BI_RR.  With rhat
 // non-NULL also rhat . r -> OP_BI_RR_RHO: the next iteration's rho and beta
 // come out of the same finalize.

@@ -10,159 +10,13 @@
 #include <cmath>
 
 #include "epilogue.hpp"
+#include "finalize.hpp"
 #include "internal.hpp"
 #include "reduce.hpp"
+#include "solver.hpp"
 
 namespace cfdla {
 namespace {
-
-__device__ void finalize(Scal *s, int op) {
-  switch (op) {
-    case OP_INIT_RR:
-      s->rr = s->red[0];
-      break;
-    case OP_SET_RZ:
-      s->rz = s->red[0];
-      break;
-    case OP_CG_ALPHA: {
-      double pq = s->red[0];
-      s->pq = pq;
-      if (!(pq > 0.0) || !isfinite(pq)) {
-        s->term = CFDLA_TERM_NONPOSITIVE_CURVATURE;
-        s->done = 2;
-      } else {
-        s->alpha = s->rz / pq;
-      }
-    } break;
-    case OP_CG_RR: {
-      double rr = s->red[0];
-      s->rr = rr;
-      s->iters += 1;
-      if (!isfinite(rr)) {
-        s->term = CFDLA_TERM_BREAKDOWN;
-        s->done = 2;
-      } else if (rr <= s->thr2) {
-        s->done = 1;
-      }
-    } break;
-    case OP_CG_BETA: {
-      double rzn = s->red[0];
-      if (rzn == 0.0 || !isfinite(rzn)) {
-        s->term = CFDLA_TERM_BREAKDOWN;
-        s->done = 2;
-      } else {
-        s->beta = s->restart_dir ? 0.0 : rzn / s->rz;
-        s->restart_dir = 0;
-        s->rz = rzn;
-      }
-    } break;
-    case OP_CG_RR_RZ: {
-      double rr = s->red[0], rzn = s->red[1];
-      s->rr = rr;
-      s->iters += 1;
-      if (!isfinite(rr)) {
-        s->term = CFDLA_TERM_BREAKDOWN;
-        s->done = 2;
-      } else if (rr <= s->thr2) {
-        s->done = 1;
-      } else if (rzn == 0.0 || !isfinite(rzn)) {
-        s->term = CFDLA_TERM_BREAKDOWN;
-        s->done = 2;
-      } else {
-        s->beta = rzn / s->rz;
-        s->rz = rzn;
-      }
-    } break;
-    case OP_BI_RHO: {
-      double rho_new = s->red[0];
-      if (rho_new == 0.0 || !isfinite(rho_new)) {
-        s->term = CFDLA_TERM_BREAKDOWN;
-        s->done = 2;
-      } else {
-        // a residual replacement far from the recurrence restarts p = r
-        s->beta = s->restart_dir ? 0.0 : (rho_new / s->rho) * (s->alpha / s->omega);
-        s->restart_dir = 0;
-        s->rho = rho_new;
-      }
-    } break;
-    case OP_BI_ALPHA: {
-      double rv = s->red[0];
-      if (rv == 0.0 || !isfinite(rv)) {
-        s->term = CFDLA_TERM_BREAKDOWN;
-        s->done = 2;
-      } else {
-        s->alpha = s->rho / rv;
-      }
-    } break;
-    case OP_BI_SNORM: {
-      double ss = s->red[0];
-      s->iters += 1;
-      if (!isfinite(ss)) {
-        s->term = CFDLA_TERM_BREAKDOWN;
-        s->done = 2;
-      } else if (ss <= s->thr2) {
-        s->done = 3;  // x += alpha * phat, then confirm on the host
-      }
-    } break;
-    case OP_BI_OMEGA: {
-      double ts = s->red[0], tt = s->red[1];
-      s->omega = tt > 0.0 ? ts / tt : 0.0;
-    } break;
-    case OP_RELIABLE: {
-      // FP64 residual of the accumulated FP64 solution (reliable-update CG)
-      // A replaced residual far above the recursive one it replaces (the
-      // FP32 operator's rounding caps what one cycle can gain) would make
-      // beta = r.z / rz blow up and wreck the direction: restart it.
-      double rr = s->red[0];
-      const double rec = s->rr;
-      s->rr = rr;
-      s->rr_true = rr;
-      s->nupd += 1;
-      if (!isfinite(rr)) {
-        s->term = CFDLA_TERM_BREAKDOWN;
-        s->done = 2;
-      } else {
-        s->done = rr <= s->thr_final2 ? 4 : 0;
-        s->restart_dir = rr > 4.0 * rec ? 1 : 0;
-        s->nrestart += s->restart_dir;
-      }
-    } break;
-    case OP_BI_RR:
-    case OP_BI_RR_RHO: {
-      double rr = s->red[0];
-      s->rr = rr;
-      if (!isfinite(rr)) {
-        s->term = CFDLA_TERM_BREAKDOWN;
-        s->done = 2;
-      } else if (rr <= s->thr2) {
-        s->done = 1;
-      } else if (s->omega == 0.0 || !isfinite(s->omega)) {
-        s->term = CFDLA_TERM_BREAKDOWN;
-        s->done = 2;
-      } else if (op == OP_BI_RR_RHO) {
-        // the next iteration's OP_BI_RHO, with rho_new = rhat . r
-        double rho_new = s->red[1];
-        if (rho_new == 0.0 || !isfinite(rho_new)) {
-          s->term = CFDLA_TERM_BREAKDOWN;
-          s->done = 2;
-        } else {
-          s->beta = s->restart_dir ? 0.0 : (rho_new / s->rho) * (s->alpha / s->omega);
-          s->restart_dir = 0;
-          s->rho = rho_new;
-        }
-      }
-    } break;
-    default:
-      break;
-  }
-}
-
-// Reducing kernels only write their block partials; the finalize op runs in
-// the single-block k_finalize launched right after them on the same stream.
-template <int NV>
-__device__ __forceinline__ void reduce_and_finalize(double (&v)[NV], Scal *, int, double *partials, unsigned *) {
-  block_partials<NV>(v, partials);
-}
 
 template <int NV>
 __global__ __launch_bounds__(kBlock) void k_finalize(Scal *s, int op, int nblocks, const double *partials,
@@ -179,13 +33,67 @@ __global__ __launch_bounds__(kBlock) void k_finalize(Scal *s, int op, int nblock
 
 }  // namespace
 
-void finish(int nv, Scal *s, int op, int nblocks, RedWs &ws, bool check_done) {
-  if (nv == 1)
-    hipLaunchKernelGGL((k_finalize<1>), dim3(1), dim3(kBlock), 0, stream(), s, op, nblocks, ws.partials.p,
-                       check_done ? 1 : 0);
+// ---- pending reductions ------------------------------------------------------
+// Host side of consume (finalize.hpp).  The scalars of solve slot i live in
+// scal[i] or its twin scal[i + kScalSlots]; a consuming kernel reads one and
+// writes the other.
+Scal *live_scal(Scal *s) {
+  Context &c = ctx();
+  const int i = (int)((s - c.scal.p) % kScalSlots);
+  return c.scal.p + i + kScalSlots * c.twin[i];
+}
+
+void flush_pending() {
+  Context &c = ctx();
+  if (!c.pend.nblocks) return;
+  const Pend p = c.pend;
+  c.pend.nblocks = 0;
+  Scal *s = live_scal(p.out);
+  if (p.nv == 1)
+    hipLaunchKernelGGL((k_finalize<1>), dim3(1), dim3(kBlock), 0, stream(), s, p.op, p.nblocks, p.partials,
+                       p.check_done);
   else
-    hipLaunchKernelGGL((k_finalize<2>), dim3(1), dim3(kBlock), 0, stream(), s, op, nblocks, ws.partials.p,
-                       check_done ? 1 : 0);
+    hipLaunchKernelGGL((k_finalize<2>), dim3(1), dim3(kBlock), 0, stream(), s, p.op, p.nblocks, p.partials,
+                       p.check_done);
+  CFDLA_HIP(hipGetLastError());
+}
+
+// The scalars a kernel works on, with every reduction before it finalized.
+Scal *settled_scal(Scal *s) {
+  flush_pending();
+  return live_scal(s);
+}
+
+// The pending reduction on s for a kernel that consumes it, or none
+// (nblocks = 0) with the settled scalars as in and out.
+Pend take_pending(Scal *s) {
+  Context &c = ctx();
+  const int i = (int)((s - c.scal.p) % kScalSlots);
+  if (!c.pend.nblocks || c.pend.nblocks > kConsumeBlocks || (int)((c.pend.out - c.scal.p) % kScalSlots) != i) {
+    flush_pending();
+    Pend none{};
+    none.in = none.out = live_scal(s);
+    return none;
+  }
+  Pend p = c.pend;
+  c.pend.nblocks = 0;
+  p.in = live_scal(s);
+  c.twin[i] ^= 1;
+  p.out = live_scal(s);
+  return p;
+}
+
+bool pending_on(Scal *s) {
+  Context &c = ctx();
+  return c.pend.nblocks > 0 && c.pend.nblocks <= kConsumeBlocks &&
+         (int)((c.pend.out - c.scal.p) % kScalSlots) == (int)((s - c.scal.p) % kScalSlots);
+}
+
+// A reducing kernel has written its partials (ws.current()).
+void finish(int nv, Scal *s, int op, int nblocks, RedWs &ws, bool check_done) {
+  Context &c = ctx();
+  c.pend = Pend{nblocks, nv, op, check_done ? 1 : 0, ws.current(), nullptr, live_scal(s)};
+  if (nblocks > kConsumeBlocks) flush_pending();
 }
 
 // Grid of a multiple of 8 blocks (one per XCD round-robin), at most cap.
@@ -637,10 +545,11 @@ template <typename T, int EPI, bool DOT, bool C16, bool NT, int LAYOUT>
 void launch_csr_rb_k(const DevCsr &A, int blocks, const T *x, const T *b, const T *dinv, double omega, T *y,
                      const T *dotw, Scal *s, bool check_done, RedWs &ws, T *y2) {
   const int2 *rb = reinterpret_cast<const int2 *>(A.rb<T>());
+  s = settled_scal(s);
   hipLaunchKernelGGL((k_csr_rb<T, EPI, DOT, C16, NT, LAYOUT>), dim3(blocks), dim3(kBlock), 0, stream(), A.nrb<T>(), rb,
                      A.rp.p, C16 ? nullptr : A.rb_cols<T>(), C16 ? A.cols16<T>() : nullptr,
                      C16 ? A.cbase<T>() : nullptr, A.rb_vals<T>(), x, b, dinv, (T)omega, y, dotw, s,
-                     check_done ? 1 : 0, ws.partials.p, y2);
+                     check_done ? 1 : 0, DOT ? ws.next() : ws.partials.p, y2);
 }
 
 template <typename T, int EPI, bool DOT>
@@ -783,6 +692,8 @@ template <typename T, int EPI, bool DOT>
 void launch_sell(const DevCsr &A, const T *x, const T *b, const T *dinv, double omega, T *y, const T *dotw,
                  Scal *s, bool check_done, int op, RedWs &ws) {
   const int cd = check_done ? 1 : 0;
+  s = settled_scal(s);
+  double *part = DOT ? ws.next() : ws.partials.p;
   if (A.sell_group == 4) {
     // 4 wavefronts per slice, one group in flight per step.  On the first
     // AMG level of the 128^3 problem (solves FP64 / FP32-refined, ms): one
@@ -793,7 +704,7 @@ void launch_sell(const DevCsr &A, const T *x, const T *b, const T *dinv, double 
     const int blocks = xcd_grid(A.nslices, (kBlock / 64) / KS, kMaxBlocks);
     hipLaunchKernelGGL((k_sell<T, EPI, DOT, 4, 1, KS>), dim3(blocks), dim3(kBlock), 0, stream(), A.n, A.nslices,
                        A.sell_ptr.p, A.sell_delta.p, A.sell_vals<T>(), x, b, dinv, (T)omega, y, dotw, s, cd,
-                       ws.partials.p);
+                       part);
     if (DOT) finish(1, s, op, blocks, ws, check_done);
   } else {
     // 8 entries per unrolled step: on the first AMG level of the 128^3
@@ -802,7 +713,7 @@ void launch_sell(const DevCsr &A, const T *x, const T *b, const T *dinv, double 
     const int blocks = xcd_grid(A.nslices, kBlock / 64);
     hipLaunchKernelGGL((k_sell<T, EPI, DOT, 1, 8, 1>), dim3(blocks), dim3(kBlock), 0, stream(), A.n, A.nslices,
                        A.sell_ptr.p, A.sell_delta.p, A.sell_vals<T>(), x, b, dinv, (T)omega, y, dotw, s, cd,
-                       ws.partials.p);
+                       part);
     if (DOT) finish(1, s, op, blocks, ws, check_done);
   }
 }
@@ -825,7 +736,7 @@ void launch_csr_e(const DevCsr &A, const T *x, const T *b, const T *dinv, double
 template <typename T, int NV>
 __global__ __launch_bounds__(kBlock) void k_dot(int n, const T *__restrict__ a0, const T *__restrict__ b0,
                                                 const T *__restrict__ a1, const T *__restrict__ b1, Scal *s,
-                                                int check_done, int op, double *partials, unsigned *counter) {
+                                                int check_done, double *partials) {
   if (check_done && s->done) return;
   double v[NV];
 #pragma unroll
@@ -834,7 +745,7 @@ __global__ __launch_bounds__(kBlock) void k_dot(int n, const T *__restrict__ a0,
     v[0] += (double)a0[i] * (double)b0[i];
     if constexpr (NV > 1) v[1] += (double)a1[i] * (double)b1[i];
   }
-  reduce_and_finalize<NV>(v, s, op, partials, counter);
+  block_partials<NV>(v, partials);
 }
 
 template <typename T>
@@ -845,28 +756,69 @@ __global__ __launch_bounds__(kBlock) void k_jacobi_first(int n, const T *__restr
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) x[i] = omega * dinv[i] * b[i];
 }
 
+// ---- vector updates that take a pending reduction along ------------------------
+// Each lane's first kAhead elements (all of them up to 2M rows) are loaded
+// before the block sums the pending partials, so the sum runs in the loads'
+// latency; later elements follow in batches of kAhead.  Elements are visited
+// in the order of a plain grid-stride loop.
+constexpr int kAhead = 4;
+
+// load(u, i) for a batch, then consume, then use(u, i) for it and the batches
+// after it; false, with nothing used, for a stopped solve.
+template <typename Load, typename Use>
+__device__ __forceinline__ bool update_loop(int n, const Pend &pd, Scal &sc, Load &&load, Use &&use) {
+  const int64_t step = (int64_t)gridDim.x * kBlock;
+  const int64_t base = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u)
+    if (base + u * step < n) load(u, (int)(base + u * step));
+  consume(pd, sc);
+  if (sc.done) return false;
+  for (int64_t at = base; at < n; at += kAhead * step) {
+    if (at != base) {
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u)
+        if (at + u * step < n) load(u, (int)(at + u * step));
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+      if (at + u * step < n) use(u, (int)(at + u * step));
+  }
+  return true;
+}
+
 template <typename T, bool JAC>
 __global__ __launch_bounds__(kBlock) void k_cg_update(int n, const T *__restrict__ p, const T *__restrict__ q,
                                                       T *__restrict__ x, T *__restrict__ r,
-                                                      const T *__restrict__ jdinv, T *__restrict__ z, Scal *s,
-                                                      double *partials, unsigned *counter) {
-  if (s->done) return;
-  const T alpha = (T)s->alpha;
-  double v[JAC ? 2 : 1];
-  v[0] = 0.0;
-  if constexpr (JAC) v[1] = 0.0;
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
-    T ri = r[i] - alpha * q[i];
-    x[i] += alpha * p[i];
-    r[i] = ri;
-    v[0] += (double)ri * (double)ri;
-    if constexpr (JAC) {
-      T zi = jdinv[i] * ri;
-      z[i] = zi;
-      v[1] += (double)ri * (double)zi;
-    }
-  }
-  reduce_and_finalize<JAC ? 2 : 1>(v, s, JAC ? OP_CG_RR_RZ : OP_CG_RR, partials, counter);
+                                                      const T *__restrict__ jdinv, T *__restrict__ z, Pend pd,
+                                                      double *partials) {
+  __shared__ Scal sc;
+  T rv[kAhead], qv[kAhead], xv[kAhead], pv[kAhead], jv[kAhead];
+  double v[JAC ? 2 : 1] = {};
+  const bool run = update_loop(
+      n, pd, sc,
+      [&](int u, int i) {
+        rv[u] = r[i];
+        qv[u] = q[i];
+        xv[u] = x[i];
+        pv[u] = p[i];
+        if constexpr (JAC) jv[u] = jdinv[i];
+      },
+      [&](int u, int i) {
+        const T alpha = (T)sc.alpha;
+        const T ri = rv[u] - alpha * qv[u];
+        T xi = xv[u];
+        xi += alpha * pv[u];
+        x[i] = xi;
+        r[i] = ri;
+        v[0] += (double)ri * (double)ri;
+        if constexpr (JAC) {
+          const T zi = jv[u] * ri;
+          z[i] = zi;
+          v[1] += (double)ri * (double)zi;
+        }
+      });
+  if (run) block_partials<JAC ? 2 : 1>(v, partials);
 }
 
 // The FP32 update of a step that replaces the residual, with the correction
@@ -876,29 +828,45 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(int n, const T *__restrict
 // k_fold_correction.
 __global__ __launch_bounds__(kBlock) void k_cg_update_fold(int n, const float *__restrict__ p,
                                                            const float *__restrict__ q, float *__restrict__ xc,
-                                                           double *__restrict__ x64, float *__restrict__ r, Scal *s,
-                                                           double *partials, unsigned *counter) {
-  if (s->done) return;
-  const float alpha = (float)s->alpha;
+                                                           double *__restrict__ x64, float *__restrict__ r, Pend pd,
+                                                           double *partials) {
+  __shared__ Scal sc;
+  float rv[kAhead], qv[kAhead], cv[kAhead], pv[kAhead];
+  double xv[kAhead];
   double v[1] = {0.0};
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
-    float ri = r[i] - alpha * q[i];
-    float ci = xc[i];
-    ci += alpha * p[i];
-    x64[i] += (double)ci;
-    xc[i] = 0.0f;
-    r[i] = ri;
-    v[0] += (double)ri * (double)ri;
-  }
-  reduce_and_finalize<1>(v, s, OP_CG_RR, partials, counter);
+  const bool run = update_loop(
+      n, pd, sc,
+      [&](int u, int i) {
+        rv[u] = r[i];
+        qv[u] = q[i];
+        cv[u] = xc[i];
+        pv[u] = p[i];
+        xv[u] = x64[i];
+      },
+      [&](int u, int i) {
+        const float alpha = (float)sc.alpha;
+        const float ri = rv[u] - alpha * qv[u];
+        float ci = cv[u];
+        ci += alpha * pv[u];
+        x64[i] = xv[u] + (double)ci;
+        xc[i] = 0.0f;
+        r[i] = ri;
+        v[0] += (double)ri * (double)ri;
+      });
+  if (run) block_partials<1>(v, partials);
 }
 
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_cg_direction(int n, const T *__restrict__ z, T *__restrict__ p,
-                                                         Scal *s) {
-  if (s->done) return;
-  const T beta = (T)s->beta;
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) p[i] = cg_dir(beta, p[i], z[i]);
+__global__ __launch_bounds__(kBlock) void k_cg_direction(int n, const T *__restrict__ z, T *__restrict__ p, Pend pd) {
+  __shared__ Scal sc;
+  T zv[kAhead], pv[kAhead];
+  update_loop(
+      n, pd, sc,
+      [&](int u, int i) {
+        zv[u] = z[i];
+        pv[u] = p[i];
+      },
+      [&](int u, int i) { p[i] = cg_dir((T)sc.beta, pv[u], zv[u]); });
 }
 
 template <typename T>
@@ -976,30 +944,51 @@ __global__ __launch_bounds__(kBlock) void k_dense_gemv(int n, const double *__re
   if (lane == 0) x[row] = (T)acc;
 }
 
-// BiCGSTAB: p = r + beta (p - omega v)
-template <typename T>
+// BiCGSTAB: p = r + beta (p - omega v); JAC: ph = jd .* p
+template <typename T, bool JAC>
 __global__ __launch_bounds__(kBlock) void k_bicg_p(int n, const T *__restrict__ r, const T *__restrict__ v,
-                                                   T *__restrict__ p, Scal *s) {
-  if (s->done) return;
-  const T beta = (T)s->beta, omega = (T)s->omega;
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock)
-    p[i] = r[i] + beta * (p[i] - omega * v[i]);
+                                                   T *__restrict__ p, const T *__restrict__ jd, T *__restrict__ ph,
+                                                   Pend pd) {
+  __shared__ Scal sc;
+  T rv[kAhead], vv[kAhead], pv[kAhead], jv[kAhead];
+  update_loop(
+      n, pd, sc,
+      [&](int u, int i) {
+        rv[u] = r[i];
+        vv[u] = v[i];
+        pv[u] = p[i];
+        if constexpr (JAC) jv[u] = jd[i];
+      },
+      [&](int u, int i) {
+        const T beta = (T)sc.beta, omega = (T)sc.omega;
+        const T pi = rv[u] + beta * (pv[u] - omega * vv[u]);
+        p[i] = pi;
+        if constexpr (JAC) ph[i] = jv[u] * pi;
+      });
 }
 
-// BiCGSTAB: s = r - alpha v, ||s||^2
-template <typename T>
+// BiCGSTAB: s = r - alpha v, ||s||^2; JAC: sh = jd .* s
+template <typename T, bool JAC>
 __global__ __launch_bounds__(kBlock) void k_bicg_s(int n, const T *__restrict__ r, const T *__restrict__ v,
-                                                   T *__restrict__ sv, Scal *s, double *partials,
-                                                   unsigned *counter) {
-  if (s->done) return;
-  const T alpha = (T)s->alpha;
+                                                   T *__restrict__ sv, const T *__restrict__ jd, T *__restrict__ sh,
+                                                   Pend pd, double *partials) {
+  __shared__ Scal sc;
+  T rv[kAhead], vv[kAhead], jv[kAhead];
   double acc[1] = {0.0};
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
-    T si = r[i] - alpha * v[i];
-    sv[i] = si;
-    acc[0] += (double)si * (double)si;
-  }
-  reduce_and_finalize<1>(acc, s, OP_BI_SNORM, partials, counter);
+  const bool run = update_loop(
+      n, pd, sc,
+      [&](int u, int i) {
+        rv[u] = r[i];
+        vv[u] = v[i];
+        if constexpr (JAC) jv[u] = jd[i];
+      },
+      [&](int u, int i) {
+        const T si = rv[u] - (T)sc.alpha * vv[u];
+        sv[i] = si;
+        acc[0] += (double)si * (double)si;
+        if constexpr (JAC) sh[i] = jv[u] * si;
+      });
+  if (run) block_partials<1>(acc, partials);
 }
 
 // BiCGSTAB: x += alpha ph + omega sh; r = s - omega t; ||r||^2 (and, with
@@ -1008,18 +997,31 @@ template <typename T, bool RHO>
 __global__ __launch_bounds__(kBlock) void k_bicg_xr(int n, const T *__restrict__ ph, const T *__restrict__ sh,
                                                     const T *__restrict__ sv, const T *__restrict__ t,
                                                     T *__restrict__ x, T *__restrict__ r, const T *__restrict__ rhat,
-                                                    Scal *s, double *partials, unsigned *counter) {
-  if (s->done) return;
-  const T alpha = (T)s->alpha, omega = (T)s->omega;
+                                                    Pend pd, double *partials) {
+  __shared__ Scal sc;
+  T pv[kAhead], hv[kAhead], svv[kAhead], tv[kAhead], xv[kAhead], rh[kAhead];
   double acc[RHO ? 2 : 1] = {};
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
-    x[i] += alpha * ph[i] + omega * sh[i];
-    T ri = sv[i] - omega * t[i];
-    r[i] = ri;
-    acc[0] += (double)ri * (double)ri;
-    if constexpr (RHO) acc[1] += (double)rhat[i] * (double)ri;
-  }
-  reduce_and_finalize<RHO ? 2 : 1>(acc, s, RHO ? OP_BI_RR_RHO : OP_BI_RR, partials, counter);
+  const bool run = update_loop(
+      n, pd, sc,
+      [&](int u, int i) {
+        pv[u] = ph[i];
+        hv[u] = sh[i];
+        svv[u] = sv[i];
+        tv[u] = t[i];
+        xv[u] = x[i];
+        if constexpr (RHO) rh[u] = rhat[i];
+      },
+      [&](int u, int i) {
+        const T alpha = (T)sc.alpha, omega = (T)sc.omega;
+        T xi = xv[u];
+        xi += alpha * pv[u] + omega * hv[u];
+        x[i] = xi;
+        const T ri = svv[u] - omega * tv[u];
+        r[i] = ri;
+        acc[0] += (double)ri * (double)ri;
+        if constexpr (RHO) acc[1] += (double)rh[u] * (double)ri;
+      });
+  if (run) block_partials<RHO ? 2 : 1>(acc, partials);
 }
 
 template <typename T>
@@ -1174,6 +1176,15 @@ void csr_apply(const DevCsr &A, int epi, const T *x, const T *b, const T *dinv, 
                     "direction epilogue takes diagonal storage, z, a second output and a dot");
       launch_dia<T, EPI_DIR, true>(A, x, b, dinv, omega, y, dotw, s, check_done, dot_op, ws, y2);
       break;
+    case EPI_DOT2:
+      CFDLA_REQUIRE(dot, CFDLA_ERR_INVALID_ARG, "the two-dot epilogue takes a dot operation");
+      if (A.dia && A.dia_vals<T>() != nullptr) {
+        launch_dia<T, EPI_DOT2, true>(A, x, b, dinv, omega, y, dotw, s, check_done, dot_op, ws);
+      } else {
+        launch_csr_e<T, EPI_Y, false>(A, x, b, dinv, omega, y, dotw, s, check_done, OP_NONE, ws);
+        dot2<T>(A.n, y, dotw, y, y, s, check_done, dot_op, ws);
+      }
+      break;
     default:
       throw Error(CFDLA_ERR_INVALID_ARG, "unknown CSR epilogue");
   }
@@ -1185,18 +1196,20 @@ template <typename T>
 void dot2(int n, const T *a0, const T *b0, const T *a1, const T *b1, Scal *s, bool check_done, int op,
           RedWs &ws) {
   int blocks = blocks_for(n, kBlock * 4);
+  s = settled_scal(s);
   if (a1)
     hipLaunchKernelGGL((k_dot<T, 2>), dim3(blocks), dim3(kBlock), 0, stream(), n, a0, b0, a1, b1, s,
-                       check_done ? 1 : 0, op, ws.partials.p, ws.counter.p);
+                       check_done ? 1 : 0, ws.next());
   else
     hipLaunchKernelGGL((k_dot<T, 1>), dim3(blocks), dim3(kBlock), 0, stream(), n, a0, b0, a1, b1, s,
-                       check_done ? 1 : 0, op, ws.partials.p, ws.counter.p);
+                       check_done ? 1 : 0, ws.next());
   finish(a1 ? 2 : 1, s, op, blocks, ws, check_done);
   CFDLA_HIP(hipGetLastError());
 }
 
 template <typename T>
 void jacobi_first(int n, const T *dinv, double omega, const T *b, T *x, Scal *s, bool check_done) {
+  s = settled_scal(s);
   hipLaunchKernelGGL((k_jacobi_first<T>), dim3(blocks_for(n, kBlock * 4)), dim3(kBlock), 0, stream(), n, dinv,
                      (T)omega, b, x, s, check_done ? 1 : 0);
   CFDLA_HIP(hipGetLastError());
@@ -1205,32 +1218,35 @@ void jacobi_first(int n, const T *dinv, double omega, const T *b, T *x, Scal *s,
 template <typename T>
 void cg_update(int n, const T *p, const T *q, T *x, T *r, const T *jdinv, T *z, Scal *s, RedWs &ws) {
   int blocks = blocks_for(n, kBlock * 4);
+  const Pend pd = take_pending(s);
   if (jdinv)
-    hipLaunchKernelGGL((k_cg_update<T, true>), dim3(blocks), dim3(kBlock), 0, stream(), n, p, q, x, r, jdinv, z,
-                       s, ws.partials.p, ws.counter.p);
+    hipLaunchKernelGGL((k_cg_update<T, true>), dim3(blocks), dim3(kBlock), 0, stream(), n, p, q, x, r, jdinv, z, pd,
+                       ws.next());
   else
-    hipLaunchKernelGGL((k_cg_update<T, false>), dim3(blocks), dim3(kBlock), 0, stream(), n, p, q, x, r, jdinv,
-                       z, s, ws.partials.p, ws.counter.p);
+    hipLaunchKernelGGL((k_cg_update<T, false>), dim3(blocks), dim3(kBlock), 0, stream(), n, p, q, x, r, jdinv, z, pd,
+                       ws.next());
   finish(jdinv ? 2 : 1, s, jdinv ? OP_CG_RR_RZ : OP_CG_RR, blocks, ws, true);
   CFDLA_HIP(hipGetLastError());
 }
 
 void cg_update_fold(int n, const float *p, const float *q, float *xc, double *x64, float *r, Scal *s, RedWs &ws) {
   const int blocks = blocks_for(n, kBlock * 4);
-  hipLaunchKernelGGL(k_cg_update_fold, dim3(blocks), dim3(kBlock), 0, stream(), n, p, q, xc, x64, r, s,
-                     ws.partials.p, ws.counter.p);
+  const Pend pd = take_pending(s);
+  hipLaunchKernelGGL(k_cg_update_fold, dim3(blocks), dim3(kBlock), 0, stream(), n, p, q, xc, x64, r, pd, ws.next());
   finish(1, s, OP_CG_RR, blocks, ws, true);
   CFDLA_HIP(hipGetLastError());
 }
 
 template <typename T>
 void cg_direction(int n, const T *z, T *p, Scal *s) {
-  hipLaunchKernelGGL((k_cg_direction<T>), dim3(blocks_for(n, kBlock * 4)), dim3(kBlock), 0, stream(), n, z, p, s);
+  const Pend pd = take_pending(s);
+  hipLaunchKernelGGL((k_cg_direction<T>), dim3(blocks_for(n, kBlock * 4)), dim3(kBlock), 0, stream(), n, z, p, pd);
   CFDLA_HIP(hipGetLastError());
 }
 
 template <typename T>
 void copy_vec(int n, const T *src, T *dst, Scal *s, bool check_done) {
+  s = settled_scal(s);
   hipLaunchKernelGGL((k_copy<T>), dim3(blocks_for(n, kBlock * 4)), dim3(kBlock), 0, stream(), n, src, dst, s,
                      check_done ? 1 : 0);
   CFDLA_HIP(hipGetLastError());
@@ -1245,6 +1261,7 @@ __global__ __launch_bounds__(kBlock) void k_zero_chk(int n, T *__restrict__ dst,
 template <typename T>
 void zero_vec(int n, T *dst, Scal *s, bool check_done) {
   if (n == 0) return;
+  s = settled_scal(s);
   hipLaunchKernelGGL((k_zero_chk<T>), dim3(blocks_for(n, kBlock * 4)), dim3(kBlock), 0, stream(), n, dst, s,
                      check_done ? 1 : 0);
 }
@@ -1269,12 +1286,14 @@ void axpy_f32_to_f64(int n, double a, const float *x, double *y) {
 }
 
 void fold_correction(int n, float *xc, double *x, Scal *s, bool check_done) {
+  s = settled_scal(s);
   hipLaunchKernelGGL(k_fold_correction, dim3(blocks_for(n, kBlock * 4)), dim3(kBlock), 0, stream(), n, xc, x, s,
                      check_done ? 1 : 0);
   CFDLA_HIP(hipGetLastError());
 }
 
 void f64_to_f32(int n, const double *src, float *dst, Scal *s, bool check_done) {
+  s = settled_scal(s);
   hipLaunchKernelGGL(k_f64_to_f32, dim3(blocks_for(n, kBlock * 4)), dim3(kBlock), 0, stream(), n, src, dst, s,
                      check_done ? 1 : 0);
   CFDLA_HIP(hipGetLastError());
@@ -1282,6 +1301,7 @@ void f64_to_f32(int n, const double *src, float *dst, Scal *s, bool check_done) 
 
 template <typename T>
 void dense_gemv(int n, const double *ainv, const T *b, T *x, Scal *s, bool check_done, int parts) {
+  s = settled_scal(s);
   int blocks = (int)(((int64_t)n * 64 + kBlock - 1) / kBlock);
   if (blocks < 1) blocks = 1;
   hipLaunchKernelGGL((k_dense_gemv<T>), dim3(blocks), dim3(kBlock), (size_t)n * sizeof(double), stream(), n, ainv,
@@ -1290,16 +1310,24 @@ void dense_gemv(int n, const double *ainv, const T *b, T *x, Scal *s, bool check
 }
 
 template <typename T>
-void bicg_p_update(int n, const T *r, const T *v, T *p, Scal *s) {
-  hipLaunchKernelGGL((k_bicg_p<T>), dim3(blocks_for(n, kBlock * 4)), dim3(kBlock), 0, stream(), n, r, v, p, s);
+void bicg_p_update(int n, const T *r, const T *v, T *p, Scal *s, const T *jd, T *ph) {
+  const Pend pd = take_pending(s);
+  const dim3 grid(blocks_for(n, kBlock * 4));
+  if (jd) hipLaunchKernelGGL((k_bicg_p<T, true>), grid, dim3(kBlock), 0, stream(), n, r, v, p, jd, ph, pd);
+  else hipLaunchKernelGGL((k_bicg_p<T, false>), grid, dim3(kBlock), 0, stream(), n, r, v, p, jd, ph, pd);
   CFDLA_HIP(hipGetLastError());
 }
 
 template <typename T>
-void bicg_s_update(int n, const T *r, const T *v, T *sv, Scal *s, RedWs &ws) {
+void bicg_s_update(int n, const T *r, const T *v, T *sv, Scal *s, RedWs &ws, const T *jd, T *sh) {
   const int blocks = blocks_for(n, kBlock * 4);
-  hipLaunchKernelGGL((k_bicg_s<T>), dim3(blocks), dim3(kBlock), 0, stream(), n, r, v, sv, s, ws.partials.p,
-                     ws.counter.p);
+  const Pend pd = take_pending(s);
+  if (jd)
+    hipLaunchKernelGGL((k_bicg_s<T, true>), dim3(blocks), dim3(kBlock), 0, stream(), n, r, v, sv, jd, sh, pd,
+                       ws.next());
+  else
+    hipLaunchKernelGGL((k_bicg_s<T, false>), dim3(blocks), dim3(kBlock), 0, stream(), n, r, v, sv, jd, sh, pd,
+                       ws.next());
   finish(1, s, OP_BI_SNORM, blocks, ws, true);
   CFDLA_HIP(hipGetLastError());
 }
@@ -1308,13 +1336,14 @@ template <typename T>
 void bicg_x_r_update(int n, const T *ph, const T *sh, const T *sv, const T *t, T *x, T *r, Scal *s, RedWs &ws,
                      const T *rhat) {
   const int blocks = blocks_for(n, kBlock * 4);
+  const Pend pd = take_pending(s);
   if (rhat) {
-    hipLaunchKernelGGL((k_bicg_xr<T, true>), dim3(blocks), dim3(kBlock), 0, stream(), n, ph, sh, sv, t, x, r, rhat,
-                       s, ws.partials.p, ws.counter.p);
+    hipLaunchKernelGGL((k_bicg_xr<T, true>), dim3(blocks), dim3(kBlock), 0, stream(), n, ph, sh, sv, t, x, r, rhat, pd,
+                       ws.next());
     finish(2, s, OP_BI_RR_RHO, blocks, ws, true);
   } else {
     hipLaunchKernelGGL((k_bicg_xr<T, false>), dim3(blocks), dim3(kBlock), 0, stream(), n, ph, sh, sv, t, x, r,
-                       nullptr, s, ws.partials.p, ws.counter.p);
+                       nullptr, pd, ws.next());
     finish(1, s, OP_BI_RR, blocks, ws, true);
   }
   CFDLA_HIP(hipGetLastError());
@@ -1322,6 +1351,7 @@ void bicg_x_r_update(int n, const T *ph, const T *sh, const T *sv, const T *t, T
 
 template <typename T>
 void axpy_scal(int n, const T *x, T *y, Scal *s, int /*which*/) {
+  s = settled_scal(s);
   hipLaunchKernelGGL((k_axpy_alpha<T>), dim3(blocks_for(n, kBlock * 4)), dim3(kBlock), 0, stream(), n, x, y, s);
   CFDLA_HIP(hipGetLastError());
 }
@@ -1330,6 +1360,7 @@ template <typename T>
 void sor_colour(int count, const int *perm, const int *rp, const int *ci, const T *v, const T *piv, const T *r, T *z,
                 Scal *s, bool check_done) {
   if (count == 0) return;
+  s = settled_scal(s);
   hipLaunchKernelGGL((k_sor_colour<T>), dim3(blocks_for(count, kBlock * 4)), dim3(kBlock), 0, stream(), count, perm,
                      rp, ci, v, piv, r, z, s, check_done ? 1 : 0);
   CFDLA_HIP(hipGetLastError());
@@ -1338,6 +1369,7 @@ template <typename T>
 void gs_colour(int count, const int *perm, const int *rp, const int *ci, const T *v, const T *b, T *x, double omega,
                Scal *s, bool check_done) {
   if (count == 0) return;
+  s = settled_scal(s);
   hipLaunchKernelGGL((k_gs_colour<T>), dim3(blocks_for(count, kBlock * 4)), dim3(kBlock), 0, stream(), count, perm,
                      rp, ci, v, b, x, (T)omega, s, check_done ? 1 : 0);
   CFDLA_HIP(hipGetLastError());
@@ -1349,6 +1381,7 @@ template void gs_colour<float>(int, const int *, const int *, const int *, const
 template <typename T>
 void sor_first(int n, const uint8_t *first, const T *piv, const T *r, T *z, Scal *s, bool check_done) {
   if (n == 0) return;
+  s = settled_scal(s);
   hipLaunchKernelGGL((k_sor_first<T>), dim3(blocks_for(n, kBlock * 4)), dim3(kBlock), 0, stream(), n, first, piv, r,
                      z, s, check_done ? 1 : 0);
   CFDLA_HIP(hipGetLastError());
@@ -1362,21 +1395,25 @@ template void sor_colour<float>(int, const int *, const int *, const int *, cons
                                 const float *, float *, Scal *, bool);
 
 void scal_reset(Scal *s, double thr2) {
+  s = settled_scal(s);
   hipLaunchKernelGGL(k_scal_reset, dim3(1), dim3(64), 0, stream(), s, thr2);
   CFDLA_HIP(hipGetLastError());
 }
 
 void scal_set_done(Scal *s, int value) {
+  s = settled_scal(s);
   hipLaunchKernelGGL(k_scal_set_done, dim3(1), dim3(64), 0, stream(), s, value);
   CFDLA_HIP(hipGetLastError());
 }
 
 void scal_set_final(Scal *s, double thr_final2) {
+  s = settled_scal(s);
   hipLaunchKernelGGL(k_scal_set_final, dim3(1), dim3(64), 0, stream(), s, thr_final2);
   CFDLA_HIP(hipGetLastError());
 }
 
 void scal_bicg_restart(Scal *s) {
+  s = settled_scal(s);
   hipLaunchKernelGGL(k_scal_bicg_restart, dim3(1), dim3(64), 0, stream(), s);
   CFDLA_HIP(hipGetLastError());
 }
@@ -1400,8 +1437,8 @@ void coef_grad_poisson2d(int64_t nx, int64_t ny, double inv_h2, int dir_mask, co
   template void copy_vec<T>(int, const T *, T *, Scal *, bool);                                                \
   template void fill_vec<T>(int, T, T *);                                                                      \
   template void dense_gemv<T>(int, const double *, const T *, T *, Scal *, bool, int);                             \
-  template void bicg_p_update<T>(int, const T *, const T *, T *, Scal *);                                      \
-  template void bicg_s_update<T>(int, const T *, const T *, T *, Scal *, RedWs &);                             \
+  template void bicg_p_update<T>(int, const T *, const T *, T *, Scal *, const T *, T *);                      \
+  template void bicg_s_update<T>(int, const T *, const T *, T *, Scal *, RedWs &, const T *, T *);             \
   template void bicg_x_r_update<T>(int, const T *, const T *, const T *, const T *, T *, T *, Scal *, RedWs &,  \
                                    const T *);                                                               \
   template void axpy_scal<T>(int, const T *, T *, Scal *, int);

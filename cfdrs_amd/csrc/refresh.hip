@@ -641,6 +641,7 @@ void simple_refresh(int64_t nx, int64_t ny, double dx, double dy, bool negate, c
                     double *v64, double *rhs, bool want_max) {
   const int grid = grid_for(nx * ny);
   RedWs &ws = ctx().ws;
+  flush_pending();
   hipLaunchKernelGGL(k_simple_refresh, dim3(grid), dim3(kBlock), 0, stream(), nx, ny, dx, dy, negate ? 1 : 0, u, v,
                      p, du, dv, rho, rp, v64, rhs, ws.partials.p);
   if (!want_max) return;

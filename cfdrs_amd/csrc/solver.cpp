@@ -63,7 +63,7 @@ void init_device(int dev) {
   d.ready = true;
   d.context = std::make_unique<Context>();
   d.context->ws.init();
-  d.context->scal.alloc(4);
+  d.context->scal.alloc(2 * kScalSlots);
   CFDLA_HIP(hipHostMalloc(reinterpret_cast<void **>(&d.context->host), sizeof(Scal), hipHostMallocDefault));
 }
 
@@ -99,41 +99,39 @@ Context &ctx() {
 }
 
 Scal Context::read(Scal *dev) {
-  CFDLA_HIP(hipMemcpyAsync(host, dev, sizeof(Scal), hipMemcpyDeviceToHost, stream()));
+  CFDLA_HIP(hipMemcpyAsync(host, settled_scal(dev), sizeof(Scal), hipMemcpyDeviceToHost, stream()));
   CFDLA_HIP(hipStreamSynchronize(stream()));
   return *host;
 }
 
 void RedWs::init() {
-  partials.alloc((size_t)kMaxRed * kMaxBlocks);
-  counter.alloc(1);
-  CFDLA_HIP(hipMemsetAsync(counter.p, 0, sizeof(unsigned), stream()));
-  CFDLA_HIP(hipStreamSynchronize(stream()));
+  partials.alloc((size_t)2 * kMaxRed * kMaxBlocks);
 }
 
-// Lagged poll: after each enqueued step, copy Scal to a pinned slot and
-// record an event; check the previous step's slot.
+// Lagged poll: copies Scal to a pinned slot and records an event.  advanced()
+// is posted within a chunk of steps, right after its first kernel that took
+// the previous chunk's last reduction along: the copy holds the state at that
+// chunk's end, no launch is spent on finalizing it, and the host that waits
+// for it has the rest of the chunk queued.  settled() is the state of
+// everything enqueued.
 struct Poller {
   int k = 0;
   Scal *dev;
   explicit Poller(Scal *s) : dev(s) {}
-  void post() {
-    DeviceState &d = dstate();
-    CFDLA_HIP(hipMemcpyAsync(d.poll + (k & 1), dev, sizeof(Scal), hipMemcpyDeviceToHost, stream()));
-    CFDLA_HIP(hipEventRecord(d.ev[k & 1], stream()));
-    ++k;
-  }
-  // State as of the step before the last one posted (nullptr if none).
-  const Scal *lagged() {
-    if (k < 2) return nullptr;
-    DeviceState &d = dstate();
-    CFDLA_HIP(hipEventSynchronize(d.ev[(k - 2) & 1]));
-    return d.poll + ((k - 2) & 1);
-  }
+  void advanced() { post(live_scal(dev)); }
+  void settled() { post(settled_scal(dev)); }
   const Scal *latest() {
     DeviceState &d = dstate();
     CFDLA_HIP(hipEventSynchronize(d.ev[(k - 1) & 1]));
     return d.poll + ((k - 1) & 1);
+  }
+
+ private:
+  void post(const Scal *from) {
+    DeviceState &d = dstate();
+    CFDLA_HIP(hipMemcpyAsync(d.poll + (k & 1), from, sizeof(Scal), hipMemcpyDeviceToHost, stream()));
+    CFDLA_HIP(hipEventRecord(d.ev[k & 1], stream()));
+    ++k;
   }
 };
 
@@ -1323,7 +1321,7 @@ SolveOut pcg(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int64_t 
   int64_t enq = 0;
   Poller poll(s);
   ConvergenceGate gate;
-  bool finished = false;
+  bool finished = false, behind = false;  // behind: a chunk is enqueued whose end has not been polled
   while (!finished) {
     const Scal *h = nullptr;
     if (enq < max_it) {
@@ -1336,6 +1334,7 @@ SolveOut pcg(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int64_t 
           csr_apply<T>(A, EPI_Y, p, nullptr, nullptr, 0.0, q, s, true, OP_CG_ALPHA, p, ws);
         }
         fresh = false;
+        if (k == 0 && behind) poll.advanced();
         if (jd) {
           cg_update<T>(n, p, q, x, r, jd, z, s, ws);
         } else {
@@ -1345,14 +1344,18 @@ SolveOut pcg(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int64_t 
         if (!fuse) cg_direction<T>(n, z, p, s);
       }
       enq += steps;
-      poll.post();
-      h = poll.lagged();
+      if (!behind) {
+        behind = true;
+        continue;
+      }
+      h = poll.latest();
     } else {
+      poll.settled();
       h = poll.latest();
     }
-    if (!h) continue;
     if (h->done == 0 && enq < max_it) {
       if (!gate.expect(h->rr, thr * thr)) continue;
+      poll.settled();
       h = poll.latest();
       if (h->done == 0) continue;
     }
@@ -1376,7 +1379,7 @@ SolveOut pcg(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int64_t 
       }
       scal_set_done(s, 0);  // residual replacement: restart from the explicit residual
       start_direction();
-      poll = Poller(s);
+      behind = false;
     } else {
       finished = true;  // budget exhausted
     }
@@ -1459,6 +1462,7 @@ SolveOut pcg_reliable(const DevCsr &A, Precond *M, const double *b, double *x, d
   bool want = false;         // a reduction by delta was seen: replace in the next step
   Poller poll(s);
   ConvergenceGate gate;
+  bool behind = false;  // a chunk is enqueued whose end has not been polled
   for (;;) {
     const Scal *h = nullptr;
     if (enq < max_it) {
@@ -1471,6 +1475,7 @@ SolveOut pcg_reliable(const DevCsr &A, Precond *M, const double *b, double *x, d
           csr_apply<float>(A, EPI_Y, p, nullptr, nullptr, 0.0, q, s, true, OP_CG_ALPHA, p, ws);
         }
         fresh = false;
+        if (k == 0 && behind) poll.advanced();
         const bool rep = want || (interval > 0 && (enq + k + 1) % interval == 0);
         if (rep) ++replacements;
         want = false;
@@ -1491,12 +1496,15 @@ SolveOut pcg_reliable(const DevCsr &A, Precond *M, const double *b, double *x, d
         }
       }
       enq += steps;
-      poll.post();
-      h = poll.lagged();
+      if (!behind) {
+        behind = true;
+        continue;
+      }
+      h = poll.latest();
     } else {
+      poll.settled();
       h = poll.latest();
     }
-    if (!h) continue;
     if (h->done == 0 && enq < max_it) {
       // Reduction trigger (Clark et al. 2010): once every replacement enqueued
       // so far shows in the polled state, replace again when the recursive
@@ -1507,6 +1515,7 @@ SolveOut pcg_reliable(const DevCsr &A, Precond *M, const double *b, double *x, d
       const double de = std::min(0.5, delta * std::pow(10.0, (double)h->nrestart));
       if (delta > 0.0 && h->nupd >= replacements && h->rr <= de * de * ref) want = true;
       if (!gate.expect(h->rr, thr * thr)) continue;
+      poll.settled();
       h = poll.latest();
       if (h->done == 0) continue;
     }
@@ -1519,9 +1528,8 @@ SolveOut pcg_reliable(const DevCsr &A, Precond *M, const double *b, double *x, d
       const Scal conf = c.read(s);
       if (conf.done != 4) {
         direction();
-        poll = Poller(s);
         gate = ConvergenceGate();
-        poll.post();  // the replaced state, so latest() is defined once the budget is spent
+        behind = false;
         continue;
       }
     }
@@ -1554,6 +1562,7 @@ SolveOut bicgstab(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int
   const int n = A.n;
   T *r = vec<T>(0, n), *rhat = vec<T>(1, n), *p = vec<T>(2, n), *v = vec<T>(3, n);
   T *ph = vec<T>(4, n), *sv = vec<T>(5, n), *sh = vec<T>(6, n), *t = vec<T>(7, n);
+  const T *jd = jdinv<T>(M);
   Scal *s = c.s(0);
   SolveOut o;
   o.thr = thr;
@@ -1577,7 +1586,7 @@ SolveOut bicgstab(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int
   if (chunk <= 0) chunk = auto_chunk(M, n);
   int64_t enq = 0;
   Poller poll(s);
-  bool finished = false;
+  bool finished = false, behind = false;  // behind: a chunk is enqueued whose end has not been polled
   while (!finished) {
     const Scal *h = nullptr;
     if (enq < max_it) {
@@ -1585,22 +1594,26 @@ SolveOut bicgstab(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int
       for (int64_t k = 0; k < steps; ++k) {
         if (need_rho) dot2<T>(n, rhat, r, nullptr, nullptr, s, true, OP_BI_RHO, ws);
         need_rho = false;
-        bicg_p_update<T>(n, r, v, p, s);
-        M->apply(p, ph, s, true);
+        // the Jacobi preconditioner rides on the updates
+        bicg_p_update<T>(n, r, v, p, s, jd, ph);
+        if (k == 0 && behind) poll.advanced();
+        if (!jd) M->apply(p, ph, s, true);
         csr_apply<T>(A, EPI_Y, ph, nullptr, nullptr, 0.0, v, s, true, OP_BI_ALPHA, rhat, ws);
-        bicg_s_update<T>(n, r, v, sv, s, ws);
-        M->apply(sv, sh, s, true);
-        csr_apply<T>(A, EPI_Y, sh, nullptr, nullptr, 0.0, t, s, true, OP_NONE, nullptr, ws);
-        dot2<T>(n, t, sv, t, t, s, true, OP_BI_OMEGA, ws);
+        bicg_s_update<T>(n, r, v, sv, s, ws, jd, sh);
+        if (!jd) M->apply(sv, sh, s, true);
+        csr_apply<T>(A, EPI_DOT2, sh, nullptr, nullptr, 0.0, t, s, true, OP_BI_OMEGA, sv, ws);
         bicg_x_r_update<T>(n, ph, sh, sv, t, x, r, s, ws, rhat);
       }
       enq += steps;
-      poll.post();
-      h = poll.lagged();
+      if (!behind) {
+        behind = true;
+        continue;
+      }
+      h = poll.latest();
     } else {
+      poll.settled();
       h = poll.latest();
     }
-    if (!h) continue;
     if (h->done == 0 && enq < max_it) continue;
     sync_stream();
     Scal now = c.read(s);
@@ -1618,7 +1631,7 @@ SolveOut bicgstab(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int
       }
       scal_set_done(s, 0);
       restart();
-      poll = Poller(s);
+      behind = false;
     } else {
       finished = true;
     }
@@ -1646,6 +1659,7 @@ SolveOut bicgstab_reliable(const DevCsr &A, Precond *M, const double *b, double 
   double *r64 = c.dv_at(8, n);
   float *r = c.fv_at(0, n), *rhat = c.fv_at(1, n), *p = c.fv_at(2, n), *v = c.fv_at(3, n);
   float *ph = c.fv_at(4, n), *sv = c.fv_at(5, n), *sh = c.fv_at(6, n), *t = c.fv_at(7, n), *xc = c.fv_at(8, n);
+  const float *jd = jdinv<float>(M);
   Scal *s = c.s(0);
   SolveOut o;
   o.thr = thr;
@@ -1674,6 +1688,7 @@ SolveOut bicgstab_reliable(const DevCsr &A, Precond *M, const double *b, double 
   int32_t replacements = 0;
   bool want = false;
   Poller poll(s);
+  bool behind = false;  // a chunk is enqueued whose end has not been polled
   for (;;) {
     const Scal *h = nullptr;
     if (enq < max_it) {
@@ -1685,22 +1700,26 @@ SolveOut bicgstab_reliable(const DevCsr &A, Precond *M, const double *b, double 
           want = false;
         }
         dot2<float>(n, rhat, r, nullptr, nullptr, s, true, OP_BI_RHO, ws);
-        bicg_p_update<float>(n, r, v, p, s);
-        M->apply(p, ph, s, true);
+        // the Jacobi preconditioner rides on the updates
+        bicg_p_update<float>(n, r, v, p, s, jd, ph);
+        if (k == 0 && behind) poll.advanced();
+        if (!jd) M->apply(p, ph, s, true);
         csr_apply<float>(A, EPI_Y, ph, nullptr, nullptr, 0.0, v, s, true, OP_BI_ALPHA, rhat, ws);
-        bicg_s_update<float>(n, r, v, sv, s, ws);
-        M->apply(sv, sh, s, true);
-        csr_apply<float>(A, EPI_Y, sh, nullptr, nullptr, 0.0, t, s, true, OP_NONE, nullptr, ws);
-        dot2<float>(n, t, sv, t, t, s, true, OP_BI_OMEGA, ws);
+        bicg_s_update<float>(n, r, v, sv, s, ws, jd, sh);
+        if (!jd) M->apply(sv, sh, s, true);
+        csr_apply<float>(A, EPI_DOT2, sh, nullptr, nullptr, 0.0, t, s, true, OP_BI_OMEGA, sv, ws);
         bicg_x_r_update<float>(n, ph, sh, sv, t, xc, r, s, ws);
       }
       enq += steps;
-      poll.post();
-      h = poll.lagged();
+      if (!behind) {
+        behind = true;
+        continue;
+      }
+      h = poll.latest();
     } else {
+      poll.settled();
       h = poll.latest();
     }
-    if (!h) continue;
     if (h->done == 0 && enq < max_it) {
       const double ref = h->nupd > 0 ? h->rr_true : o.rn0 * o.rn0;
       const double de = std::min(0.5, delta * std::pow(10.0, (double)h->nrestart));
@@ -1729,7 +1748,7 @@ SolveOut bicgstab_reliable(const DevCsr &A, Precond *M, const double *b, double 
         return o;
       }
       restart();
-      poll = Poller(s);
+      behind = false;
       continue;
     }
     if (now.done == 4) {

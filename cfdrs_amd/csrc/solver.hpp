@@ -13,7 +13,9 @@ namespace cfdla {
 // and pooled solver vectors.
 struct Context {
   RedWs ws;
-  DevBuf<Scal> scal;  // 4 slots
+  DevBuf<Scal> scal;  // kScalSlots slots and their twins
+  int twin[kScalSlots] = {};  // 1: slot i's scalars are in its twin
+  Pend pend{};
   Scal *host = nullptr;
   DevBuf<double> dv[12];
   DevBuf<float> fv[12];
