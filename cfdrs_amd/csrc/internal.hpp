@@ -324,6 +324,9 @@ Scal *live_scal(Scal *s);
 void flush_pending();
 Scal *settled_scal(Scal *s);
 Pend take_pending(Scal *s);
+// The other slot of the settled scalars s, which becomes the live one: for a
+// kernel that reads s and writes its successor there.
+Scal *twin_scal(Scal *s);
 bool pending_on(Scal *s);  // take_pending(s) would return a reduction
 
 enum FinalizeOp : int {
@@ -490,16 +493,24 @@ void axpy_scal(int n, const T *x, T *y, Scal *s, int which);  // y += s->{alpha}
 template <typename T>
 void sor_colour(int count, const int *perm, const int *rp, const int *ci, const T *v, const T *piv, const T *r, T *z,
                 Scal *s, bool check_done);
-// The first colour from z = 0, which sees no nonzero neighbour:
-// z_i = piv_i r_i where first[i], 0 elsewhere (all 0 when check_done and
-// s->done != 0).
 // One colour of a multicolour Gauss-Seidel sweep (rows perm[0..count)),
 // x_i += omega ((b_i - sum_{j != i} a_ij x_j) / a_ii - x_i) where |a_ii| > 1e-15.
 template <typename T>
 void gs_colour(int count, const int *perm, const int *rp, const int *ci, const T *v, const T *b, T *x, double omega,
                Scal *s, bool check_done);
+// The start of a sweep from z = 0.  w = 0: the first colour, which sees no
+// nonzero neighbour, z_i = piv_i r_i where cls[i] = 0, 0 elsewhere.  w > 0
+// (sor_start_width): the second colour too, z_i = piv_i (r_i - sum a_ij z_j)
+// with z_j formed from r on the fly, entries slot-major in ci, v.  All 0 when
+// check_done and s->done != 0.
+int sor_start_width(int longest);  // slots per row the start kernel takes, 0: too many
+// the slot-major couplings of the second colour to the first, from CSR on the
+// device; every other slot holds the row itself and 0
+void sor_start_slots(int n, int w, const uint8_t *cls, const int *rp, const int *ci, const double *v64, int *sci,
+                     double *sv64, float *sv32);
 template <typename T>
-void sor_first(int n, const uint8_t *first, const T *piv, const T *r, T *z, Scal *s, bool check_done);
+void sor_start(int n, int w, const uint8_t *cls, const int *ci, const T *v, const T *piv, const T *r, T *z, Scal *s,
+               bool check_done);
 
 // Scalars helpers
 void scal_reset(Scal *s, double thr2);

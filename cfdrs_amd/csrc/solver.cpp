@@ -790,32 +790,48 @@ ColoredSorPrecond::ColoredSorPrecond(const HostCsr &a, double omega) {
   for (double p : piv) CFDLA_REQUIRE(std::isfinite(p), CFDLA_ERR_NUMERICAL, "SOR: non-finite pivot");
   std::vector<int32_t> rp32((size_t)n + 1);
   for (int i = 0; i <= n; ++i) rp32[(size_t)i] = (int32_t)a.rp[(size_t)i];
-  std::vector<float> v32h(a.v.size()), piv32h(piv.size());
-  for (size_t k = 0; k < a.v.size(); ++k) v32h[k] = (float)a.v[k];
-  for (size_t k = 0; k < piv.size(); ++k) piv32h[k] = (float)piv[k];
-  std::vector<uint8_t> first_h((size_t)n);
-  for (int i = 0; i < n; ++i) first_h[(size_t)i] = colour[(size_t)i] == 0 ? 1 : 0;
-  first.upload(first_h.data(), first_h.size());
+  std::vector<uint8_t> cls_h((size_t)n);
+  for (int i = 0; i < n; ++i) cls_h[(size_t)i] = (uint8_t)std::min(colour[(size_t)i], 2);
+  // the second colour's longest row of couplings to the first
+  int longest = 0;
+  for (int i = 0; i < n; ++i) {
+    if (colour[(size_t)i] != 1) continue;
+    int m = 0;
+    for (int64_t k = a.rp[i]; k < a.rp[i + 1]; ++k) m += colour[(size_t)a.ci[k]] == 0;
+    longest = std::max(longest, m);
+  }
+  start_w = ncolours > 1 ? sor_start_width(longest) : 0;
+  if ((int64_t)start_w * n > 2 * a.nnz() + 4096) start_w = 0;  // the padding at most doubles the matrix
+  cls.upload(cls_h.data(), cls_h.size());
   perm.upload(order.data(), order.size());
   rp.upload(rp32.data(), rp32.size());
   ci.upload(a.ci.data(), a.ci.size());
   v64.upload(a.v.data(), a.v.size());
-  v32.upload(v32h.data(), v32h.size());
   piv64.upload(piv.data(), piv.size());
-  piv32.upload(piv32h.data(), piv32h.size());
+  // FP32 copies and the slot-major layout are made on the device
+  v32.alloc(a.v.size());
+  piv32.alloc((size_t)n);
+  if (a.nnz() > 0) f64_to_f32_scaled((int)a.nnz(), v64.p, 1.0, v32.p);
+  if (n > 0) f64_to_f32_scaled(n, piv64.p, 1.0, piv32.p);
+  if (start_w > 0) {
+    start_ci.alloc((size_t)start_w * (size_t)n);
+    start_v64.alloc((size_t)start_w * (size_t)n);
+    start_v32.alloc((size_t)start_w * (size_t)n);
+    sor_start_slots(n, start_w, cls.p, rp.p, ci.p, v64.p, start_ci.p, start_v64.p, start_v32.p);
+  }
   sync_stream();
 }
 
 void ColoredSorPrecond::apply(const double *r, double *z, Scal *s, bool chk) {
-  sor_first<double>(n, first.p, piv64.p, r, z, s, chk);
-  for (int c = 1; c < ncolours; ++c)
+  sor_start<double>(n, start_w, cls.p, start_ci.p, start_v64.p, piv64.p, r, z, s, chk);
+  for (int c = start_w > 0 ? 2 : 1; c < ncolours; ++c)
     sor_colour<double>(colour_off[(size_t)c + 1] - colour_off[(size_t)c], perm.p + colour_off[(size_t)c], rp.p, ci.p,
                        v64.p, piv64.p, r, z, s, chk);
 }
 
 void ColoredSorPrecond::apply(const float *r, float *z, Scal *s, bool chk) {
-  sor_first<float>(n, first.p, piv32.p, r, z, s, chk);
-  for (int c = 1; c < ncolours; ++c)
+  sor_start<float>(n, start_w, cls.p, start_ci.p, start_v32.p, piv32.p, r, z, s, chk);
+  for (int c = start_w > 0 ? 2 : 1; c < ncolours; ++c)
     sor_colour<float>(colour_off[(size_t)c + 1] - colour_off[(size_t)c], perm.p + colour_off[(size_t)c], rp.p, ci.p,
                       v32.p, piv32.p, r, z, s, chk);
 }

@@ -66,7 +66,14 @@ struct ColoredSorPrecond : Precond {
   int n = 0, ncolours = 0;
   std::vector<int32_t> colour_off;  // ncolours + 1 offsets into perm
   DevBuf<int32_t> perm, rp, ci;      // rows grouped by colour; the matrix pattern
-  DevBuf<uint8_t> first;             // 1 on the rows of the first colour
+  DevBuf<uint8_t> cls;               // 0 on the first colour's rows, 1 on the second's, 2 elsewhere
+  // The second colour's couplings to the first, slot-major over all rows
+  // (start_w slots; padding, and every slot of the other rows: the row itself),
+  // for sweeps whose start is one launch; start_w = 0: rows too long or uneven.
+  int start_w = 0;
+  DevBuf<int32_t> start_ci;
+  DevBuf<double> start_v64;
+  DevBuf<float> start_v32;
   DevBuf<double> v64, piv64;         // values; omega / pivot (unit pivot where the diagonal is absent or zero)
   DevBuf<float> v32, piv32;
   ColoredSorPrecond(const HostCsr &a, double omega);
