@@ -204,6 +204,15 @@ struct DevCsr {
   DevBuf<int16_t> sell_delta; // col - row, kSellPad for padding
   DevBuf<double> sell_v64;
   DevBuf<float> sell_v32;
+  // Padded rows, for the small operators of an AMG hierarchy (allow_ell of
+  // upload): every row ell_lanes groups of 4 entries, one group per lane
+  // (padding: column -1), columns int32, row-major.  An operator stored this
+  // way carries no row blocks.
+  bool ell = false;
+  int ell_lanes = 0;
+  DevBuf<int32_t> ell_ci;
+  DevBuf<double> ell_v64;
+  DevBuf<float> ell_v32;
   bool dia = false;
   bool general_dia = false;  // a device update broke symmetry once: keep every diagonal from then on
   DiaDesc dia_desc;
@@ -213,7 +222,7 @@ struct DevCsr {
   // format from the matrix (diagonal, then sliced ELL, then row-block CSR);
   // a fixed one skips the others, for measuring one product kernel.
   int fmt_request = -1;
-  void upload(const HostCsr &h, bool want_fp32, bool want_dinv, bool allow_sell = true);
+  void upload(const HostCsr &h, bool want_fp32, bool want_dinv, bool allow_sell = true, bool allow_ell = false);
   // Device value refresh.  v64 (CSR order) is the truth; build_maps (once,
   // from the host pattern) records for every CSR slot its position in the
   // diagonal or sliced-ELL value arrays (fmt_pos, -1: none), for symmetric
@@ -224,6 +233,7 @@ struct DevCsr {
   // v64; it returns false, having changed nothing, when v64 is no longer
   // symmetric under a symmetric diagonal layout (the caller then rebuilds
   // the layout through the host with general_dia set).
+  void upload_ell(const HostCsr &h, bool want_fp32, bool want_dinv);
   bool maps_ready = false;
   DevBuf<int32_t> fmt_pos, fmt_mirror, diag_slot;
   void build_maps(const HostCsr &h);
@@ -232,6 +242,7 @@ struct DevCsr {
   template <typename T> const T *sdinv() const;
   template <typename T> const T *sell_vals() const;
   template <typename T> const T *dia_vals() const;
+  template <typename T> const T *ell_vals() const;
   template <typename T> const int *rb() const { return sizeof(T) == 8 ? rb64.p : rb32.p; }
   template <typename T> int nrb() const { return sizeof(T) == 8 ? nrb64 : nrb32; }
   template <typename T> bool has_cols16() const { return sizeof(T) == 8 ? c16_f64 : c16_f32; }
@@ -250,10 +261,22 @@ template <> inline const double *DevCsr::sell_vals<double>() const { return sell
 template <> inline const float *DevCsr::sell_vals<float>() const { return sell_v32.p; }
 template <> inline const double *DevCsr::dia_vals<double>() const { return dia_v64.p; }
 template <> inline const float *DevCsr::dia_vals<float>() const { return dia_v32.p; }
+template <> inline const double *DevCsr::ell_vals<double>() const { return ell_v64.p; }
+template <> inline const float *DevCsr::ell_vals<float>() const { return ell_v32.p; }
 template <> inline const double *DevCsr::rb_vals<double>() const { return layout64 == kRbSorted ? sv64.p : v64.p; }
 template <> inline const float *DevCsr::rb_vals<float>() const { return layout32 == kRbSorted ? sv32.p : v32.p; }
 
 
+// Padded rows pay where a product is latency, not bytes: up to 700,000 slots
+// 2.5-3.1 us against 4.0-4.3 us in row blocks (the coarse levels of a 383x255
+// grid, FP64).  Above, the padding and the 32-bit columns cost more than the
+// row blocks' barrier: a level of 8,732 rows with 72 entries each (1.1M slots)
+// 8.1 us against 7.1, FP32, and the whole 128^3 solve 4.11 against 4.01 ms.
+constexpr int kEllMaxLanes = 64;
+constexpr int64_t kEllMaxSlots = 700000;
+// Lanes per row of the padded-row layout (a power of two of 4-entry groups),
+// or 0 when the operator is not small or its rows are too long or uneven.
+int ell_lanes_for(const HostCsr &h);
 // span > 0: a block also closes before its columns would span more than
 // `span` (so 16-bit column offsets fit every block whose rows each do).
 void build_row_blocks(const HostCsr &h, int cap, int max_rows, std::vector<int32_t> &rb, int64_t span = 0);

@@ -24,6 +24,26 @@ __device__ __forceinline__ double dpp_move(double v) {
   return __builtin_bit_cast(double, (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
 
+// v of this lane plus v of the lane W (16 or 32) away.
+template <int W>
+__device__ __forceinline__ auto lane_swap(unsigned v) {
+  if constexpr (W == 32) return __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  else return __builtin_amdgcn_permlane16_swap(v, v, false, false);
+}
+template <int W>
+__device__ __forceinline__ double add_across(double v) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+  const auto lo = lane_swap<W>((unsigned)b), hi = lane_swap<W>((unsigned)(b >> 32));
+  return __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]) +
+         __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
+}
+template <int W>
+__device__ __forceinline__ float add_across(float v) {
+  const auto p = lane_swap<W>(__builtin_bit_cast(unsigned, v));
+  const unsigned a = p[0], b = p[1];  // (a bit cast of a vector's element reads its first one)
+  return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+}
+
 // Sum of a wavefront, in every lane: the xor tree 32, 16, 8, 4, 2, 1 without
 // LDS traffic.  The lane swaps of gfx950 add the halves (lane ^ 32) and then
 // the rows (lane ^ 16); within a row the partial sums repeat with the period
@@ -34,20 +54,8 @@ __device__ __forceinline__ double dpp_move(double v) {
 // iteration: 10.5 -> 8.8 ms for 750 iterations; 600 networks of 30-700 nodes
 // with their adjoint: 6.41 -> 5.75 ms).
 __device__ __forceinline__ double wave_sum(double v) {
-  {
-    const long long b = __builtin_bit_cast(long long, v);
-    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)b, (unsigned)b, false, false);
-    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
-    v = __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]) +
-        __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
-  }
-  {
-    const long long b = __builtin_bit_cast(long long, v);
-    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)b, (unsigned)b, false, false);
-    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
-    v = __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]) +
-        __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
-  }
+  v = add_across<32>(v);
+  v = add_across<16>(v);
   v += dpp_move<0x128>(v);  // row_ror:8
   v += dpp_move<0x124>(v);  // row_ror:4
   v += dpp_move<0x122>(v);  // row_ror:2

@@ -600,8 +600,8 @@ void fused_values(const DevCsr &A, double w, double *sv, double *ev) {
 
 void scatter_formats(DevCsr &d) {
   if (d.nnz > 0) {
-    double *f64 = d.dia ? d.dia_v64.p : (d.sell ? d.sell_v64.p : nullptr);
-    float *f32 = d.dia ? d.dia_v32.p : (d.sell ? d.sell_v32.p : nullptr);
+    double *f64 = d.dia ? d.dia_v64.p : d.sell ? d.sell_v64.p : d.ell ? d.ell_v64.p : nullptr;
+    float *f32 = d.dia ? d.dia_v32.p : d.sell ? d.sell_v32.p : d.ell ? d.ell_v32.p : nullptr;
     hipLaunchKernelGGL(k_scatter, dim3(grid_for(d.nnz)), dim3(kBlock), 0, stream(), d.nnz, d.v64.p, d.v32.p,
                        d.fmt_pos.p, f64, f32);
   }

@@ -474,7 +474,18 @@ bool build_dia(const HostCsr &h, DiaDesc &d, std::vector<double> &val, bool allo
 }
 }  // namespace
 
-void DevCsr::upload(const HostCsr &h, bool want_fp32, bool want_dinv, bool allow_sell) {
+int ell_lanes_for(const HostCsr &h) {
+  if (h.n < 1 || h.m < 1) return 0;
+  int64_t w = 0;
+  for (int64_t i = 0; i < h.n; ++i) w = std::max<int64_t>(w, h.rp[i + 1] - h.rp[i]);
+  int lanes = 1;
+  while (4 * lanes < w) lanes *= 2;
+  if (lanes > kEllMaxLanes) return 0;
+  const int64_t slots = 4 * (int64_t)lanes * h.n;
+  return slots <= kEllMaxSlots && slots <= 3 * h.nnz() + 4096 ? lanes : 0;
+}
+
+void DevCsr::upload(const HostCsr &h, bool want_fp32, bool want_dinv, bool allow_sell, bool allow_ell) {
   CFDLA_REQUIRE(h.n < INT32_MAX && h.m < INT32_MAX && h.nnz() < INT32_MAX, CFDLA_ERR_INVALID_ARG,
                 "matrix too large for 32-bit device indices");
   n = (int)h.n;
@@ -483,6 +494,20 @@ void DevCsr::upload(const HostCsr &h, bool want_fp32, bool want_dinv, bool allow
   std::vector<int32_t> rp32((size_t)h.n + 1);
   for (int64_t i = 0; i <= h.n; ++i) rp32[i] = (int32_t)h.rp[i];
   rp.upload(rp32.data(), rp32.size());
+  std::vector<double> dvals;
+  const bool want_dia = fmt_request == -1 || fmt_request == CFDLA_STORAGE_DIA;
+  const bool want_sell = fmt_request == -1 || fmt_request == CFDLA_STORAGE_SELL64;
+  dia = allow_sell && want_dia && build_dia(h, dia_desc, dvals, !general_dia);
+  maps_ready = false;
+  ell_lanes = allow_ell && !dia && gather_request == CFDLA_GATHER_AUTO && fmt_request == -1 ? ell_lanes_for(h) : 0;
+  ell = ell_lanes > 0;
+  if (ell) {
+    upload_ell(h, want_fp32, want_dinv);
+    return;
+  }
+  ell_ci.release();
+  ell_v64.release();
+  ell_v32.release();
   std::vector<int32_t> blocks;
   // (Smaller caps for small matrices, to reach 8 blocks per CU, measured
   // slower on every AMG level of the 128^3 problem: 7.6 -> 10.4 us per level-2
@@ -540,11 +565,6 @@ void DevCsr::upload(const HostCsr &h, bool want_fp32, bool want_dinv, bool allow
     for (size_t k = 0; k < d.size(); ++k) df[k] = (float)d[k];
     sdinv32.upload(df.data(), df.size());
   }
-  std::vector<double> dvals;
-  const bool want_dia = fmt_request == -1 || fmt_request == CFDLA_STORAGE_DIA;
-  const bool want_sell = fmt_request == -1 || fmt_request == CFDLA_STORAGE_SELL64;
-  dia = allow_sell && want_dia && build_dia(h, dia_desc, dvals, !general_dia);
-  maps_ready = false;
   if (dia) {
     dia_v64.upload(dvals.data(), dvals.size());
     if (want_fp32) {
@@ -629,6 +649,44 @@ void DevCsr::upload(const HostCsr &h, bool want_fp32, bool want_dinv, bool allow
   sync_stream();
 }
 
+// The padded-row layout: the CSR values (the truth of a device refresh) and
+// the padded copy.
+void DevCsr::upload_ell(const HostCsr &h, bool want_fp32, bool want_dinv) {
+  for (auto *b : {&rb64, &rb32, &cbase64, &cbase32, &sci, &sell_ptr}) b->release();
+  for (auto *b : {&c16_64, &c16_32}) b->release();
+  for (auto *b : {&sv64, &dia_v64, &sell_v64}) b->release();
+  for (auto *b : {&sv32, &dia_v32, &sell_v32, &v32}) b->release();
+  sell_delta.release();
+  nrb64 = nrb32 = 0;
+  c16_f64 = c16_f32 = sell = false;
+  layout64 = layout32 = kRbQuad;
+  ci.upload_padded(h.ci.data(), h.ci.size(), kRbPad);
+  v64.upload_padded(h.v.data(), h.v.size(), kRbPad);
+  const size_t slots = (size_t)4 * ell_lanes * (size_t)h.n;
+  std::vector<int32_t> ec(slots, -1);
+  std::vector<double> ev(slots, 0.0), d;
+  for (int64_t i = 0; i < h.n; ++i) {
+    const size_t o = (size_t)i * 4 * ell_lanes;
+    for (int64_t k = h.rp[i]; k < h.rp[i + 1]; ++k) {
+      ec[o + (size_t)(k - h.rp[i])] = h.ci[(size_t)k];
+      ev[o + (size_t)(k - h.rp[i])] = h.v[(size_t)k];
+    }
+  }
+  ell_ci.upload(ec.data(), ec.size());
+  ell_v64.upload(ev.data(), ev.size());
+  if (want_fp32) {
+    ell_v32.ensure(slots);
+    f64_to_f32_scaled((int)slots, ell_v64.p, 1.0, ell_v32.p);
+  }
+  if (want_dinv) {
+    smoother_dinv(h, d);
+    sdinv64.upload(d.data(), d.size());
+    sdinv32.ensure(d.size());
+    f64_to_f32_scaled((int)d.size(), sdinv64.p, 1.0, sdinv32.p);
+  }
+  sync_stream();
+}
+
 void DevCsr::build_maps(const HostCsr &h) {
   std::vector<int32_t> pos((size_t)h.nnz(), -1), mirror, dslot((size_t)h.n, -1);
   if (dia && dia_desc.sym) mirror.assign((size_t)h.nnz(), -1);
@@ -657,6 +715,10 @@ void DevCsr::build_maps(const HostCsr &h) {
       for (int64_t k = h.rp[r]; k < h.rp[r + 1]; ++k)
         pos[(size_t)k] = (int32_t)sell_pos(sp[(size_t)(r / 64)], k - h.rp[r], r % 64, sell_group);
   }
+  if (ell)
+    for (int64_t r = 0; r < h.n; ++r)
+      for (int64_t k = h.rp[r]; k < h.rp[r + 1]; ++k)
+        pos[(size_t)k] = (int32_t)(r * 4 * ell_lanes + k - h.rp[r]);
   fmt_pos.upload(pos.data(), pos.size());
   if (!mirror.empty()) fmt_mirror.upload(mirror.data(), mirror.size());
   diag_slot.upload(dslot.data(), dslot.size());
@@ -925,10 +987,10 @@ void AmgPrecond::upload() {
     HostLevel &h = host.levels[l];
     DevLevel &d = lv[l];
     d.A.gather_request = d.P.gather_request = d.R.gather_request = gather_request;
-    d.A.upload(h.A, true, true);
+    d.A.upload(h.A, true, true, true, l > 0 && cfg.smoother == 2);
     if (l + 1 < L) {
-      d.P.upload(h.P, true, false);
-      d.R.upload(h.R, true, false);
+      d.P.upload(h.P, true, false, true, true);
+      d.R.upload(h.R, true, false, true, true);
     }
     if (cfg.smoother != 2) {
       std::vector<int32_t> colour, order;
@@ -978,7 +1040,7 @@ void refresh_level(DevCsr &d, HostCsr &h, bool want_dinv) {
   d.v64.download(h.v.data(), h.v.size());
   sync_stream();
   d.general_dia = true;
-  d.upload(h, true, want_dinv);
+  d.upload(h, true, want_dinv);  // (a diagonal layout: never padded rows)
 }
 
 void put_plan(DevPlan &d, const ProductPlan &p) {
@@ -1014,34 +1076,40 @@ bool AmgPrecond::build_fused(size_t l) {
   // F stands in for a sweep and a residual over A and the restriction R;
   // keep the three products when it would stream more than twice their bytes
   if ((double)(S.nnz() + f.M.nnz()) > 2.0 * (2.0 * (double)A.nnz() + (double)R.nnz())) return false;
-  // M's rows (thousands of entries on the level above a 641-row coarsest
-  // level) are cut into `parts` pieces of at most one row block's capacity,
-  // so they pack into ordinary row blocks instead of running as single-
-  // block long rows (31 against 13 us FP64 at 128^3); the dense coarse solve
-  // adds each row's pieces.  Pieces are consecutive slices of the row, so
-  // F's values are S's followed by M's unchanged.
-  const int64_t piece = rb_cap<double>();
-  int64_t parts = 1;
-  for (int64_t j = 0; j < f.M.n; ++j) parts = std::max(parts, (f.M.rp[j + 1] - f.M.rp[j] + piece - 1) / piece);
   HostCsr &F = f.F;
-  F.n = A.n + f.M.n * parts;
   F.m = A.m;
-  F.rp = S.rp;
-  F.rp.reserve((size_t)F.n + 1);
-  for (int64_t j = 0; j < f.M.n; ++j)
-    for (int64_t k = 1; k <= parts; ++k)
-      F.rp.push_back(S.nnz() + std::min(f.M.rp[j + 1], f.M.rp[j] + k * piece));
   F.ci = S.ci;
   F.ci.insert(F.ci.end(), f.M.ci.begin(), f.M.ci.end());
   F.v = S.v;
   F.v.insert(F.v.end(), f.M.v.begin(), f.M.v.end());
+  // M's rows (thousands of entries on the level above a 641-row coarsest
+  // level) are cut into `parts` pieces; the dense coarse solve adds each
+  // row's pieces.  Pieces are consecutive slices of the row, so F's values
+  // are S's followed by M's unchanged.
+  const auto cut = [&](int64_t piece) {
+    int64_t parts = 1;
+    for (int64_t j = 0; j < f.M.n; ++j) parts = std::max(parts, (f.M.rp[j + 1] - f.M.rp[j] + piece - 1) / piece);
+    f.parts = (int)parts;
+    F.n = A.n + f.M.n * parts;
+    F.rp = S.rp;
+    F.rp.reserve((size_t)F.n + 1);
+    for (int64_t j = 0; j < f.M.n; ++j)
+      for (int64_t k = 1; k <= parts; ++k)
+        F.rp.push_back(S.nnz() + std::min(f.M.rp[j + 1], f.M.rp[j] + k * piece));
+  };
+  // A small F has padded rows: pieces as long as the rows of S have room for.
+  // Otherwise a piece is at most one row block's capacity, so that the pieces
+  // pack into ordinary row blocks instead of running as single-block long
+  // rows (31 against 13 us FP64 at 128^3).
+  const int lanes = gather_request == CFDLA_GATHER_AUTO ? ell_lanes_for(S) : 0;
+  if (lanes > 0) cut(4 * std::max(8, lanes));
+  if (lanes == 0 || ell_lanes_for(F) == 0) cut(rb_cap<double>());
   DevLevel &dl = lv[l];
   dl.F.gather_request = gather_request;
-  dl.F.upload(F, true, false, false);
+  dl.F.upload(F, true, false, false, true);
   dl.fx64.alloc((size_t)F.n);
   dl.fx32.alloc((size_t)F.n);
   f.level = (int)l;
-  f.parts = (int)parts;
   fused = std::move(f);
   return true;
 }
