@@ -423,7 +423,8 @@ void product_numeric(int nslots, const int32_t *ptr, const int32_t *pa, const in
                      const double *bv, double *cv);
 // n x n inverse of a CSR matrix by Gauss-Jordan with partial pivoting, the
 // host's operation order (throws CFDLA_ERR_NUMERICAL when singular).
-void dense_inverse_device(int n, const int32_t *rp, const int32_t *ci, const double *v, double *inv);
+void dense_inverse_device(int n, const int32_t *rp, const int32_t *ci, const double *v, double *inv,
+                          DevBuf<double> (&keep)[2]);
 
 // Sparse product (diagonal, sliced-ELL or row-block CSR) with epilogue:
 //   EPI_Y       y = A x

@@ -38,6 +38,13 @@ __device__ __forceinline__ double add_across(double v) {
          __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
 }
 template <int W>
+__device__ __forceinline__ double max_across(double v) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+  const auto lo = lane_swap<W>((unsigned)b), hi = lane_swap<W>((unsigned)(b >> 32));
+  return fmax(__builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]),
+              __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]));
+}
+template <int W>
 __device__ __forceinline__ float add_across(float v) {
   const auto p = lane_swap<W>(__builtin_bit_cast(unsigned, v));
   const unsigned a = p[0], b = p[1];  // (a bit cast of a vector's element reads its first one)

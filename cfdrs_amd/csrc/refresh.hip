@@ -21,6 +21,7 @@
 
 #include "internal.hpp"
 #include "fused_jacobi.hpp"
+#include "reduce.hpp"
 #include "simple_stencil.hpp"
 #include "solver.hpp"
 
@@ -354,146 +355,269 @@ __global__ __launch_bounds__(kBlock) void k_gj_step(int n, int c, const double *
   }
 }
 
-// Gauss-Jordan steps c0 .. c0 + B - 1 on [A | I] (column-major, entry
-// (r, j) at j n + r) in one launch, for n <= kGjMaxRows.  Every block loads
-// the B panel columns (contiguous) into LDS and
-// replays the B steps on them -- pivot row, swap, scale by d = 1 / m_pc,
-// eliminate with f = m_rc -- with the operations of k_gj_step (and of the
-// host), applying each step to its own kGjCols columns held in registers
-// (rows threadIdx.x + 256 q).  The columns left of the panel are dead, and
-// the panel's own columns are dead once its steps are done, so only columns
-// >= c0 + B are carried, src -> dst.  Each element meets the host's
+// Gauss-Jordan steps c0 .. c0 + b - 1 on [A | I] (column-major, entry
+// (r, j) at j n + r) in one launch, for n <= kGjMaxRows.  Every block replays
+// the steps on the b panel columns and applies each to its own kGjCols
+// columns, with the operations of k_gj_step (and of the host).  Thread r holds
+// row r of both in registers: m[kk] is its entry in panel column c + kk, so a
+// step writes one place to the left.  The columns left of the panel are dead,
+// and the panel's own columns are dead once its steps are done, so only
+// columns >= c0 + b are carried, src -> dst; after the last step they are the
+// inverse, stored row-major into inv.  Each element meets the host's
 // operations in the host's order, so the inverse is the host's bit for bit.
-constexpr int kGjPanel = 8;      // steps per launch (fewer when n * B * 8 B exceeds 60 KiB)
+//
+// A step is a serial chain (largest value of the column, its reciprocal, the
+// exchange of the pivot row), so it has one barrier: every wave writes its own
+// best row, scaled, beside its best value, and after the barrier all pick the
+// same winner.  The buffers alternate, so the next step's writes need no
+// barrier.  641 rows 2.25 -> 1.99 ms, 1000 rows 4.91 -> 4.57 ms against the
+// panel in LDS with four barriers per step; bound by the LDS traffic of the
+// exchanged rows (16 steps per launch write wider ones: 2.19 ms).
+constexpr int kGjPanel = 8;      // steps per launch
 constexpr int kGjCols = 4;       // columns per block
-constexpr int kGjMaxRows = 1024; // rows held by one block (4 per thread)
-constexpr int kGjPanelLds = 7680;  // doubles of the LDS panel
-__global__ __launch_bounds__(kBlock) void k_gj_panel(int n, int c0, int B, const double *src, double *dst,
-                                                     int *bad) {
+constexpr int kGjMaxRows = 1024; // one row per thread
+
+__device__ __forceinline__ double wave_max(double v) {
+  v = max_across<32>(v);
+  v = max_across<16>(v);
+  v = fmax(v, dpp_move<0x128>(v));
+  v = fmax(v, dpp_move<0x124>(v));
+  v = fmax(v, dpp_move<0x122>(v));
+  v = fmax(v, dpp_move<0x121>(v));
+  return v;
+}
+
+template <int NW>  // wavefronts per block, n <= 64 NW
+__global__ __launch_bounds__(64 * NW) void k_gj_panel(int n, int c0, int b, const double *__restrict__ src,
+                                                      double *__restrict__ dst, double *__restrict__ inv, int *bad) {
 #pragma clang fp contract(off)
-  extern __shared__ double pnl[];  // n x B, column-major: entry (r, k) at k n + r
-  __shared__ double u[kGjCols];    // row c of this block's columns, scaled
-  __shared__ double sw[2][kGjCols];
-  __shared__ int s_p;
-  constexpr int RQ = kGjMaxRows / kBlock;
+  constexpr int B = kGjPanel, W = kGjPanel + kGjCols;
+  __shared__ __align__(16) double s_row[2][NW][W];  // each wave's best row from its second entry on, scaled
+  __shared__ __align__(16) double s_c[2][W];        // row c
+  __shared__ __align__(16) double s_max[2][NW];
   if (*bad) return;  // an earlier step found the matrix singular
-  const int tid = threadIdx.x;
+  const int r = threadIdx.x, wave = r >> 6;
   const int64_t w = 2 * (int64_t)n;
-  const int64_t j0 = c0 + B + (int64_t)blockIdx.x * kGjCols;
-  for (int e = tid; e < n * B; e += kBlock) pnl[e] = src[(int64_t)c0 * n + e];
-  double x[RQ][kGjCols];
+  const int64_t j0 = c0 + b + (int64_t)blockIdx.x * kGjCols;
+  double m[W];  // panel, then this block's columns
 #pragma unroll
-  for (int q = 0; q < RQ; ++q)
+  for (int k = 0; k < B; ++k) m[k] = r < n && k < b ? src[(int64_t)(c0 + k) * n + r] : 0.0;
 #pragma unroll
-    for (int jj = 0; jj < kGjCols; ++jj) {
-      const int r = tid + q * kBlock;
-      x[q][jj] = r < n && j0 + jj < w ? src[(j0 + jj) * n + r] : 0.0;
+  for (int j = 0; j < kGjCols; ++j) m[B + j] = r < n && j0 + j < w ? src[(j0 + j) * n + r] : 0.0;
+  for (int k = 0; k < b; ++k) {
+    const int c = c0 + k, q = k & 1;
+    // row c's NaN makes the column singular, as does an infinite pivot
+    double key = -1.0;
+    if (r >= c && r < n) key = m[0] == m[0] ? fabs(m[0]) : (r == c ? HUGE_VAL : -1.0);
+    double d = 1.0 / m[0];
+    asm volatile("" : "+v"(d));  // here, where the reduction has cycles to spare, and not after it
+    const double best = wave_max(key);
+    const bool first = (r & 63) == __builtin_ctzll(__ballot(key == best));  // the wave's lowest row of that value
+    if (first) {
+      s_max[q][wave] = best;
+#pragma unroll
+      for (int j = 1; j < W; ++j) s_row[q][wave][j - 1] = m[j] * d;
     }
-  __syncthreads();
-  for (int k = 0; k < B; ++k) {
-    const int c = c0 + k;
-    Piv mine{-1.0, INT_MAX};
-    for (int r = c + tid; r < n; r += kBlock) mine = piv_better(mine, piv_of(pnl[k * n + r], r));
-    const Piv best = piv_block(mine);
-    if (tid == 0) {
-      const double mcc = pnl[k * n + c];
-      s_p = (mcc != mcc || !(best.val > 0.0 && best.val <= 1.7976931348623157e308)) ? -1 : best.row;
+    double f = m[0];
+    if (r == c) {
+      // its new row u is formed below as -0 - (-1) u, which is u for every u
+#pragma unroll
+      for (int j = 0; j < W; ++j) {
+        s_c[q][j] = m[j];
+        m[j] = -0.0;
+      }
+      f = -1.0;
     }
     __syncthreads();
-    const int p = s_p;
-    if (p < 0) {
-      if (tid == 0) *bad = 1;
+    double top = s_max[q][0];
+    int at = 0;
+#pragma unroll
+    for (int i = 1; i < NW; ++i) {
+      const bool better = s_max[q][i] > top;
+      top = better ? s_max[q][i] : top;
+      at = better ? i : at;
+    }
+    if (!(top > 0.0 && top <= 1.7976931348623157e308)) {  // the same in every thread
+      if (r == 0) *bad = 1;
       return;
     }
-    const double d = 1.0 / pnl[k * n + p];
-    if (p != c) {
-      // rows c and p trade places: the panel, then this block's columns
-      if (tid < B) {
-        const double a = pnl[tid * n + c], b = pnl[tid * n + p];
-        pnl[tid * n + c] = b;
-        pnl[tid * n + p] = a;
-      }
+    if (first && wave == at && r != c) {  // rows c and p trade places
 #pragma unroll
-      for (int q = 0; q < RQ; ++q)
-#pragma unroll
-        for (int jj = 0; jj < kGjCols; ++jj) {
-          const int r = tid + q * kBlock;
-          if (r == c) sw[0][jj] = x[q][jj];
-          if (r == p) sw[1][jj] = x[q][jj];
-        }
-      __syncthreads();
-#pragma unroll
-      for (int q = 0; q < RQ; ++q)
-#pragma unroll
-        for (int jj = 0; jj < kGjCols; ++jj) {
-          const int r = tid + q * kBlock;
-          if (r == c) x[q][jj] = sw[1][jj];
-          if (r == p) x[q][jj] = sw[0][jj];
-        }
+      for (int j = 0; j < W; ++j) m[j] = s_c[q][j];
+      f = m[0];
     }
-    __syncthreads();
-    // row c scaled by d
-    if (tid >= k && tid < B) pnl[tid * n + c] = pnl[tid * n + c] * d;
+    // every row with f != 0: m_rj - f m_cj
+    if (__builtin_expect(__ballot(f == 0.0 && r < n) != 0, 0)) {
 #pragma unroll
-    for (int q = 0; q < RQ; ++q)
-      if (tid + q * kBlock == c)
-#pragma unroll
-        for (int jj = 0; jj < kGjCols; ++jj) {
-          x[q][jj] = x[q][jj] * d;
-          u[jj] = x[q][jj];
-        }
-    __syncthreads();
-    // every other row r with f = m_rc != 0: m_rj - f m_cj
-#pragma unroll
-    for (int q = 0; q < RQ; ++q) {
-      const int r = tid + q * kBlock;
-      if (r >= n || r == c) continue;
-      const double f = pnl[k * n + r];
-      if (f == 0.0) continue;
-      for (int kk = k; kk < B; ++kk) {
-        const double t = f * pnl[kk * n + c];
-        pnl[kk * n + r] = pnl[kk * n + r] - t;
+      for (int j = 1; j < W; ++j) {
+        const double t = f * s_row[q][at][j - 1], e = m[j] - t;
+        m[j < B ? j - 1 : j] = f == 0.0 ? m[j] : e;
       }
+    } else {
 #pragma unroll
-      for (int jj = 0; jj < kGjCols; ++jj) {
-        const double t = f * u[jj];
-        x[q][jj] = x[q][jj] - t;
+      for (int j = 1; j < W; ++j) {
+        const double t = f * s_row[q][at][j - 1];
+        m[j < B ? j - 1 : j] = m[j] - t;
       }
     }
-    __syncthreads();
+    m[B - 1] = 0.0;
   }
+  if (r >= n) return;
 #pragma unroll
-  for (int q = 0; q < RQ; ++q)
-#pragma unroll
-    for (int jj = 0; jj < kGjCols; ++jj) {
-      const int r = tid + q * kBlock;
-      if (r < n && j0 + jj < w) dst[(j0 + jj) * n + r] = x[q][jj];
+  for (int j = 0; j < kGjCols; ++j)
+    if (j0 + j < w) {
+      if (inv) inv[(int64_t)r * n + (j0 + j - n)] = m[B + j];
+      else dst[(j0 + j) * n + r] = m[B + j];
     }
 }
 
-// [A | I] column-major (entry (r, j) at j n + r), for the panel path: the
-// panel and each block's columns are then contiguous.
-__global__ __launch_bounds__(kBlock) void k_dense_fill_cm(int n, double *m) {
-  for (int64_t e = blockIdx.x * (int64_t)kBlock + threadIdx.x; e < 2 * (int64_t)n * n;
-       e += (int64_t)gridDim.x * kBlock) {
-    const int64_t j = e / n, r = e - j * n;
+// The same steps for n <= 512 with one wavefront per column: up to 8 rows per
+// lane, so nothing goes through LDS or waits at a barrier.  A panel never
+// crosses a multiple of 64 (B divides 64), so slot 0 can hold the 64 rows
+// around c and the later slots the rows after them, cyclically; row c is then
+// lane c & 63 of slot 0 in every step.  On the diagonally dominant operators of a
+// hierarchy the diagonal is the pivot: one comparison per slot settles that,
+// and the search and the exchange run only where it is not.  The whole inverse
+// of 63 / 153 / 218 / 407 rows: 170 / 352 / 493 / 1144 us with the panel in LDS,
+// 125 / 251 / 341 / 715 in k_gj_panel, 91 / 152 / 224 / 585 here, about 0.7 us per
+// step at 218 rows, most of it instruction issue of the one wavefront (16 steps
+// per launch: 264, the registers of two panel widths no longer fit).  Above 512
+// rows a lane's rows don't fit its registers.
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  const long long b = __builtin_bit_cast(long long, v);
+  const unsigned lo = __builtin_amdgcn_readlane((int)b, lane), hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// Steps k .. min(k + 4, b) - 1, of which NC panel columns are left: m[s][j] is
+// the entry in column c0 + k + j, m[s][B] the one in the carried column.
+template <int RQ, int B, int NC>
+__device__ __forceinline__ bool gj_steps(int n, int c0, int k0, int b, double (&m)[RQ][B + 1]) {
+#pragma clang fp contract(off)
+  const int lane = threadIdx.x, qc = c0 >> 6;
+  const auto first_row = [&](int s) { return (qc + s < RQ ? qc + s : qc + s - RQ) * 64; };
+  for (int k = k0; k < min(k0 + 4, b); ++k) {
+    const int c = c0 + k, cl = c & 63;
+    double mcc = lane_value(m[0][0], cl), d = 1.0 / m[0][0];
+    uint64_t larger = __ballot(fabs(m[0][0]) > fabs(mcc)) & (~1ull << cl);
+#pragma unroll
+    for (int s = 1; s < RQ; ++s) {
+      const uint64_t l = __ballot(fabs(m[s][0]) > fabs(mcc));
+      larger |= qc + s < RQ ? l : 0;  // (rows past n hold zeros)
+    }
+    if (larger != 0) {
+      Piv best{-1.0, INT_MAX};
+#pragma unroll
+      for (int s = 0; s < RQ; ++s) {
+        const int row = first_row(s) + lane;
+        if (row >= c && row < n) best = piv_better(best, piv_of(m[s][0], row));
+      }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1)
+        best = piv_better(best, Piv{__shfl_xor(best.val, o, 64), __shfl_xor(best.row, o, 64)});
+      const int p = __builtin_amdgcn_readfirstlane(best.row), pl = p & 63;
+#pragma unroll
+      for (int s = 0; s < RQ; ++s)
+        if (first_row(s) == p - pl) {  // rows c and p trade places
+#pragma unroll
+          for (int j = 0; j <= B; ++j) {
+            if (j >= NC && j < B) continue;
+            const double at_c = lane_value(m[0][j], cl), at_p = lane_value(m[s][j], pl);
+            m[0][j] = lane == cl ? at_p : m[0][j];
+            m[s][j] = lane == pl ? at_c : m[s][j];
+          }
+        }
+      mcc = lane_value(m[0][0], cl);
+      d = 1.0 / m[0][0];
+    }
+    if (!(fabs(mcc) > 0.0 && fabs(mcc) <= 1.7976931348623157e308)) return false;
+    // row c scaled by d; its own row is formed below as -0 - (-1) u, which is
+    // u for every u
+    double u[B + 1], f[RQ];
+#pragma unroll
+    for (int j = 1; j <= B; ++j)
+      if (j < NC || j == B) u[j] = lane_value(m[0][j] * d, cl);
+    uint64_t zero = 0;
+#pragma unroll
+    for (int s = 0; s < RQ; ++s) {
+      f[s] = m[s][0];
+      const int rows = n - first_row(s);
+      zero |= __ballot(f[s] == 0.0) & (rows >= 64 ? ~0ull : (1ull << max(rows, 0)) - 1);
+    }
+    if (lane == cl) {
+      f[0] = -1.0;
+#pragma unroll
+      for (int j = 1; j <= B; ++j)
+        if (j < NC || j == B) m[0][j] = -0.0;
+    }
+    // every row with f != 0: m_rj - f m_cj
+    if (zero != 0) {
+#pragma unroll
+      for (int s = 0; s < RQ; ++s)
+#pragma unroll
+        for (int j = 1; j <= B; ++j) {
+          if (j >= NC && j < B) continue;
+          const double t = f[s] * u[j], e = m[s][j] - t;
+          m[s][j < B ? j - 1 : j] = f[s] == 0.0 ? m[s][j] : e;
+        }
+    } else {
+#pragma unroll
+      for (int s = 0; s < RQ; ++s)
+#pragma unroll
+        for (int j = 1; j <= B; ++j) {
+          if (j >= NC && j < B) continue;
+          const double t = f[s] * u[j];
+          m[s][j < B ? j - 1 : j] = m[s][j] - t;
+        }
+    }
+  }
+  return true;
+}
+
+template <int RQ>
+__global__ __launch_bounds__(64, RQ <= 4 ? 2 : 1) void k_gj_wave(int n, int c0, int b, const double *__restrict__ src,
+                                                double *__restrict__ dst, double *__restrict__ inv, int *bad) {
+  constexpr int B = kGjPanel;
+  static_assert(64 % B == 0, "a panel stays within 64 rows");
+  constexpr int ld = 64 * RQ;  // rows n .. ld - 1 hold zeros; the B columns after the last are there to be read
+  if (*bad) return;  // an earlier step found the matrix singular
+  const int lane = threadIdx.x, qc = c0 >> 6;
+  const int64_t col = c0 + b + (int64_t)blockIdx.x;
+  double m[RQ][B + 1];
+#pragma unroll
+  for (int s = 0; s < RQ; ++s) {
+    const int row = (qc + s < RQ ? qc + s : qc + s - RQ) * 64 + lane;
+#pragma unroll
+    for (int k = 0; k < B; ++k) m[s][k] = src[(int64_t)(c0 + k) * ld + row];
+    m[s][B] = src[col * ld + row];
+  }
+  if (!gj_steps<RQ, B, B>(n, c0, 0, b, m) || !gj_steps<RQ, B, B - 4>(n, c0, 4, b, m)) {
+    if (lane == 0) *bad = 1;
+    return;
+  }
+#pragma unroll
+  for (int s = 0; s < RQ; ++s) {
+    const int row = (qc + s < RQ ? qc + s : qc + s - RQ) * 64 + lane;
+    if (!inv) dst[col * ld + row] = m[s][B];
+    else if (row < n) inv[(int64_t)row * n + (col - n)] = m[s][B];
+  }
+}
+
+// [A | I] column-major (entry (r, j) at j ld + r, rows n .. ld - 1 zero), for
+// the panel paths: the panel and each block's columns are then contiguous.
+__global__ __launch_bounds__(kBlock) void k_dense_fill_cm(int n, int ld, int64_t count, double *m) {
+  for (int64_t e = blockIdx.x * (int64_t)kBlock + threadIdx.x; e < count; e += (int64_t)gridDim.x * kBlock) {
+    const int64_t j = e / ld, r = e - j * ld;
     m[e] = j == n + r ? 1.0 : 0.0;
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_dense_scatter_cm(int n, const int32_t *__restrict__ rp,
+__global__ __launch_bounds__(kBlock) void k_dense_scatter_cm(int n, int ld, const int32_t *__restrict__ rp,
                                                              const int32_t *__restrict__ ci,
                                                              const double *__restrict__ v, double *m) {
   for (int r = blockIdx.x; r < n; r += gridDim.x)
     for (int k = rp[r] + (int)threadIdx.x; k < rp[r + 1]; k += kBlock)
-      m[(int64_t)ci[k] * n + r] = m[(int64_t)ci[k] * n + r] + v[k];
-}
-
-__global__ __launch_bounds__(kBlock) void k_gj_extract_cm(int n, const double *m, double *inv) {
-  for (int64_t e = blockIdx.x * (int64_t)kBlock + threadIdx.x; e < (int64_t)n * n; e += (int64_t)gridDim.x * kBlock) {
-    const int64_t r = e / n, c = e - r * n;
-    inv[e] = m[(n + c) * (int64_t)n + r];
-  }
+      m[(int64_t)ci[k] * ld + r] = m[(int64_t)ci[k] * ld + r] + v[k];
 }
 
 __global__ __launch_bounds__(kBlock) void k_gj_extract(int n, const double *m, double *inv) {
@@ -684,35 +808,52 @@ void product_numeric(int nslots, const int32_t *ptr, const int32_t *pa, const in
                      dim3(kBlock), 0, stream(), nslots, ptr, pa, pb, av, bv, cv);
 }
 
-void dense_inverse_device(int n, const int32_t *rp, const int32_t *ci, const double *v, double *inv) {
-  DevBuf<double> buf[2];
-  buf[0].alloc((size_t)n * 2 * n);
-  buf[1].alloc((size_t)n * 2 * n);
-  const int nb = (n + kGjRows - 1) / kGjRows;
-  DevBuf<double> pv[2];
-  DevBuf<int> pr[2];
-  for (int k = 0; k < 2; ++k) {
-    pv[k].alloc((size_t)nb);
-    pr[k].alloc((size_t)nb);
-  }
+void dense_inverse_device(int n, const int32_t *rp, const int32_t *ci, const double *v, double *inv,
+                          DevBuf<double> (&keep)[2]) {
+  // up to kGjMaxRows rows (32 MiB) the two matrices stay with the caller
+  DevBuf<double> own[2];
+  DevBuf<double> (&buf)[2] = n <= kGjMaxRows ? keep : own;
+  const int ld = n <= 512 ? (n + 63) / 64 * 64 : n;
+  const size_t count = (size_t)ld * (2 * (size_t)n + kGjPanel);
+  buf[0].ensure(count);
+  buf[1].ensure(count);
   int *bad = flag_reset();
   if (n <= kGjMaxRows) {
-    hipLaunchKernelGGL(k_dense_fill_cm, dim3(grid_for((int64_t)n * 2 * n)), dim3(kBlock), 0, stream(), n, buf[0].p);
-    hipLaunchKernelGGL(k_dense_scatter_cm, dim3(std::min(n, kMaxBlocks)), dim3(kBlock), 0, stream(), n, rp, ci, v,
+    hipLaunchKernelGGL(k_dense_fill_cm, dim3(grid_for((int64_t)count)), dim3(kBlock), 0, stream(), n, ld,
+                       (int64_t)count, buf[0].p);
+    hipLaunchKernelGGL(k_dense_scatter_cm, dim3(std::min(n, kMaxBlocks)), dim3(kBlock), 0, stream(), n, ld, rp, ci, v,
                        buf[0].p);
-    // B steps per launch (641 launches become 81 for a 641-row level)
-    const int B = std::min(kGjPanel, kGjPanelLds / n);
+    const int B = kGjPanel, cols = n <= 512 ? 1 : kGjCols;
     int it = 0;
     for (int c0 = 0; c0 < n; c0 += B, ++it) {
       const int b = std::min(B, n - c0);
       const int64_t live = 2 * (int64_t)n - (c0 + b);
-      const int blocks = (int)((live + kGjCols - 1) / kGjCols);
-      hipLaunchKernelGGL(k_gj_panel, dim3(blocks), dim3(kBlock), (size_t)n * b * sizeof(double), stream(), n, c0,
-                         b, buf[it & 1].p, buf[(it + 1) & 1].p, bad);
+      const dim3 grid((unsigned)((live + cols - 1) / cols));
+      double *out = c0 + b == n ? inv : nullptr;
+      const auto go = [&](auto *kernel, int threads) {
+        hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, stream(), n, c0, b, buf[it & 1].p, buf[(it + 1) & 1].p,
+                           out, bad);
+      };
+      switch (n <= 512 ? ld / 64 : 0) {
+        case 1: go(k_gj_wave<1>, 64); break;
+        case 2: go(k_gj_wave<2>, 64); break;
+        case 3: go(k_gj_wave<3>, 64); break;
+        case 4: go(k_gj_wave<4>, 64); break;
+        case 5: go(k_gj_wave<5>, 64); break;
+        case 6: go(k_gj_wave<6>, 64); break;
+        case 7: go(k_gj_wave<7>, 64); break;
+        case 8: go(k_gj_wave<8>, 64); break;
+        default: go(k_gj_panel<16>, 1024);
+      }
     }
-    hipLaunchKernelGGL(k_gj_extract_cm, dim3(grid_for((int64_t)n * n)), dim3(kBlock), 0, stream(), n,
-                       buf[it & 1].p, inv);
   } else {
+    const int nb = (n + kGjRows - 1) / kGjRows;
+    DevBuf<double> pv[2];
+    DevBuf<int> pr[2];
+    for (int k = 0; k < 2; ++k) {
+      pv[k].alloc((size_t)nb);
+      pr[k].alloc((size_t)nb);
+    }
     hipLaunchKernelGGL(k_dense_fill, dim3(grid_for((int64_t)n * 2 * n)), dim3(kBlock), 0, stream(), n, buf[0].p);
     hipLaunchKernelGGL(k_dense_scatter, dim3(std::min(n, kMaxBlocks)), dim3(kBlock), 0, stream(), n, rp, ci, v,
                        buf[0].p);
@@ -722,6 +863,8 @@ void dense_inverse_device(int n, const int32_t *rp, const int32_t *ci, const dou
                          pv[c & 1].p, pr[c & 1].p, pv[(c + 1) & 1].p, pr[(c + 1) & 1].p, nb, bad);
     hipLaunchKernelGGL(k_gj_extract, dim3(grid_for((int64_t)n * n)), dim3(kBlock), 0, stream(), n, buf[n & 1].p,
                        inv);
+    CFDLA_HIP(hipGetLastError());
+    sync_stream();  // before pv and pr go
   }
   CFDLA_REQUIRE(flag_read() == 0, CFDLA_ERR_NUMERICAL,
                 "AMG coarsest operator is singular; use coarse_solver = reference sweeps");

@@ -1165,7 +1165,7 @@ void AmgPrecond::update_values_device(const double *fine_values) {
   if (tail.level >= 0) tail.refresh(lv);
   if (cfg.coarse_solver == 1) {
     const DevCsr &cA = lv.back().A;
-    dense_inverse_device(coarse_n, cA.rp.p, cA.ci.p, cA.v64.p, coarse_inv.p);
+    dense_inverse_device(coarse_n, cA.rp.p, cA.ci.p, cA.v64.p, coarse_inv.p, gj_ws);
   }
   host_stale = true;
 }

@@ -202,6 +202,7 @@ struct AmgPrecond : Precond {
   HostHierarchy host;
   std::vector<DevLevel> lv;
   DevBuf<double> coarse_inv;
+  DevBuf<double> gj_ws[2];  // the device recompute's [A | I], held once it has run
   int coarse_n = 0;
   double setup_time = 0.0;
   bool on_device = false;
