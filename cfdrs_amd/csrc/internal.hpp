@@ -309,7 +309,7 @@ struct Scal {
   int32_t nupd;   // reliable-update CG: FP64 residual replacements performed
   int32_t restart_dir;  // reliable updates: the next OP_CG_BETA / OP_BI_RHO restarts the direction (beta = 0)
   int32_t nrestart;     // reliable-update CG: replacements that restarted the direction
-  int32_t pad;
+  int32_t pad;          // 1: a kernel with a bounded wait gave up (grid_krylov.hip)
 };
 
 // Reduction workspace: two sets of block partials used in turn, so a kernel

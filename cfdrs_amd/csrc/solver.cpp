@@ -1406,9 +1406,22 @@ SolveOut pcg(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int64_t 
   Poller poll(s);
   ConvergenceGate gate;
   bool finished = false, behind = false;  // behind: a chunk is enqueued whose end has not been polled
+  bool resident = (jd || M->kind() == 0) && grid_krylov_takes<T>(A, false);
   while (!finished) {
     const Scal *h = nullptr;
-    if (enq < max_it) {
+    if (resident && enq < max_it) {
+      const int64_t steps = std::min<int64_t>(kGridSteps, max_it - enq);
+      grid_cg<T>(A, jd, x, r, p, vec<T>(11, 3 * (size_t)n), s, (int)steps);
+      const Scal now = c.read(s);
+      enq = now.iters;
+      if (now.pad) {  // the blocks never met: from here a launch per phase
+        resident = false;
+        true_residual<T>(A, b, x, r, s);
+        start_direction();
+        continue;
+      }
+      if (now.done == 0 && enq < max_it) continue;
+    } else if (enq < max_it) {
       int64_t steps = std::min<int64_t>(chunk, max_it - enq);
       for (int64_t k = 0; k < steps; ++k) {
         if (fuse && !fresh) {
@@ -1437,7 +1450,7 @@ SolveOut pcg(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int64_t 
       poll.settled();
       h = poll.latest();
     }
-    if (h->done == 0 && enq < max_it) {
+    if (h && h->done == 0 && enq < max_it) {
       if (!gate.expect(h->rr, thr * thr)) continue;
       poll.settled();
       h = poll.latest();
@@ -1671,9 +1684,24 @@ SolveOut bicgstab(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int
   int64_t enq = 0;
   Poller poll(s);
   bool finished = false, behind = false;  // behind: a chunk is enqueued whose end has not been polled
+  bool resident = (jd || M->kind() == 0) && grid_krylov_takes<T>(A, true);
   while (!finished) {
     const Scal *h = nullptr;
-    if (enq < max_it) {
+    if (resident && enq < max_it) {
+      const int64_t steps = std::min<int64_t>(kGridSteps, max_it - enq);
+      if (need_rho) dot2<T>(n, rhat, r, nullptr, nullptr, s, true, OP_BI_RHO, ws);
+      need_rho = false;
+      grid_bicgstab<T>(A, jd, x, r, rhat, p, v, ph, vec<T>(11, 4 * (size_t)n), s, (int)steps);
+      const Scal now = c.read(s);
+      enq = now.iters;
+      if (now.pad) {  // the blocks never met: from here a launch per phase
+        resident = false;
+        true_residual<T>(A, b, x, r, s);
+        restart();
+        continue;
+      }
+      if (now.done == 0 && enq < max_it) continue;
+    } else if (enq < max_it) {
       int64_t steps = std::min<int64_t>(chunk, max_it - enq);
       for (int64_t k = 0; k < steps; ++k) {
         if (need_rho) dot2<T>(n, rhat, r, nullptr, nullptr, s, true, OP_BI_RHO, ws);
@@ -1698,7 +1726,7 @@ SolveOut bicgstab(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int
       poll.settled();
       h = poll.latest();
     }
-    if (h->done == 0 && enq < max_it) continue;
+    if (h && h->done == 0 && enq < max_it) continue;
     sync_stream();
     Scal now = c.read(s);
     o.iters = now.iters;

@@ -16,6 +16,7 @@ struct Context {
   DevBuf<Scal> scal;  // kScalSlots slots and their twins
   int twin[kScalSlots] = {};  // 1: slot i's scalars are in its twin
   Pend pend{};
+  DevBuf<unsigned long long> grid_slots;  // exchanged sums of grid_krylov.hip
   Scal *host = nullptr;
   DevBuf<double> dv[12];
   DevBuf<float> fv[12];
@@ -25,6 +26,20 @@ struct Context {
   Scal read(Scal *dev);  // synchronous copy of one slot
 };
 Context &ctx();
+
+// Many iterations of a Krylov solve in one launch (grid_krylov.hip), for the
+// operators that grid_krylov_takes: up to `steps` more from the vectors and
+// scalars that the launch-per-phase loop would start them with, and back into
+// them.  edge: 3 n values of scratch for CG, 4 n for BiCGSTAB.  Scal::pad is 1
+// afterwards when a block gave up waiting; x and the scalars then are as they
+// were, r and the directions are to be formed anew.
+constexpr int kGridSteps = 2048;
+template <typename T> bool grid_krylov_takes(const DevCsr &A, bool bicg);
+template <typename T>
+void grid_cg(const DevCsr &A, const T *jd, T *x, T *r, T *p, T *edge, Scal *s, int steps);
+template <typename T>
+void grid_bicgstab(const DevCsr &A, const T *jd, T *x, T *r, const T *rhat, T *p, T *v, T *ph, T *edge, Scal *s,
+                   int steps);
 
 struct Precond {
   virtual ~Precond() = default;
