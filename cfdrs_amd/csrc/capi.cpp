@@ -604,7 +604,8 @@ cfdla_status cfdla_amg_stats(cfdla_precond p, cfdla_amg_statistics *out) {
     amg->sync_host();
     const auto &lv = amg->host.levels;
     out->num_levels = (int32_t)lv.size();
-    out->fused_level = amg->on_device ? amg->fused.level : -1;
+    // (within a dense cycle the level's sweeps and restriction are one product too)
+    out->fused_level = !amg->on_device ? -1 : amg->dense.level >= 0 ? (int)lv.size() - 2 : amg->fused.level;
     auto count = [](const HostCsr &a) {
       int64_t c = 0;
       for (double x : a.v) c += std::fabs(x) > 1e-15;

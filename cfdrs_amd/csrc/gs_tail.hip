@@ -23,8 +23,10 @@
 // vector, so it adds nothing whatever the vector holds.
 //
 // V-cycle of the 7,680 -> 3,840 -> 977 -> 250 -> 65 -> 18 row hierarchy: about
-// 760 us in launches, 154 us here (the two largest levels 70, the coarsest
-// one's 60 colour steps 28); BiCGSTAB to 1e-12 with it 11.25 -> 2.24 ms.
+// 760 us in launches, 154 us in one (the two largest levels 70, the coarsest
+// one's 60 colour steps 28); BiCGSTAB to 1e-12 with it 11.25 -> 2.24 ms.  With
+// the levels from 977 rows on as one dense operator (dense_cycle.hip) between a
+// launch down and one up, 35 us each, 1.39 ms.
 //
 // Rows of a colour are not coupled, so the update order within a colour does
 // not matter and the iterates are those of k_gs_colour bit for bit; the
@@ -78,9 +80,18 @@ struct MemRows {
   const CFDLA_GLOBAL T *v, *d, *b;
   const CFDLA_GLOBAL uint16_t *col, *row;
 };
+// (of workgroup k: the k-th right-hand side and iterate)
+template <typename T>
+__device__ __forceinline__ auto rhs_of(const TailLevelDev &D) {
+  return TailVals<T>::b(D) + (size_t)blockIdx.x * D.n;
+}
+template <typename T>
+__device__ __forceinline__ auto iterate_of(const TailLevelDev &D) {
+  return TailVals<T>::x(D) + (size_t)blockIdx.x * D.n;
+}
 template <typename T>
 __device__ __forceinline__ MemRows<T> mem_rows(const TailLevelDev &D) {
-  return {TailVals<T>::v(D), TailVals<T>::d(D), TailVals<T>::b(D), global_ptr(D.col), global_ptr(D.row)};
+  return {TailVals<T>::v(D), TailVals<T>::d(D), rhs_of<T>(D), global_ptr(D.col), global_ptr(D.row)};
 }
 
 typedef unsigned short v4u16 __attribute__((ext_vector_type(4)));
@@ -212,8 +223,13 @@ __device__ __forceinline__ void tail_sweeps(const Rows &A, const int4 *meta, int
 // their entries in LDS; b, x: the finest level's vectors; LDS: the colours'
 // meta data, two vectors u and w of the most rows of a level, and for the
 // inner levels two vectors of icap rows and their entries.
+//
+// part: TAIL_WHOLE; TAIL_DOWN to the right-hand side of level L - 1; TAIL_UP
+// from its iterate; TAIL_COLUMN the whole, workgroup k on the k-th unit vector
+// in position order, into column k of x.
+enum { TAIL_WHOLE, TAIL_DOWN, TAIL_UP, TAIL_COLUMN };
 template <typename T>
-__global__ __launch_bounds__(kTailThreads) void k_gs_tail(const TailLevelDev *__restrict__ lv, int L, int inner,
+__global__ __launch_bounds__(kTailThreads) void k_gs_tail(int part, const TailLevelDev *__restrict__ lv, int L, int inner,
                                                           int cap, int icap, int itotal,
                                                           const int4 *__restrict__ gmeta, int ncol, const T *b, T *x,
                                                           T omega, int pre, int post, int symmetric,
@@ -228,15 +244,19 @@ __global__ __launch_bounds__(kTailThreads) void k_gs_tail(const TailLevelDev *__
   for (int c = tid; c < ncol; c += kTailThreads) meta[c] = gmeta[c];
   T *u = base, *w = base + cap + 1;
   // right-hand side of the finest level in position order
-  if (inner > 0) {
-    auto bp = TailVals<T>::b(lv[0]);
-    for (int p = tid; p < lv[0].n; p += kTailThreads) bp[p] = b[global_ptr(lv[0].row)[p]];
+  auto rhs = [&](int p) {
+    return part == TAIL_COLUMN ? T(p == (int)blockIdx.x ? 1 : 0) : b[global_ptr(lv[0].row)[p]];
+  };
+  if (inner > 0 && part != TAIL_UP) {
+    auto bp = rhs_of<T>(lv[0]);
+    for (int p = tid; p < lv[0].n; p += kTailThreads) bp[p] = rhs(p);
   }
   auto lds_rows = [&](const TailLevelDev &D) {
     return LdsRows<T>{store + D.iv, store + D.id, store + D.ib, istore + D.icol, istore + D.irow};
   };
-  for (int l = 0; l < L; ++l) {
+  for (int l = part == TAIL_UP ? L : 0; l < L; ++l) {
     const TailLevelDev &D = lv[l];
+    if (part == TAIL_DOWN && l + 1 == L) return;  // its right-hand side is in memory
     if (l == inner) {
       // The larger levels' iterates are in memory now: the inner levels take
       // the LDS over.  Their first right-hand side came through memory.
@@ -253,14 +273,14 @@ __global__ __launch_bounds__(kTailThreads) void k_gs_tail(const TailLevelDev *__
           istore[I.irow + k] = global_ptr(I.row)[k];
         }
       }
-      for (int k = tid; k < D.n; k += kTailThreads) store[D.ib + k] = l == 0 ? b[global_ptr(D.row)[k]] : TailVals<T>::b(D)[k];
+      for (int k = tid; k < D.n; k += kTailThreads) store[D.ib + k] = l == 0 ? rhs(k) : rhs_of<T>(D)[k];
       __syncthreads();
     }
     const bool in = l >= inner;
     if (l + 1 == L && inv) {
       // dense coarsest level: the right-hand side in row order, one
       // wavefront per row
-      for (int p = tid; p < D.n; p += kTailThreads) w[global_ptr(D.row)[p]] = in ? store[D.ib + p] : TailVals<T>::b(D)[p];
+      for (int p = tid; p < D.n; p += kTailThreads) w[global_ptr(D.row)[p]] = in ? store[D.ib + p] : rhs_of<T>(D)[p];
       __syncthreads();
       for (int i = tid >> 6; i < D.n; i += kTailThreads / 64) {
         double acc = 0.0;
@@ -278,8 +298,8 @@ __global__ __launch_bounds__(kTailThreads) void k_gs_tail(const TailLevelDev *__
     const int4 *mt = meta + D.meta;
     const bool last = l + 1 == L;
     // the coarsest level is the pre-smoothing and 10 more sweeps (amg.rs:501)
-    for (int part = 0; part < (last ? 2 : 1); ++part) {
-      const int k = part == 0 ? pre : 10;
+    for (int more = 0; more < (last ? 2 : 1); ++more) {
+      const int k = more == 0 ? pre : 10;
       if (in) {
         const LdsRows<T> A = lds_rows(D);
         tail_sweeps<T>(A, mt, D.nc, omega, k, symmetric, u);
@@ -296,7 +316,7 @@ __global__ __launch_bounds__(kTailThreads) void k_gs_tail(const TailLevelDev *__
     } else {
       const MemRows<T> A = mem_rows<T>(D);
       for (int c = 0; c < D.nc; ++c) tail_colour<T, true>(A, uniform(mt[c]), omega, u, w);
-      auto xl = TailVals<T>::x(D);
+      auto xl = iterate_of<T>(D);
       for (int i = tid; i < D.n; i += kTailThreads) xl[i] = u[i];
     }
     __syncthreads();
@@ -306,17 +326,23 @@ __global__ __launch_bounds__(kTailThreads) void k_gs_tail(const TailLevelDev *__
       T sum[1];
       tail_rows<T, 1>(global_ptr(D.rcol) + p * D.rw, TailVals<T>::r(D) + p * D.rw, D.rw, 0, w, sum);
       if (in) store[C.ib + p] = sum[0];
-      else TailVals<T>::b(C)[p] = sum[0];
+      else rhs_of<T>(C)[p] = sum[0];
     }
+    __syncthreads();
+  }
+  if (part == TAIL_UP) {
+    auto xc = iterate_of<T>(lv[L - 1]);
+    for (int i = tid; i < lv[L - 1].n; i += kTailThreads) u[i] = xc[i];
+    if (tid == 0) u[lv[L - 1].n] = T(0);
     __syncthreads();
   }
   for (int l = L - 2; l >= 0; --l) {
     const TailLevelDev &D = lv[l];
     const bool in = l >= inner;
-    if (l + 1 == inner) {
+    if (l + 1 == inner && part != TAIL_UP) {
       // back to the larger levels: the coarse iterate moves behind the room
       // of the level's own, through memory
-      auto xc = TailVals<T>::x(lv[inner]);
+      auto xc = iterate_of<T>(lv[inner]);
       const int nc = lv[inner].n;
       for (int i = tid; i < nc; i += kTailThreads) xc[i] = u[i];
       __syncthreads();
@@ -333,7 +359,7 @@ __global__ __launch_bounds__(kTailThreads) void k_gs_tail(const TailLevelDev *__
         w[i] = store[D.ix + i] + sum[0];
       }
     } else {
-      auto xl = TailVals<T>::x(D);
+      auto xl = iterate_of<T>(D);
       for (int i = tid; i < D.n; i += kTailThreads) {
         T sum[1];
         tail_rows<T, 1>(global_ptr(D.pcol) + i * D.pw, TailVals<T>::p(D) + i * D.pw, D.pw, 0, u, sum);
@@ -355,7 +381,7 @@ __global__ __launch_bounds__(kTailThreads) void k_gs_tail(const TailLevelDev *__
     }
   }
   const int n0 = lv[0].n;
-  for (int i = tid; i < n0; i += kTailThreads) x[i] = u[i];
+  for (int i = tid; i < n0; i += kTailThreads) x[(size_t)blockIdx.x * n0 + i] = u[i];
 }
 
 // Slot values from the level's CSR values (src: CSR slot or -1), after a device refresh.
@@ -555,6 +581,17 @@ void GsTail::build(const HostHierarchy &h, int first, const std::vector<std::vec
   lds_vals = inner > 0 ? 2 * (cap + 1) : 0;
   lds_words = iwords;
   ncolours = (int)meta.size() / 4;
+  // The dense operator: from the first small level behind the first one.  A
+  // hierarchy that fits in LDS whole (inner = 0) runs there faster than in
+  // three launches.
+  dense.level = -1;
+  for (int q = inner; q >= 1 && desc[(size_t)std::min<int>(q, (int)desc.size() - 1)].n <= kDenseCycleRows; --q)
+    if (q < (int)desc.size()) dense.level = q;
+  if (dense.level >= 0) {
+    dense.n = desc[(size_t)dense.level].n;
+    dense.ld = (dense.n + 15) / 16 * 16;
+    dense.c.ensure((size_t)dense.n * (size_t)dense.ld);
+  }
   d_meta.upload(meta.data(), meta.size());
   d_desc.upload(desc.data(), desc.size());
   sync_stream();
@@ -579,17 +616,69 @@ void GsTail::refresh(const std::vector<DevLevel> &dev) {
   CFDLA_HIP(hipGetLastError());
 }
 
+namespace {
+template <typename T> T *tail_rhs(const TailLevel &t);
+template <> double *tail_rhs<double>(const TailLevel &t) { return t.b64.p; }
+template <> float *tail_rhs<float>(const TailLevel &t) { return t.b32.p; }
+template <typename T> T *tail_iterate(const TailLevel &t);
+template <> double *tail_iterate<double>(const TailLevel &t) { return t.x64.p; }
+template <> float *tail_iterate<float>(const TailLevel &t) { return t.x32.p; }
+
+// The LDS of k_gs_tail: the 16-bit words follow the inner levels' values,
+// inside or past the larger levels' two vectors.
+size_t tail_bytes(const GsTail &t, size_t elem) {
+  return std::max((size_t)t.lds_vals * elem,
+                  (2 * ((size_t)t.icap + 1) + t.itotal) * elem + (size_t)t.lds_words * sizeof(uint16_t));
+}
+}  // namespace
+
+// The columns of the dense operator, one workgroup each, with the larger of
+// its levels' vectors in memory once per column.
+void GsTail::form_dense(double omega, int pre, int post, bool symmetric, const double *inv) {
+  const size_t L = lv.size(), q0 = (size_t)dense.level;
+  std::vector<TailLevelDev> desc(L);
+  if (dense.ws.empty()) {
+    dense.ws.resize(1 + 2 * (L - q0));
+    dense.ws[0].ensure((size_t)dense.n * (size_t)dense.n);
+    d_desc.download(desc.data(), L);
+    sync_stream();
+    for (size_t q = q0; q < L && q <= (size_t)inner; ++q) {
+      const size_t count = (size_t)dense.n * (size_t)desc[q].n;
+      DevBuf<double> &b = dense.ws[1 + 2 * (q - q0)], &x = dense.ws[2 + 2 * (q - q0)];
+      b.ensure(count);
+      x.ensure(count);
+      desc[q].b64 = b.p;
+      desc[q].x64 = x.p;
+    }
+    d_column.upload(desc.data(), L);
+    sync_stream();
+  }
+  hipLaunchKernelGGL((k_gs_tail<double>), dim3((unsigned)dense.n), dim3(kTailThreads), tail_bytes(*this, sizeof(double)),
+                     stream(), (int)TAIL_COLUMN, d_column.p + q0, (int)(L - q0), inner - (int)q0, dense.n, icap, itotal,
+                     reinterpret_cast<const int4 *>(d_meta.p), ncolours, (const double *)nullptr, dense.ws[0].p, omega,
+                     pre, post, symmetric ? 1 : 0, inv, (Scal *)nullptr, 0);
+  CFDLA_HIP(hipGetLastError());
+  dense.from_columns(dense.ws[0].p);
+}
+
 template <typename T>
 void gs_tail(const GsTail &t, const T *b, T *x, double omega, int pre, int post, bool symmetric, const double *inv,
              Scal *s, bool check_done) {
-  // the 16-bit words follow the inner levels' values, inside or past the
-  // larger levels' two vectors
-  const size_t bytes = std::max((size_t)t.lds_vals * sizeof(T),
-                                (2 * ((size_t)t.icap + 1) + t.itotal) * sizeof(T) + (size_t)t.lds_words * sizeof(uint16_t));
   s = settled_scal(s);
-  hipLaunchKernelGGL((k_gs_tail<T>), dim3(1), dim3(kTailThreads), bytes, stream(), t.d_desc.p, (int)t.lv.size(),
-                     t.inner, t.cap, t.icap, t.itotal, reinterpret_cast<const int4 *>(t.d_meta.p), t.ncolours, b, x,
-                     (T)omega, pre, post, symmetric ? 1 : 0, inv, s, check_done ? 1 : 0);
+  const auto run = [&](int part, int L, int inner) {
+    hipLaunchKernelGGL((k_gs_tail<T>), dim3(1), dim3(kTailThreads), tail_bytes(t, sizeof(T)), stream(), part,
+                       t.d_desc.p, L, inner, t.cap, t.icap, t.itotal, reinterpret_cast<const int4 *>(t.d_meta.p),
+                       t.ncolours, b, x, (T)omega, pre, post, symmetric ? 1 : 0, inv, s, check_done ? 1 : 0);
+  };
+  const int q = t.dense.level;
+  if (q >= 0) {
+    const TailLevel &D = t.lv[(size_t)q];
+    run(TAIL_DOWN, q + 1, t.inner);
+    t.dense.apply<T>(tail_rhs<T>(D), tail_iterate<T>(D), s, check_done);
+    run(TAIL_UP, q + 1, t.inner);
+  } else {
+    run(TAIL_WHOLE, (int)t.lv.size(), t.inner);
+  }
   CFDLA_HIP(hipGetLastError());
 }
 template void gs_tail<double>(const GsTail &, const double *, double *, double, int, int, bool, const double *, Scal *,

@@ -1006,10 +1006,17 @@ void AmgPrecond::upload() {
     d.t64.alloc(n); d.r64.alloc(n); d.t32.alloc(n); d.r32.alloc(n);
   }
   fused = FusedOp{};
-  if (L >= 3 && cfg.smoother == 2 && cfg.coarse_solver == 1 && cfg.pre_smooth_iterations == 2 &&
-      !cfg.separate_coarse_restriction)
-    build_fused(L - 2);
+  dense.level = -1;
   coarse_n = (int)host.levels.back().A.n;
+  if (L >= 3 && cfg.smoother == 2 && cfg.coarse_solver == 1 && cfg.pre_smooth_iterations == 2 &&
+      !cfg.separate_coarse_restriction) {
+    // The finest small level but the first; a forced gather layout asks for
+    // the row-block products of every level.  A dense coarsest level of more
+    // than 512 rows makes forming the operator dear.
+    if (gather_request == CFDLA_GATHER_AUTO && coarse_n <= 512)
+      for (size_t l = L - 2; l >= 1 && host.levels[l].A.n <= kDenseCycleRows; --l) dense.level = (int)l;
+    if (dense.level < 0) build_fused(L - 2);
+  }
   if (cfg.coarse_solver == 1) {
     CFDLA_REQUIRE(coarse_n <= 8192, CFDLA_ERR_CONFIG,
                   "AMG coarsest level too large for the dense direct solve; raise max_levels");
@@ -1021,8 +1028,18 @@ void AmgPrecond::upload() {
     const int first = gs_tail_first(host, gs_order, gs_off, cfg.coarse_solver == 1);
     if (first >= 0) tail.build(host, first, gs_order, gs_off);
   }
+  form_dense();
+  for (auto *d : {&dense, &tail.dense}) d->ws.clear();
   sync_stream();
   on_device = true;
+}
+
+void AmgPrecond::form_dense() {
+  const double *inv = cfg.coarse_solver == 1 ? coarse_inv.p : nullptr;
+  if (dense.level >= 0) dense.form_jacobi(lv, cfg, inv);
+  if (tail.level >= 0 && tail.dense.level >= 0)
+    tail.form_dense(cfg.relaxation_factor, cfg.pre_smooth_iterations, cfg.post_smooth_iterations, cfg.smoother == 1,
+                    inv);
 }
 
 void AmgPrecond::update_values(const double *values) {
@@ -1167,6 +1184,7 @@ void AmgPrecond::update_values_device(const double *fine_values) {
     const DevCsr &cA = lv.back().A;
     dense_inverse_device(coarse_n, cA.rp.p, cA.ci.p, cA.v64.p, coarse_inv.p, gj_ws);
   }
+  form_dense();
   host_stale = true;
 }
 
@@ -1182,6 +1200,7 @@ T *AmgPrecond::first_sweep_target(int l) {
   DevLevel &L = lv[(size_t)l];
   const bool coarsest = (size_t)l + 1 == lv.size();
   if (coarsest && cfg.coarse_solver == 1) return nullptr;
+  if (l == dense.level) return nullptr;
   if (l == fused.level) return nullptr;  // the fused product starts from b alone
   const int down = coarsest ? cfg.pre_smooth_iterations + 10 : cfg.pre_smooth_iterations;
   const int up = coarsest ? 0 : cfg.post_smooth_iterations;
@@ -1247,6 +1266,11 @@ void AmgPrecond::vcycle(int l, const T *b, T *x, Scal *s, bool chk, int dot_op, 
   const bool coarsest = (size_t)l + 1 == lv.size();
   const double w = cfg.relaxation_factor;
   const T *dinv = L.A.sdinv<T>();
+  if (l == dense.level) {
+    dense.apply<T>(b, x, s, chk);
+    if (dot_op != OP_NONE) dot2<T>(n, b, x, nullptr, nullptr, s, chk, dot_op, ws);
+    return;
+  }
   if (coarsest && cfg.coarse_solver == 1) {
     dense_gemv<T>(n, coarse_inv.p, b, x, s, chk);
     if (dot_op != OP_NONE) dot2<T>(n, b, x, nullptr, nullptr, s, chk, dot_op, ctx().ws);

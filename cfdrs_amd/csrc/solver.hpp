@@ -184,6 +184,18 @@ constexpr int kTailRows = kTailLds / 16 - 1;
 constexpr int64_t kTailNnzPerColour = 32000;
 // Rows of a dense coarsest level that one workgroup multiplies in a few us.
 constexpr int kTailDenseRows = 256;
+// The V-cycle from `level` on as a dense operator (dense_cycle.hip).
+constexpr int kDenseCycleRows = 2048;
+struct DenseCycle {
+  int level = -1;  // (-1: none)
+  int n = 0, ld = 0;
+  DevBuf<double> c;                // row-major, rows of ld
+  std::vector<DevBuf<double>> ws;  // scratch of a forming, kept for the next one after a device recompute
+  template <typename T> void apply(const T *b, T *x, Scal *s, bool check_done) const;
+  void form_jacobi(std::vector<DevLevel> &lv, const cfdla_amg_config &cfg, const double *inv);
+  void from_columns(const double *columns);  // c from its columns, one after the other
+};
+
 struct GsTail {
   int level = -1;  // first level of the tail (-1: none)
   int cap = 0;     // the most rows of its levels
@@ -194,8 +206,14 @@ struct GsTail {
   DevBuf<int32_t> d_meta;  // 4 per colour: first position, rows, first slot, slots per row
   void build(const HostHierarchy &h, int first, const std::vector<std::vector<int32_t>> &order,
              const std::vector<std::vector<int32_t>> &off);
+  // The tail's levels from dense.level (an index into lv) on as one operator
+  // on right-hand sides in position order; columns: d_column is the levels'
+  // description with a right-hand side and an iterate per column.
+  DenseCycle dense;
+  DevBuf<TailLevelDev> d_column;
   // entries and diagonals from the levels' device values
   void refresh(const std::vector<DevLevel> &dev);
+  void form_dense(double omega, int pre, int post, bool symmetric, const double *inv);
 };
 int gs_tail_first(const HostHierarchy &h, const std::vector<std::vector<int32_t>> &order,
                   const std::vector<std::vector<int32_t>> &off, bool direct);
@@ -229,6 +247,8 @@ struct AmgPrecond : Precond {
   // Jacobi with two pre-sweeps (level -1: none).
   FusedOp fused;
   GsTail tail;  // the small levels of a Gauss-Seidel hierarchy
+  DenseCycle dense;  // the last levels of a Jacobi hierarchy
+  void form_dense();
   bool build_fused(size_t l);
   void refresh_fused_device();
   // AlgebraicMultigrid::recompute (amg.rs:179-214) on the device from
