@@ -132,10 +132,10 @@ __device__ __forceinline__ double swap_add(double a, double b) {
 }
 
 // part[k * nb + blockIdx.x] = the block's sum of accumulator k, k < jp1
-template <int JB>
+template <int JB, int THREADS>
 __device__ __forceinline__ void block_sums(double (&acc)[JB], int jp1, double *__restrict__ part) {
   static_assert(JB % 4 == 0, "four rows of 16 lanes hold a quarter of the sums each");
-  __shared__ double sh[kBlock / 64][JB];
+  __shared__ double sh[THREADS / 64][JB];
   constexpr int Q = JB / 4;
   double half[2 * Q], quarter[Q];
 #pragma unroll
@@ -153,10 +153,10 @@ __device__ __forceinline__ void block_sums(double (&acc)[JB], int jp1, double *_
     if ((lane & 15) == 0) sh[wave][(lane >> 4) * Q + k] = v;  // row r of lanes: sums r Q .. r Q + Q - 1
   }
   __syncthreads();
-  for (int k = threadIdx.x; k < jp1; k += kBlock) {
+  for (int k = threadIdx.x; k < jp1; k += THREADS) {
     double t = 0.0;
 #pragma unroll
-    for (int w = 0; w < kBlock / 64; ++w) t += sh[w][k];
+    for (int w = 0; w < THREADS / 64; ++w) t += sh[w][k];
     part[(size_t)k * gridDim.x + blockIdx.x] = t;
   }
 }
@@ -198,8 +198,114 @@ __global__ __launch_bounds__(kBlock) void k_gram(int n, int jp1, const T *__rest
     }
     if constexpr (NORM) nv[0] += (double)wn * (double)wn;
   }
-  if constexpr (DOTS) block_sums<JB>(acc, jp1, part);
+  if constexpr (DOTS) block_sums<JB, kBlock>(acc, jp1, part);
   if constexpr (NORM) block_partials<1>(nv, part);
+}
+
+// ---- the same passes with one element per thread -------------------------------
+// Up to kRowBlocks blocks of 1024 rows: so few partials that the next pass's
+// blocks sum them themselves, each wavefront a vector's, while their own
+// entries are in flight, instead of a launch between (k_mdot_fin, 2.7 us); and
+// the first pass forms its element of w itself where A is diagonal storage,
+// which saves the product's launch (3.6 us).  Bound: the basis bytes out of the
+// Infinity Cache for long bases, two round trips of latency for short ones.  384
+// x 384 momentum matrix, 8 / 16 / 24 / 32 vectors: dots with the product 6.1 /
+// 7.4 / 9.2 / 10.7 us, update and dots 5.1 / 6.8 / 8.2 / 10.3, update and norm 4.6 /
+// 5.7 / 6.4 / 8.2; a step 36 -> 27 us with the start of the sweep in the scaling
+// (k_gm_arnoldi_sor), GMRES(30) with SOR there 8.9 -> 6.7 ms.  (Smaller blocks,
+// one on every CU, cost more in the partials: 6.9 ms; visiting the vectors
+// backwards in every other pass gained nothing.)
+// PASS_DOTS: dots of w; PASS_PRODUCT: w = A z and its dots; PASS_BOTH: w -=
+// sum_k h_k V_k, then dots; PASS_LAST: w -= sum_k h_k V_k and its norm.  h from
+// in (nb partials per vector); hc collects them over the two passes.
+constexpr int kRowThreads = 1024;
+constexpr int kRowBlocks = 256;
+enum { PASS_DOTS, PASS_PRODUCT, PASS_BOTH, PASS_LAST };
+template <typename T, int JB, int PASS, int NS>
+__global__ __launch_bounds__(kRowThreads) void k_gram_row(int n, int jp1, const T *__restrict__ V, size_t ld,
+                                                          DiaRows A, const T *__restrict__ av,
+                                                          const T *__restrict__ z, const double *__restrict__ in,
+                                                          double *__restrict__ hc, T *__restrict__ w, const Scal *s,
+                                                          double *__restrict__ out) {
+  if (s->done) return;
+  constexpr int W = kRowThreads / 64;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nb = gridDim.x;
+  const int mine = blockIdx.x * kRowThreads + tid;
+  const bool live = mine < n;
+  const int i = live ? mine : n - 1;
+  constexpr bool UPDATE = PASS == PASS_BOTH || PASS == PASS_LAST;
+  constexpr int R = (JB + W - 1) / W, Q = kRowBlocks / 64;
+  // the partials first: loads return in order, and h is summed while the
+  // entries are on their way
+  double hv[R][Q];
+  if constexpr (UPDATE) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const int k = min(wave + r * W, jp1 - 1), b = lane + 64 * q;
+        const double t = in[(size_t)k * nb + min(b, nb - 1)];
+        hv[r][q] = b < nb ? t : 0.0;
+      }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  T v[JB];
+#pragma unroll
+  for (int k = 0; k < JB; ++k) v[k] = V[(size_t)min(k, jp1 - 1) * ld + i];
+  double wn;
+  if constexpr (PASS == PASS_PRODUCT) {
+    T a[NS], g[NS];
+#pragma unroll
+    for (int q = 0; q < NS; ++q) {
+      const int c = i + A.off[q];
+      const bool ok = q < A.count && c >= 0 && c < n;
+      const T e = av[(size_t)A.k[q] * n + (ok && A.lower[q] ? c : i)];
+      a[q] = ok ? e : T(0);
+      g[q] = z[ok ? c : i];
+    }
+    T sum = T(0);
+#pragma unroll
+    for (int q = 0; q < NS; ++q) sum += a[q] != T(0) ? a[q] * g[q] : T(0);
+    wn = (double)sum;
+    if (live) w[i] = sum;
+  } else {
+    wn = (double)w[i];
+  }
+  if constexpr (UPDATE) {
+    __shared__ double h[R * W];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      double t = hv[r][0];
+#pragma unroll
+      for (int q = 1; q < Q; ++q) t += hv[r][q];
+      t = wave_sum(t);
+      if (lane == 0) h[wave + r * W] = t;
+    }
+    __syncthreads();
+    if (blockIdx.x == 0 && tid < jp1) hc[tid] = PASS == PASS_BOTH ? h[tid] : hc[tid] + h[tid];
+#pragma unroll
+    for (int k = 0; k < JB; ++k)
+      if (k < jp1) wn -= h[k] * (double)v[k];
+    const T t = (T)wn;
+    wn = (double)t;
+    if (live) w[i] = t;
+  }
+  if constexpr (PASS == PASS_LAST) {
+    __shared__ double sh[W];
+    const double t = wave_sum(live ? wn * wn : 0.0);
+    if (lane == 0) sh[wave] = t;
+    __syncthreads();
+    if (wave == 0) {
+      const double sum = wave_sum(lane < W ? sh[lane] : 0.0);
+      if (lane == 0) out[blockIdx.x] = sum;
+    }
+  } else {
+    double acc[JB];
+#pragma unroll
+    for (int k = 0; k < JB; ++k) acc[k] = live ? (double)v[k] * wn : 0.0;
+    block_sums<JB, kRowThreads>(acc, jp1, out);
+  }
 }
 
 // ||w|| from its partials, v_{j+1} = w / ||w|| in place, and (block 0) the
@@ -209,58 +315,46 @@ __global__ __launch_bounds__(kBlock) void k_gram(int n, int jp1, const T *__rest
 // earlier rotations in LDS, so thread 0's rotation chain waits on arithmetic,
 // not on global memory, beside the other blocks' scaling (4.8 us; 3.7 + 2.9 us
 // with the scaling as a launch of its own, 147,456 rows).
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_gm_arnoldi(int j, int n, T *__restrict__ w, int nblocks,
-                                                       const double *partials, const Scal *in, Scal *out, GmLayout L) {
-  __shared__ double col[258], cs[256], sn[256];
+struct Column {
+  double h[258], cs[256], sn[256];
+  Scal sc;
+};
+// block 0, before the norm is summed
+__device__ __forceinline__ void load_column(Column &c, int j, const Scal *in, const GmLayout &L) {
   const int tid = threadIdx.x;
-  constexpr int kWords = sizeof(Scal) / sizeof(int);
-  const bool first = blockIdx.x == 0;
-  if (in->done) {
-    if (first && tid < kWords) reinterpret_cast<int *>(out)[tid] = reinterpret_cast<const int *>(in)[tid];
-    return;
+  if (tid < (int)(sizeof(Scal) / sizeof(int))) reinterpret_cast<int *>(&c.sc)[tid] = reinterpret_cast<const int *>(in)[tid];
+  for (int k = tid; k <= j; k += kBlock) c.h[k] = L.hc[k];
+  for (int k = tid; k < j; k += kBlock) {
+    c.cs[k] = L.cs[k];
+    c.sn[k] = L.sn[k];
   }
-  const int i0 = blockIdx.x * kBlock + tid, step = gridDim.x * kBlock;
-  T w0 = T(0);
-  if (i0 < n) w0 = w[i0];
-  __shared__ Scal sc;
-  if (first) {
-    if (tid < kWords) reinterpret_cast<int *>(&sc)[tid] = reinterpret_cast<const int *>(in)[tid];
-    for (int k = tid; k <= j; k += kBlock) col[k] = L.hc[k];
-    for (int k = tid; k < j; k += kBlock) {
-      cs[k] = L.cs[k];
-      sn[k] = L.sn[k];
-    }
-  }
-  double tot[1];
-  sum_partials<1>(nblocks, partials, tot);  // synchronizes the block
-  const double hn = sqrt(tot[0]);
-  const double a = hn > 0.0 ? 1.0 / hn : 0.0;
-  // (a breakdown or a non-finite norm ends the cycle: the vector is not used)
-  for (int i = i0; i < n; i += step) w[i] = (T)((double)(i == i0 ? w0 : w[i]) * a);
-  if (!first) return;
-  const int m = L.m;
+}
+// block 0, with the norm hn and its reciprocal a
+__device__ __forceinline__ void finish_column(Column &c, int j, double hn, double a, Scal *out, const GmLayout &L) {
+  const int tid = threadIdx.x, m = L.m;
   if (tid == 0) {
+    Scal &sc = c.sc;
+    double *col = c.h;
     sc.hn = hn;
     col[j + 1] = hn;
     for (int k = 0; k < j; ++k) {
       const double t0 = col[k], t1 = col[k + 1];
-      col[k] = cs[k] * t0 + sn[k] * t1;
-      col[k + 1] = -sn[k] * t0 + cs[k] * t1;
+      col[k] = c.cs[k] * t0 + c.sn[k] * t1;
+      col[k + 1] = -c.sn[k] * t0 + c.cs[k] * t1;
     }
     const double h0 = col[j], h1 = col[j + 1];
     const double den = hypot(h0, h1);
     if (den == 0.0 || !isfinite(den)) {
       sc.done = 4;  // breakdown: the cycle ends with kstep = j
     } else {
-      const double c = h0 / den, sj = h1 / den;
-      L.cs[j] = c;
+      const double cj = h0 / den, sj = h1 / den;
+      L.cs[j] = cj;
       L.sn[j] = sj;
       col[j] = den;
       col[j + 1] = 0.0;
       const double gj = L.g[j];
       L.g[j + 1] = -sj * gj;
-      L.g[j] = c * gj;
+      L.g[j] = cj * gj;
       sc.kstep = j + 1;
       sc.iters += 1;
       sc.alpha = a;
@@ -268,10 +362,100 @@ __global__ __launch_bounds__(kBlock) void k_gm_arnoldi(int j, int n, T *__restri
     }
   }
   __syncthreads();
-  if (tid < kWords) reinterpret_cast<int *>(out)[tid] = reinterpret_cast<const int *>(&sc)[tid];
+  if (tid < (int)(sizeof(Scal) / sizeof(int))) reinterpret_cast<int *>(out)[tid] = reinterpret_cast<const int *>(&c.sc)[tid];
   // the column as the host-visible Hessenberg H(0:j+1, j); on breakdown the
   // rotated entries up to j + 1, as before the rotation that failed
-  for (int k = tid; k <= j + 1; k += kBlock) L.H[(size_t)k * m + j] = col[k];
+  for (int k = tid; k <= j + 1; k += kBlock) L.H[(size_t)k * m + j] = c.h[k];
+}
+__device__ __forceinline__ void keep_scal(const Scal *in, Scal *out) {
+  const int tid = threadIdx.x;
+  if (blockIdx.x == 0 && tid < (int)(sizeof(Scal) / sizeof(int)))
+    reinterpret_cast<int *>(out)[tid] = reinterpret_cast<const int *>(in)[tid];
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_gm_arnoldi(int j, int n, T *__restrict__ w, int nblocks,
+                                                       const double *partials, const Scal *in, Scal *out, GmLayout L) {
+  __shared__ Column c;
+  const int tid = threadIdx.x;
+  const bool first = blockIdx.x == 0;
+  if (in->done) {
+    keep_scal(in, out);
+    return;
+  }
+  const int i0 = blockIdx.x * kBlock + tid, step = gridDim.x * kBlock;
+  T w0 = T(0);
+  if (i0 < n) w0 = w[i0];
+  if (first) load_column(c, j, in, L);
+  double tot[1];
+  sum_partials<1>(nblocks, partials, tot);  // synchronizes the block
+  const double hn = sqrt(tot[0]);
+  const double a = hn > 0.0 ? 1.0 / hn : 0.0;
+  // (a breakdown or a non-finite norm ends the cycle: the vector is not used)
+  for (int i = i0; i < n; i += step) w[i] = (T)((double)(i == i0 ? w0 : w[i]) * a);
+  if (first) finish_column(c, j, hn, a, out, L);
+}
+
+// The same with v_{j+1} = w / ||w|| going to its own place and, in the same
+// launch, the start of the multicolour sweep on it (k_sor_start in
+// kernels.hip: the first colour z_i = piv_i v_i, the second from the first's
+// values formed at the gathers; the other colours 0).  The neighbours' entries
+// of v are formed from w as the own one is, so z has the bits of the sweep on
+// the stored v.
+template <typename T, int W>
+__global__ __launch_bounds__(kBlock) void k_gm_arnoldi_sor(int j, int n, const T *__restrict__ w, T *__restrict__ v,
+                                                           T *__restrict__ z, const uint8_t *__restrict__ cls,
+                                                           const int *__restrict__ ci, const T *__restrict__ sv,
+                                                           const T *__restrict__ piv, int nblocks,
+                                                           const double *partials, const Scal *in, Scal *out,
+                                                           GmLayout L) {
+  __shared__ Column c;
+  const bool first = blockIdx.x == 0;
+  if (in->done) {
+    keep_scal(in, out);
+    return;
+  }
+  if (first) load_column(c, j, in, L);
+  double hn = 0.0, a = 0.0;
+  bool summed = false;
+  for (int base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock) {
+    const bool live = base + (int)threadIdx.x < n;
+    const int i = live ? base + (int)threadIdx.x : n - 1;
+    const int k = cls[i];
+    const T pi = piv[i], wi = w[i];
+    int col[W];
+    T e[W], pj[W], wj[W];
+#pragma unroll
+    for (int q = 0; q < W; ++q) {
+      col[q] = ci[(size_t)q * n + i];
+      e[q] = sv[(size_t)q * n + i];
+    }
+#pragma unroll
+    for (int q = 0; q < W; ++q) {
+      pj[q] = piv[col[q]];
+      wj[q] = w[col[q]];
+    }
+    if (!summed) {
+      double tot[1];
+      sum_partials<1>(nblocks, partials, tot);  // synchronizes the block
+      hn = sqrt(tot[0]);
+      a = hn > 0.0 ? 1.0 / hn : 0.0;
+      summed = true;
+    }
+    const T ri = (T)((double)wi * a);
+    T acc = ri;
+#pragma unroll
+    for (int q = 0; q < W; ++q)
+      if (col[q] != i) {
+        const T zj = pj[q] * (T)((double)wj[q] * a);
+        acc -= e[q] * zj;
+      }
+    if (live) {
+      v[i] = ri;
+      z[i] = k > 1 ? T(0) : pi * acc;
+    }
+  }
+  if (first) finish_column(c, j, hn, a, out, L);
 }
 
 // Back substitution H(0:k,0:k) y = g(0:k), k = kstep, by one wavefront: the
@@ -420,6 +604,48 @@ SolveOut gmres(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int64_
     }
     return eb;
   };
+  // One row per thread, as long as the blocks' partials are few (above, and
+  // for a basis of more than 32 vectors: gram).
+  const DiaRows rows = dia_rows<T>(A);
+  const int rb = (n + kRowThreads - 1) / kRowThreads;
+  const bool by_row = rb <= kRowBlocks && m <= 32;
+  auto gram_row = [&](int j, const T *zj, T *w, Scal *sc) {
+    const int jp1 = j + 1;
+    double *part[2] = {L.part, L.part + (size_t)(m + 1) * kRowBlocks};
+    const T *av = rows.count > 0 ? A.dia_vals<T>() : nullptr;
+    if (rows.count == 0) csr_apply<T>(A, EPI_Y, zj, nullptr, nullptr, 0.0, w, sc, true, OP_NONE, nullptr, ws);
+    const auto go = [&](auto *kernel, const double *in, double *out) {
+      hipLaunchKernelGGL(kernel, dim3(rb), dim3(kRowThreads), 0, stream(), n, jp1, V, ld, rows, av, zj, in, L.hc, w,
+                         sc, out);
+    };
+#define CFDLA_GRAM_ROW(JB)                                                                  \
+  do {                                                                                      \
+    if (rows.count == 0) go(k_gram_row<T, JB, PASS_DOTS, 1>, nullptr, part[0]);              \
+    else if (rows.count <= 5) go(k_gram_row<T, JB, PASS_PRODUCT, 5>, nullptr, part[0]);      \
+    else go(k_gram_row<T, JB, PASS_PRODUCT, kDiaRowMax>, nullptr, part[0]);                  \
+    go(k_gram_row<T, JB, PASS_BOTH, 1>, part[0], part[1]);                                   \
+    go(k_gram_row<T, JB, PASS_LAST, 1>, part[1], ws.current());                              \
+  } while (0)
+    if (jp1 <= 8) CFDLA_GRAM_ROW(8);
+    else if (jp1 <= 16) CFDLA_GRAM_ROW(16);
+    else if (jp1 <= 24) CFDLA_GRAM_ROW(24);
+    else CFDLA_GRAM_ROW(32);
+#undef CFDLA_GRAM_ROW
+    return rb;
+  };
+  // a multicolour sweep whose start takes the scaling of its argument along
+  auto *sor = by_row ? dynamic_cast<ColoredSorPrecond *>(M) : nullptr;
+  if (sor && sor->start_w == 0) sor = nullptr;
+  T *wt = sor ? vec<T>(3, n) : nullptr;
+  auto arnoldi_sor = [&](const ColoredSorPrecond &p, int j, const T *w, T *v, int parts, const Scal *in, Scal *out) {
+    const auto go = [&](auto *kernel) {
+      hipLaunchKernelGGL(kernel, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, stream(), j, n, w, v, z, p.cls.p,
+                         p.start_ci.p, p.start_v<T>(), p.piv<T>(), parts, ws.current(), in, out, L);
+    };
+    if (p.start_w == 4) go(k_gm_arnoldi_sor<T, 4>);
+    else if (p.start_w == 6) go(k_gm_arnoldi_sor<T, 6>);
+    else go(k_gm_arnoldi_sor<T, 8>);
+  };
   int64_t enq = 0;
   while (true) {
     // the residual's read left no reduction pending, and the cycle's kernels
@@ -428,11 +654,22 @@ SolveOut gmres(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int64_
     hipLaunchKernelGGL((k_gm_restart<T>), dim3(eb), dim3(kBlock), 0, stream(), n, r, beta, V, s, L);
     int steps = (int)std::min<int64_t>(m, max_it - enq);
     for (int j = 0; j < steps; ++j) {
-      T *vj = V + (size_t)j * ld, *w = V + (size_t)(j + 1) * ld;
-      M->apply(vj, z, s, true);
-      csr_apply<T>(A, EPI_Y, z, nullptr, nullptr, 0.0, w, s, true, OP_NONE, nullptr, ws);
-      const int parts = gram(j, w, s);
+      T *vj = V + (size_t)j * ld, *w = sor ? wt : V + (size_t)(j + 1) * ld;
+      if (!sor || j == 0) M->apply(vj, z, s, true);
+      int parts;
+      if (by_row) {
+        parts = gram_row(j, z, w, s);
+      } else {
+        csr_apply<T>(A, EPI_Y, z, nullptr, nullptr, 0.0, w, s, true, OP_NONE, nullptr, ws);
+        parts = gram(j, w, s);
+      }
       Scal *next = twin_scal(s);
+      if (sor && j + 1 < steps) {
+        arnoldi_sor(*sor, j, w, vj + ld, parts, s, next);
+        s = next;
+        sor->rest(vj + ld, z, s, true);
+        continue;
+      }
       hipLaunchKernelGGL((k_gm_arnoldi<T>), dim3(eb), dim3(kBlock), 0, stream(), j, n, w, parts, ws.current(), s, next,
                          L);
       s = next;

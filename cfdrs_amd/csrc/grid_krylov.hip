@@ -29,20 +29,11 @@ constexpr int kGridThreads = 1024;
 constexpr int kGridWaves = kGridThreads / 64;
 constexpr int kGridBlocks = 128;
 constexpr int kGridHalo = 1024;   // largest |offset|: 2 halo entries per thread
-constexpr int kGridNs = 7;        // entries per row
 constexpr int kGridSums = 3;      // sums per exchange
 constexpr int kGridSpin = 1 << 17;  // polls (about 0.7 us each) before a block gives up
 constexpr int kGridSet = kGridSums * kGridBlocks;
 constexpr unsigned long long kEmpty = 0x7ff8dead0000beefull;  // a NaN that no sum is stored as
 constexpr int kScalWords = (int)(sizeof(Scal) / sizeof(int));
-
-// The matrix rows: entry j of row i is at column i + off[j], its value at
-// dv[k[j] n + i], or with lower[j] (the mirrored half of symmetric storage)
-// at dv[k[j] n + i + off[j]]; in column order.
-struct GridMat {
-  int n = 0, halo = 0;
-  int off[kGridNs] = {}, k[kGridNs] = {}, lower[kGridNs] = {};
-};
 
 struct GridShared {
   Scal sc;
@@ -131,10 +122,10 @@ template <typename T, int NS, int RPT>
 struct GridRows {
   static constexpr int rows = kGridThreads * RPT;
   T a[RPT][NS];
-  const GridMat &g;
+  const DiaRows &g;
   const int r0;
 
-  __device__ GridRows(const GridMat &g_, const T *__restrict__ dv) : g(g_), r0(blockIdx.x * rows) {
+  __device__ GridRows(const DiaRows &g_, const T *__restrict__ dv) : g(g_), r0(blockIdx.x * rows) {
 #pragma unroll
     for (int u = 0; u < RPT; ++u) {
       const int row = r0 + u * kGridThreads + (int)threadIdx.x;
@@ -202,7 +193,7 @@ __global__ __launch_bounds__(256) void k_grid_commit(int n, const T *__restrict_
 // x, r, p and the scalars, with p the next direction; the new x and scalars go
 // to xn and sn.  edge: 2 n values.
 template <typename T, int NS, int RPT>
-__global__ __launch_bounds__(kGridThreads) void k_grid_cg(GridMat g, const T *__restrict__ dv,
+__global__ __launch_bounds__(kGridThreads) void k_grid_cg(DiaRows g, const T *__restrict__ dv,
                                                           const T *__restrict__ jd, const T *__restrict__ x,
                                                           T *xn, T *r, T *p, T *edge, Scal *s, Scal *sn,
                                                           unsigned long long *slots, int steps) {
@@ -293,7 +284,7 @@ __global__ __launch_bounds__(kGridThreads) void k_grid_cg(GridMat g, const T *__
 // (beta of the first iteration formed), the new x and scalars into xn and sn;
 // leaves jd .* p in ph.  edge: 3 n values.
 template <typename T, int NS, int RPT>
-__global__ __launch_bounds__(kGridThreads) void k_grid_bicg(GridMat g, const T *__restrict__ dv,
+__global__ __launch_bounds__(kGridThreads) void k_grid_bicg(DiaRows g, const T *__restrict__ dv,
                                                             const T *__restrict__ jd, const T *__restrict__ x,
                                                             T *xn, T *r, const T *__restrict__ rhat, T *p, T *v,
                                                             T *ph, T *edge, Scal *s, Scal *sn,
@@ -429,27 +420,6 @@ __global__ __launch_bounds__(kGridThreads) void k_grid_bicg(GridMat g, const T *
   store_scal(sh, sn);
 }
 
-GridMat grid_mat(const DevCsr &A) {
-  GridMat g;
-  const DiaDesc &d = A.dia_desc;
-  g.n = A.n;
-  int m = 0;
-  if (d.sym)
-    for (int k = d.nd - 1; k > 0; --k, ++m) {
-      g.off[m] = -d.off[k];
-      g.k[m] = k;
-      g.lower[m] = 1;
-    }
-  for (int k = 0; k < d.nd; ++k, ++m) {
-    g.off[m] = d.off[k];
-    g.k[m] = k;
-  }
-  for (int j = 0; j < m; ++j) g.halo = std::max(g.halo, std::abs(g.off[j]));
-  return g;
-}
-
-int entries(const DiaDesc &d) { return d.sym ? 2 * d.nd - 1 : d.nd; }
-
 // Rows per thread: an exchange costs more with every block that takes part,
 // the phases between cost more with every row.  CG on 16,384 / 36,864 / 65,536
 // / 131,044 rows, us per iteration with 1, 2 and 4 rows: 4.1, 4.3, 4.3 / 5.4,
@@ -472,10 +442,34 @@ void commit(int n, const T *xn, T *x, const Scal *sn, Scal *s) {
 }  // namespace
 
 template <typename T>
+DiaRows dia_rows(const DevCsr &A) {
+  DiaRows g;
+  const DiaDesc &d = A.dia_desc;
+  if (!A.dia || A.dia_vals<T>() == nullptr || A.n != A.m || (d.sym ? 2 * d.nd - 1 : d.nd) > kDiaRowMax) return g;
+  g.n = A.n;
+  int m = 0;
+  if (d.sym)
+    for (int k = d.nd - 1; k > 0; --k, ++m) {
+      g.off[m] = -d.off[k];
+      g.k[m] = k;
+      g.lower[m] = 1;
+    }
+  for (int k = 0; k < d.nd; ++k, ++m) {
+    g.off[m] = d.off[k];
+    g.k[m] = k;
+  }
+  g.count = m;
+  for (int j = 0; j < m; ++j) g.halo = std::max(g.halo, std::abs(g.off[j]));
+  return g;
+}
+template DiaRows dia_rows<double>(const DevCsr &);
+template DiaRows dia_rows<float>(const DevCsr &);
+
+template <typename T>
 bool grid_krylov_takes(const DevCsr &A, bool bicg) {
-  if (!A.dia || A.dia_vals<T>() == nullptr || A.n < 1 || A.n != A.m) return false;
-  const int ns = entries(A.dia_desc);
-  if (ns < 1 || ns > kGridNs || grid_mat(A).halo > kGridHalo) return false;
+  const DiaRows g = dia_rows<T>(A);
+  const int ns = g.count;
+  if (ns < 1 || A.n < 1 || g.halo > kGridHalo) return false;
   // one block per CU, and no more than half of the CUs
   const int rows = kGridThreads * rows_per_thread(A.n, ns, bicg);
   return (A.n + rows - 1) / rows <= std::min(kGridBlocks, num_cus() / 2);
@@ -488,8 +482,8 @@ void grid_cg(const DevCsr &A, const T *jd, T *x, T *r, T *p, T *edge, Scal *s, i
   c.grid_slots.ensure(4 * kGridSet + (sizeof(Scal) + 7) / 8);
   Scal *sn = reinterpret_cast<Scal *>(c.grid_slots.p + 4 * kGridSet);
   hipLaunchKernelGGL(k_grid_reset, dim3(1), dim3(256), 0, stream(), c.grid_slots.p, s);
-  const GridMat g = grid_mat(A);
-  const int ns = entries(A.dia_desc), rpt = rows_per_thread(A.n, ns, false), rows = kGridThreads * rpt;
+  const DiaRows g = dia_rows<T>(A);
+  const int ns = g.count, rpt = rows_per_thread(A.n, ns, false), rows = kGridThreads * rpt;
   const auto go = [&](auto *kernel) {
     const int lds = (rows + 2 * g.halo) * (int)sizeof(T);
     hipLaunchKernelGGL(kernel, dim3((A.n + rows - 1) / rows), dim3(kGridThreads), lds, stream(), g,
@@ -512,8 +506,8 @@ void grid_bicgstab(const DevCsr &A, const T *jd, T *x, T *r, const T *rhat, T *p
   c.grid_slots.ensure(4 * kGridSet + (sizeof(Scal) + 7) / 8);
   Scal *sn = reinterpret_cast<Scal *>(c.grid_slots.p + 4 * kGridSet);
   hipLaunchKernelGGL(k_grid_reset, dim3(1), dim3(256), 0, stream(), c.grid_slots.p, s);
-  const GridMat g = grid_mat(A);
-  const int ns = entries(A.dia_desc), rpt = rows_per_thread(A.n, ns, true), rows = kGridThreads * rpt;
+  const DiaRows g = dia_rows<T>(A);
+  const int ns = g.count, rpt = rows_per_thread(A.n, ns, true), rows = kGridThreads * rpt;
   const auto go = [&](auto *kernel) {
     const int lds = (rows + 2 * g.halo) * (int)sizeof(T);
     hipLaunchKernelGGL(kernel, dim3((A.n + rows - 1) / rows), dim3(kGridThreads), lds, stream(), g,

@@ -267,6 +267,18 @@ template <> inline const double *DevCsr::rb_vals<double>() const { return layout
 template <> inline const float *DevCsr::rb_vals<float>() const { return layout32 == kRbSorted ? sv32.p : v32.p; }
 
 
+// Diagonal storage row by row, for kernels that do more with a row than its
+// product: entry j of row i is at column i + off[j], its value at dv[k[j] n + i]
+// or, with lower[j] (the mirrored half of symmetric storage), at
+// dv[k[j] n + i + off[j]]; in column order, count of them (0: not diagonal
+// storage, or more than kDiaRowMax); halo: the largest |off|.
+constexpr int kDiaRowMax = 7;
+struct DiaRows {
+  int n = 0, count = 0, halo = 0;
+  int off[kDiaRowMax] = {}, k[kDiaRowMax] = {}, lower[kDiaRowMax] = {};
+};
+template <typename T> DiaRows dia_rows(const DevCsr &A);
+
 // Padded rows pay where a product is latency, not bytes: up to 700,000 slots
 // 2.5-3.1 us against 4.0-4.3 us in row blocks (the coarse levels of a 383x255
 // grid, FP64).  Above, the padding and the 32-bit columns cost more than the

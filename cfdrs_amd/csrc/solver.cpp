@@ -884,18 +884,27 @@ ColoredSorPrecond::ColoredSorPrecond(const HostCsr &a, double omega) {
   sync_stream();
 }
 
-void ColoredSorPrecond::apply(const double *r, double *z, Scal *s, bool chk) {
-  sor_start<double>(n, start_w, cls.p, start_ci.p, start_v64.p, piv64.p, r, z, s, chk);
+template <>
+void ColoredSorPrecond::rest<double>(const double *r, double *z, Scal *s, bool chk) {
   for (int c = start_w > 0 ? 2 : 1; c < ncolours; ++c)
     sor_colour<double>(colour_off[(size_t)c + 1] - colour_off[(size_t)c], perm.p + colour_off[(size_t)c], rp.p, ci.p,
                        v64.p, piv64.p, r, z, s, chk);
 }
-
-void ColoredSorPrecond::apply(const float *r, float *z, Scal *s, bool chk) {
-  sor_start<float>(n, start_w, cls.p, start_ci.p, start_v32.p, piv32.p, r, z, s, chk);
+template <>
+void ColoredSorPrecond::rest<float>(const float *r, float *z, Scal *s, bool chk) {
   for (int c = start_w > 0 ? 2 : 1; c < ncolours; ++c)
     sor_colour<float>(colour_off[(size_t)c + 1] - colour_off[(size_t)c], perm.p + colour_off[(size_t)c], rp.p, ci.p,
                       v32.p, piv32.p, r, z, s, chk);
+}
+
+void ColoredSorPrecond::apply(const double *r, double *z, Scal *s, bool chk) {
+  sor_start<double>(n, start_w, cls.p, start_ci.p, start_v64.p, piv64.p, r, z, s, chk);
+  rest<double>(r, z, s, chk);
+}
+
+void ColoredSorPrecond::apply(const float *r, float *z, Scal *s, bool chk) {
+  sor_start<float>(n, start_w, cls.p, start_ci.p, start_v32.p, piv32.p, r, z, s, chk);
+  rest<float>(r, z, s, chk);
 }
 
 struct IdentityPrecond : Precond {

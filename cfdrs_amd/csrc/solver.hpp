@@ -91,11 +91,22 @@ struct ColoredSorPrecond : Precond {
   DevBuf<float> start_v32;
   DevBuf<double> v64, piv64;         // values; omega / pivot (unit pivot where the diagonal is absent or zero)
   DevBuf<float> v32, piv32;
+  template <typename T> const T *start_v() const;
+  template <typename T> const T *piv() const;
+  // the colours after the start of a sweep
+  template <typename T> void rest(const T *r, T *z, Scal *s, bool check_done);
   ColoredSorPrecond(const HostCsr &a, double omega);
   int kind() const override { return 3; }
   void apply(const double *r, double *z, Scal *s, bool check_done) override;
   void apply(const float *r, float *z, Scal *s, bool check_done) override;
 };
+
+template <> void ColoredSorPrecond::rest<double>(const double *, double *, Scal *, bool);
+template <> void ColoredSorPrecond::rest<float>(const float *, float *, Scal *, bool);
+template <> inline const double *ColoredSorPrecond::start_v<double>() const { return start_v64.p; }
+template <> inline const float *ColoredSorPrecond::start_v<float>() const { return start_v32.p; }
+template <> inline const double *ColoredSorPrecond::piv<double>() const { return piv64.p; }
+template <> inline const float *ColoredSorPrecond::piv<float>() const { return piv32.p; }
 
 // Greedy colouring in breadth-first order on the symmetrized pattern of a:
 // colour per row, colour_off (ncolours + 1) and the rows grouped by colour
