@@ -28,9 +28,9 @@ namespace {
 // b in LDS meanwhile.
 template <typename T, int U>
 __global__ __launch_bounds__(kBlock) void k_cycle_gemv(int n, int ld, const double *__restrict__ c,
-                                                       const T *__restrict__ b, T *__restrict__ x, Scal *s,
-                                                       int check_done) {
-  if (check_done && s->done) return;
+                                                       const T *__restrict__ b, T *__restrict__ x,
+                                                       const int *__restrict__ done) {
+  const int stop = *done;  // (tested at the store, so that no load waits for it)
   __shared__ __align__(16) double bs[128 * U];
   const int lane = threadIdx.x & 63;
   const int row = (int)((blockIdx.x * (unsigned)kBlock + threadIdx.x) >> 6);
@@ -52,7 +52,7 @@ __global__ __launch_bounds__(kBlock) void k_cycle_gemv(int n, int ld, const doub
     if (j + 1 < n) acc += v[u].y * w.y;
   }
   acc = wave_sum(acc);
-  if (lane == 0 && row < n) x[row] = (T)acc;
+  if (lane == 0 && row < n && !stop) x[row] = (T)acc;
 }
 
 // Row i of Y (columns c of ld): PLAIN: sum_j a_ij X_j; ADD: Y + that; RESID:
@@ -226,7 +226,7 @@ void DenseCycle::apply(const T *b, T *x, Scal *s, bool check_done) const {
   s = settled_scal(s);
   const dim3 blocks((unsigned)((n + kBlock / 64 - 1) / (kBlock / 64)));
 #define CFDLA_GEMV(U)                                                                                             \
-  hipLaunchKernelGGL((k_cycle_gemv<T, U>), blocks, dim3(kBlock), 0, stream(), n, ld, c.p, b, x, s, check_done ? 1 : 0)
+  hipLaunchKernelGGL((k_cycle_gemv<T, U>), blocks, dim3(kBlock), 0, stream(), n, ld, c.p, b, x, done_flag(s, check_done))
   if (ld <= 512) CFDLA_GEMV(4);
   else if (ld <= 1024) CFDLA_GEMV(8);
   else if (ld <= 1536) CFDLA_GEMV(12);

@@ -324,6 +324,10 @@ struct Scal {
   int32_t pad;          // 1: a kernel with a bounded wait gave up (grid_krylov.hip)
 };
 
+// The done flag a kernel tests: that of the (settled) scalars, or with no
+// check one that is never set.
+const int *done_flag(const Scal *s, bool check_done);
+
 // Reduction workspace: two sets of block partials used in turn, so a kernel
 // that still sums one reduction's partials can write its own.
 struct RedWs {

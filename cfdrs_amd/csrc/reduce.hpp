@@ -51,6 +51,12 @@ __device__ __forceinline__ float add_across(float v) {
   return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
 }
 
+// v is computed, and loaded, by here.
+template <typename T>
+__device__ __forceinline__ void pin(T &v) {
+  asm volatile("" : "+v"(v));
+}
+
 // Sum of a wavefront, in every lane: the xor tree 32, 16, 8, 4, 2, 1 without
 // LDS traffic.  The lane swaps of gfx950 add the halves (lane ^ 32) and then
 // the rows (lane ^ 16); within a row the partial sums repeat with the period

@@ -63,7 +63,8 @@ void init_device(int dev) {
   d.ready = true;
   d.context = std::make_unique<Context>();
   d.context->ws.init();
-  d.context->scal.alloc(2 * kScalSlots);
+  d.context->scal.alloc(2 * kScalSlots + 1);
+  CFDLA_HIP(hipMemset(d.context->scal.p + 2 * kScalSlots, 0, sizeof(Scal)));  // (done_flag)
   CFDLA_HIP(hipHostMalloc(reinterpret_cast<void **>(&d.context->host), sizeof(Scal), hipHostMallocDefault));
 }
 

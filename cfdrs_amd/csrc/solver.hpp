@@ -13,7 +13,7 @@ namespace cfdla {
 // and pooled solver vectors.
 struct Context {
   RedWs ws;
-  DevBuf<Scal> scal;  // kScalSlots slots and their twins
+  DevBuf<Scal> scal;  // kScalSlots slots and their twins, and one that stays zero (done_flag)
   int twin[kScalSlots] = {};  // 1: slot i's scalars are in its twin
   Pend pend{};
   DevBuf<unsigned long long> grid_slots;  // exchanged sums of grid_krylov.hip
