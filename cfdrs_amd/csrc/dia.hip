@@ -290,16 +290,18 @@ __global__ __launch_bounds__(kBlock) void k_dia_vec(int n, DiaDesc dd, const T *
 }
 
 // Products that follow a reduction within an iteration take it along while it
-// is pending: the CG direction, the first product of a V-cycle, BiCGSTAB's
-// second product.
-template <int EPI>
-constexpr bool consumes() { return EPI == EPI_DIR || EPI == EPI_JACOBI0 || EPI == EPI_DOT2; }
+// is pending: the CG direction, the first product of a V-cycle (the residual
+// where the update has made the first sweeps), BiCGSTAB's second product.
+template <int EPI, bool DOT>
+constexpr bool consumes() {
+  return EPI == EPI_DIR || EPI == EPI_JACOBI0 || EPI == EPI_DOT2 || (EPI == EPI_RESID && !DOT);
+}
 
 template <typename T, int EPI, bool DOT, bool SYM, int ND>
 void launch_shape(const DevCsr &A, int blocks, const T *x, const T *b, const T *dinv, double omega, T *y,
                   const T *dotw, Scal *s, bool check_done, RedWs &ws, T *y2) {
   double *part = DOT ? nullptr : ws.partials.p;
-  if constexpr (consumes<EPI>()) {
+  if constexpr (consumes<EPI, DOT>()) {
     if (pending_on(s) && blocks <= kConsumeBlocks) {
       const Pend pd = take_pending(s);
       if (DOT) part = ws.next();
@@ -318,7 +320,7 @@ template <typename T, int EPI, bool DOT, int ND, int R>
 void launch_vec(const DevCsr &A, const T *x, const T *b, const T *dinv, double omega, T *y, const T *dotw,
                 Scal *s, bool check_done, RedWs &ws, int blocks, T *y2) {
   double *part = DOT ? nullptr : ws.partials.p;
-  if constexpr (consumes<EPI>()) {
+  if constexpr (consumes<EPI, DOT>()) {
     if (pending_on(s) && blocks <= kConsumeBlocks) {
       const Pend pd = take_pending(s);
       if (DOT) part = ws.next();
@@ -332,6 +334,68 @@ void launch_vec(const DevCsr &A, const T *x, const T *b, const T *dinv, double o
   if (DOT) part = ws.next();
   hipLaunchKernelGGL((k_dia_vec<T, EPI, DOT, ND, R, false>), dim3(blocks), dim3(kBlock), 0, stream(), A.n, A.dia_desc,
                      A.dia_vals<T>(), x, b, dinv, (T)omega, y, dotw, s, check_done ? 1 : 0, part, y2, Pend{});
+}
+
+// The PCG update and the first two Jacobi sweeps of the V-cycle that follows it
+// on symmetric diagonal storage, in one pass: x += alpha p, rn = r - alpha q
+// with its norm, and the sweeps of rn from zero (EPI_JACOBI0), whose neighbours'
+// entries of rn are formed at the gathers as the own one is.  rn is not r:
+// other blocks still read that.  Bound by latency: a launch saved per iteration
+// is the gain, three gathers per entry instead of two the cost.  On 97,665 rows
+// 5.5 us, and 4.2 for the residual product that now finishes the norm, against
+// 4.5, 4.3 and 3.2; FP64 AMG-PCG solves of five-point systems, 64x64 / 100x90 /
+// 200x151 / 383x255 / 512x512: 0.53 / 0.605 / 0.78 / 0.945 / 1.38 ms with two
+// launches, 0.50 / 0.57 / 0.735 / 0.905 / 1.33 ms.
+template <typename T, int ND>
+__global__ __launch_bounds__(kBlock) void k_cg_start(int n, DiaDesc dd, const T *__restrict__ dv,
+                                                     const T *__restrict__ r, const T *__restrict__ q,
+                                                     const T *__restrict__ dinv, T omega, const T *__restrict__ p,
+                                                     T *__restrict__ x, T *__restrict__ rn, T *__restrict__ y,
+                                                     double *partials, Pend pd) {
+  constexpr int NS = 2 * ND - 1;
+  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+  const int chunk = ((n + kBlock - 1) / kBlock + 7) >> 3;
+  const int mine = (xcd * chunk + local) * kBlock + (int)threadIdx.x;
+  const bool live = local < chunk && mine < n;
+  const int row = live ? mine : n - 1;
+  int c[NS];
+  bool ok[NS];
+  T v[NS], rv[NS], qv[NS], jv[NS];
+#pragma unroll
+  for (int j = 0; j < NS; ++j) {
+    const bool lower = j < ND - 1;
+    const int k = lower ? ND - 1 - j : j - (ND - 1);
+    const int col = lower ? row - dd.off[k] : row + dd.off[k];
+    ok[j] = col >= 0 && col < n;
+    c[j] = ok[j] ? col : row;
+    v[j] = dv[k * n + (lower && ok[j] ? col : row)];
+  }
+#pragma unroll
+  for (int j = 0; j < NS; ++j) {
+    rv[j] = r[c[j]];
+    qv[j] = q[c[j]];
+    jv[j] = dinv[c[j]];
+  }
+  const T r0 = r[row], q0 = q[row], d0 = dinv[row], p0 = p[row], x0 = x[row];
+  __shared__ Scal sc;
+  consume(pd, sc);
+  if (sc.done) return;
+  const T alpha = (T)sc.alpha;
+  const T ri = r0 - alpha * q0;
+  T sum = T(0);
+#pragma unroll
+  for (int j = 0; j < NS; ++j) {
+    const T rj = rv[j] - alpha * qv[j];
+    sum += (ok[j] && v[j] != T(0)) ? v[j] * (omega * jv[j] * rj) : T(0);
+  }
+  double acc[1] = {0.0};
+  if (live) {
+    x[row] = x0 + alpha * p0;
+    rn[row] = ri;
+    y[row] = omega * d0 * ri + omega * d0 * (ri - sum);
+    acc[0] = (double)ri * (double)ri;
+  }
+  block_partials<1>(acc, partials);
 }
 
 bool aligned(const void *p, size_t bytes) { return (reinterpret_cast<uintptr_t>(p) & (bytes - 1)) == 0; }
@@ -410,6 +474,37 @@ void launch_dia(const DevCsr &A, const T *x, const T *b, const T *dinv, double o
 #undef CFDLA_DIA
   if (DOT) finish(EPI == EPI_DOT2 ? 2 : 1, s, op, blocks, ws, check_done);
 }
+
+// At most five entries per row: with seven the gathers eat the launch saved
+// (32^3 and 64^3 rows 0.80 and 1.565 ms, fused 0.81 and 1.58).  Its norm stays
+// pending for the residual product, hence the limit of kConsumeBlocks.
+template <typename T>
+bool cg_start_takes(const DevCsr &A) {
+  return A.dia && A.dia_vals<T>() != nullptr && dia_supported(A.dia_desc) && A.dia_desc.sym && A.dia_desc.nd <= 3 &&
+         xcd_grid((A.n + kBlock - 1) / kBlock, 1, kMaxBlocks) <= kConsumeBlocks;
+}
+
+template <typename T>
+void cg_start(const DevCsr &A, const T *r, const T *q, const T *dinv, double omega, const T *p, T *x, T *rn, T *y,
+              Scal *s, RedWs &ws) {
+  const int blocks = xcd_grid((A.n + kBlock - 1) / kBlock, 1, kMaxBlocks);
+  const Pend pd = take_pending(s);
+  double *part = ws.next();
+#define CFDLA_START(ND)                                                                                        \
+  hipLaunchKernelGGL((k_cg_start<T, ND>), dim3(blocks), dim3(kBlock), 0, stream(), A.n, A.dia_desc,             \
+                     A.dia_vals<T>(), r, q, dinv, (T)omega, p, x, rn, y, part, pd)
+  if (A.dia_desc.nd == 2) CFDLA_START(2);
+  else CFDLA_START(3);
+#undef CFDLA_START
+  CFDLA_HIP(hipGetLastError());
+  finish(1, s, OP_CG_RR, blocks, ws, true);
+}
+template bool cg_start_takes<double>(const DevCsr &);
+template bool cg_start_takes<float>(const DevCsr &);
+template void cg_start<double>(const DevCsr &, const double *, const double *, const double *, double, const double *,
+                               double *, double *, double *, Scal *, RedWs &);
+template void cg_start<float>(const DevCsr &, const float *, const float *, const float *, double, const float *,
+                              float *, float *, float *, Scal *, RedWs &);
 
 #define CFDLA_DIA_INST(T, E)                                                                                   \
   template void launch_dia<T, E, false>(const DevCsr &, const T *, const T *, const T *, double, T *, const T *, \

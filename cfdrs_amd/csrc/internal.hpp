@@ -393,6 +393,12 @@ enum Epi : int { EPI_Y = 0, EPI_RESID = 1, EPI_JACOBI = 2, EPI_ADD = 3, EPI_JACO
 // Diagonal-format product with epilogue (dia.hip); A.dia must hold and the
 // stored diagonal count must be one of the instantiated shapes (dia_supported).
 bool dia_supported(const DiaDesc &d);
+// The PCG update together with the first two Jacobi sweeps on the new residual
+// rn (dia.hip), up to kConsumeBlocks blocks of rows.
+template <typename T> bool cg_start_takes(const DevCsr &A);
+template <typename T>
+void cg_start(const DevCsr &A, const T *r, const T *q, const T *dinv, double omega, const T *p, T *x, T *rn, T *y,
+              Scal *s, RedWs &ws);
 template <typename T, int EPI, bool DOT>
 void launch_dia(const DevCsr &A, const T *x, const T *b, const T *dinv, double omega, T *y, const T *dotw,
                 Scal *s, bool check_done, int op, RedWs &ws, T *y2 = nullptr);

@@ -1322,7 +1322,7 @@ void AmgPrecond::vcycle(int l, const T *b, T *x, Scal *s, bool chk, int dot_op, 
   // 26.2 + ~3 us unfused on the first coarse level of the 128^3 problem).
   if (down >= 2 && L.A.nnz <= 8 * (int64_t)n) {
     // the zero-guess sweep and the next one in a single pass
-    csr_apply<T>(L.A, EPI_JACOBI0, b, b, dinv, w, buf[cur ^ 1], s, chk, OP_NONE, nullptr, ws);
+    if (!first_ready) csr_apply<T>(L.A, EPI_JACOBI0, b, b, dinv, w, buf[cur ^ 1], s, chk, OP_NONE, nullptr, ws);
     cur ^= 1;
     k = 2;
   } else if (down >= 1) {
@@ -1360,6 +1360,16 @@ void AmgPrecond::vcycle(int l, const T *b, T *x, Scal *s, bool chk, int dot_op, 
   }
   if (cur != 0) copy_vec<T>(n, buf[cur], x, s, chk);
   if (dot_op != OP_NONE) dot2<T>(n, b, x, nullptr, nullptr, s, chk, dot_op, ws);
+}
+
+template <typename T>
+T *AmgPrecond::pair_target(int n, T *z) {
+  ensure_device();
+  if (cfg.smoother != 2 || lv.size() < 2 || dense.level == 0 || fused.level == 0) return nullptr;
+  DevLevel &L = lv[0];
+  const int down = cfg.pre_smooth_iterations;
+  if (L.A.n != n || down < 2 || L.A.nnz > 8 * (int64_t)n || !cg_start_takes<T>(L.A)) return nullptr;
+  return (down - 1 + cfg.post_smooth_iterations) % 2 == 0 ? L.t<T>() : z;
 }
 
 template void AmgPrecond::vcycle<double>(int, const double *, double *, Scal *, bool, int, bool);
@@ -1441,6 +1451,10 @@ SolveOut pcg(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int64_t 
   ConvergenceGate gate;
   bool finished = false, behind = false;  // behind: a chunk is enqueued whose end has not been polled
   bool resident = (jd || M->kind() == 0) && grid_krylov_takes<T>(A, false);
+  // an AMG cycle whose first two sweeps the update makes
+  auto *amg = M->kind() == 2 ? static_cast<AmgPrecond *>(M) : nullptr;
+  T *started = amg ? amg->pair_target<T>(n, z) : nullptr;
+  T *rn = started ? vec<T>(6, n) : nullptr;
   while (!finished) {
     const Scal *h = nullptr;
     if (resident && enq < max_it) {
@@ -1468,6 +1482,11 @@ SolveOut pcg(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int64_t 
         if (k == 0 && behind) poll.advanced();
         if (jd) {
           cg_update<T>(n, p, q, x, r, jd, z, s, ws);
+        } else if (started) {
+          const DevCsr &A0 = amg->lv[0].A;
+          cg_start<T>(A0, r, q, A0.sdinv<T>(), amg->cfg.relaxation_factor, p, x, rn, started, s, ws);
+          std::swap(r, rn);
+          amg->apply_dot_started<T>(r, z, s, true, OP_CG_BETA);
         } else {
           cg_update<T>(n, p, q, x, r, nullptr, nullptr, s, ws);
           M->apply_dot(n, r, z, s, true, OP_CG_BETA);

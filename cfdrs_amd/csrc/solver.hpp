@@ -298,6 +298,14 @@ struct AmgPrecond : Precond {
     ensure_device();
     vcycle<float>(0, r, z, s, check_done, dot_op);
   }
+  // Where level 0's first two sweeps leave their iterate, for a caller that
+  // makes them itself (cg_start) and goes on with apply_dot_started; null
+  // where the cycle does not start with the two in one pass.
+  template <typename T> T *pair_target(int n, T *z);
+  template <typename T>
+  void apply_dot_started(const T *r, T *z, Scal *s, bool check_done, int dot_op) {
+    vcycle<T>(0, r, z, s, check_done, dot_op, true);
+  }
   // first_ready: the caller's restriction already wrote the level's first
   // Jacobi iterate from zero into first_sweep_target(l).
   template <typename T> void vcycle(int l, const T *b, T *x, Scal *s, bool check_done, int dot_op,
