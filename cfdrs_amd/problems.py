@@ -1,7 +1,7 @@
 """Deterministic problem generators for the five workloads.
 
 All random inputs come from SplitMix64 streams in libcfdla
-(``cfdla_synth_uniform``), so the host, the GPU box and the tests see the
+(``cfdla_synth_uniform``), so the host, the GPU and the tests see the
 same matrices and right-hand sides.  Matrix assembly runs in the library:
 
 * ``pressure_correction_2d``: cell-centred 5-point pressure-correction

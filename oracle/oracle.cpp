@@ -1,6 +1,6 @@
 // CPU FP64 oracle for the CFDrs sparse linear-solve path.
 //
-// TEST INFRASTRUCTURE ONLY. This file is the checker: it restates, in plain
+// TEST INFRASTRUCTURE ONLY. This file is the oracle: it restates, in plain
 // sequential C++, the reference's algorithms for CSR assembly, AMG setup and
 // V-cycle, the smoothers, the Krylov recurrences and the 1D network solve
 // cascade.  Only tests/, __graft_entry__.smoke() and the cpu_baseline leg of

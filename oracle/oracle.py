@@ -1,6 +1,6 @@
 """ctypes wrapper of the CPU FP64 oracle (oracle/liboracle.so).
 
-TEST INFRASTRUCTURE ONLY: this module is the checker.  It may be imported by
+TEST INFRASTRUCTURE ONLY: this module is the oracle.  It may be imported by
 tests/, by __graft_entry__.smoke() and by the cpu_baseline leg of bench.py,
 and by nothing else.  The product package (cfdrs_amd) never imports it.
 """
