@@ -27,10 +27,22 @@ namespace {
 // EPI_DIR on a stopped solve: the product is skipped, but the new-direction
 // buffer still receives the current direction, so the caller's buffer swap
 // keeps pointing at the latest one when the iteration resumes (after a
-// residual replacement).
+// residual replacement).  Every block copies its strips, also one that has no
+// tile of the product.
 template <typename T>
 __device__ __forceinline__ void keep_direction(int n, const T *__restrict__ p, T *__restrict__ pn) {
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) pn[i] = p[i];
+}
+
+// A block of a consuming product (CONS below) that the dealing of the tiles
+// left without one: the tile loop, where the others learn that the solve has
+// stopped, does not run there.
+template <typename T>
+__device__ __forceinline__ void idle_direction(int n, const T *__restrict__ p, T *__restrict__ pn, const Pend &pd,
+                                               int check_done) {
+  __shared__ Scal sc;
+  consume(pd, sc);
+  if (check_done && sc.done) keep_direction(n, p, pn);
 }
 
 // CONS: the reduction before this product is still pending (finalize.hpp).
@@ -55,6 +67,9 @@ __global__ __launch_bounds__(kBlock) void k_dia(int n, DiaDesc dd, const T *__re
   const int chunk = (tiles + 7) >> 3;
   const int t1 = min(tiles, xcd * chunk + chunk);
   double dacc[EPI == EPI_DOT2 ? 2 : 1] = {};
+  if constexpr (CONS && EPI == EPI_DIR) {
+    if (xcd * chunk + local >= t1) idle_direction(n, x, y2, pd, check_done);
+  }
   for (int t = xcd * chunk + local; t < t1; t += per) {
     const int mine = t * kBlock + (int)threadIdx.x;
     const bool live = mine < n;
@@ -157,6 +172,9 @@ __global__ __launch_bounds__(kBlock) void k_dia_vec(int n, DiaDesc dd, const T *
   const int chunk = (tiles + 7) >> 3;
   const int t1 = min(tiles, xcd * chunk + chunk);
   double dacc[EPI == EPI_DOT2 ? 2 : 1] = {};
+  if constexpr (CONS && EPI == EPI_DIR) {
+    if (xcd * chunk + local >= t1) idle_direction(n, x, y2, pd, check_done);
+  }
   for (int t = xcd * chunk + local; t < t1; t += per) {
     const int g = t * kBlock + (int)threadIdx.x;
     const bool live = g < groups;
