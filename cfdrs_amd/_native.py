@@ -105,6 +105,7 @@ SIGNATURES = {
     "cfdla_amg_set_gather": (C.c_int, [_VP, C.c_int32]),
     "cfdla_amg_update_values_device": (C.c_int, [_VP, _VP]),
     "cfdla_amg_stats": (C.c_int, [_VP, C.POINTER(AmgStatistics)]),
+    "cfdla_amg_dense_level": (C.c_int, [_VP, _I32P]),
     "cfdla_amg_export_level": (C.c_int, [_VP, C.c_int32, C.c_int32, _I64P, _I64P, _I64P, _VP, _VP, _VP]),
     "cfdla_amg_export_map": (C.c_int, [_VP, C.c_int32, _VP]),
     "cfdla_precond_destroy": (C.c_int, [_VP]),

@@ -604,7 +604,8 @@ cfdla_status cfdla_amg_stats(cfdla_precond p, cfdla_amg_statistics *out) {
     amg->sync_host();
     const auto &lv = amg->host.levels;
     out->num_levels = (int32_t)lv.size();
-    // (within a dense cycle the level's sweeps and restriction are one product too)
+    // (a dense cycle of the Jacobi levels holds those of the level above the
+    // coarsest one: cfdla_amg_dense_level)
     out->fused_level = !amg->on_device ? -1 : amg->dense.level >= 0 ? (int)lv.size() - 2 : amg->fused.level;
     auto count = [](const HostCsr &a) {
       int64_t c = 0;
@@ -621,6 +622,16 @@ cfdla_status cfdla_amg_stats(cfdla_precond p, cfdla_amg_statistics *out) {
     out->operator_complexity = fine > 0 ? (double)tot / (double)fine : 1.0;
     out->grid_complexity = lv[0].A.n > 0 ? (double)vars / (double)lv[0].A.n : 1.0;
     out->setup_time = amg->setup_time;
+  });
+}
+
+cfdla_status cfdla_amg_dense_level(cfdla_precond p, int32_t *level) {
+  return guarded([&] {
+    require_ptr(p, "preconditioner");
+    require_ptr(level, "level");
+    auto *amg = dynamic_cast<AmgPrecond *>(p->p.get());
+    CFDLA_REQUIRE(amg != nullptr, CFDLA_ERR_INVALID_ARG, "preconditioner is not AMG");
+    *level = amg->dense_level();
   });
 }
 

@@ -259,6 +259,12 @@ struct AmgPrecond : Precond {
   FusedOp fused;
   GsTail tail;  // the small levels of a Gauss-Seidel hierarchy
   DenseCycle dense;  // the last levels of a Jacobi hierarchy
+  // first level within a dense operator, of either smoother (-1: none)
+  int dense_level() const {
+    if (!on_device) return -1;
+    if (dense.level >= 0) return dense.level;
+    return tail.level >= 0 && tail.dense.level >= 0 ? tail.level + tail.dense.level : -1;
+  }
   void form_dense();
   bool build_fused(size_t l);
   void refresh_fused_device();

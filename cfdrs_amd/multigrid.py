@@ -125,9 +125,14 @@ class AMGStatistics:
     operator_complexity: float = 1.0
     grid_complexity: float = 1.0
     setup_time: float = 0.0
-    # the level whose pre-sweeps and restriction run as one product (-1:
-    # none, or the hierarchy is not on the device yet)
+    # the level above the coarsest one when its Jacobi pre-sweeps and
+    # restriction are one product: F = [2wD - w^2 DAD; R (I - wAD)^2], or part
+    # of the dense operator where dense_level is not -1 (-1: three products, or
+    # the hierarchy is not on the device yet)
     fused_level: int = -1
+    # the first of the last levels that run as one dense operator (-1: none, or
+    # not on the device yet)
+    dense_level: int = -1
 
 
 class _Preconditioner:
@@ -247,10 +252,12 @@ class AlgebraicMultigrid(_Preconditioner):
     @property
     def statistics(self) -> AMGStatistics:
         s = N.AmgStatistics()
+        dense = C.c_int32()
         N.call("cfdla_amg_stats", self.handle, C.byref(s))
+        N.call("cfdla_amg_dense_level", self.handle, C.byref(dense))
         L = s.num_levels
         return AMGStatistics(L, list(s.level_rows[:L]), list(s.level_nnz[:L]), s.operator_complexity,
-                             s.grid_complexity, s.setup_time, s.fused_level)
+                             s.grid_complexity, s.setup_time, s.fused_level, dense.value)
 
     def level(self, level: int, which: str = "A"):
         """(row_ptr, col_indices, values, nrows, ncols) of A_l, R_l or P_l."""

@@ -144,7 +144,9 @@ typedef struct {
    * when the smoother is Jacobi with two pre-sweeps and the coarsest level
    * is solved directly, that level runs them as one product with
    * F = [2wD - w^2 DAD; R (I - wAD)^2] (D the smoother's inverse diagonal),
-   * the same operator in exact arithmetic.  No reference counterpart. */
+   * or, where the last levels are small, everything from the first small one
+   * on is one dense operator (cfdla_amg_dense_level): the same operators in
+   * exact arithmetic.  No reference counterpart. */
   int32_t separate_coarse_restriction;
 } cfdla_amg_config;
 
@@ -153,8 +155,11 @@ typedef struct {
 /* AMGStatistics (multigrid/mod.rs:366-395). */
 typedef struct {
   int32_t num_levels;
-  /* the level whose pre-sweeps and restriction run as one product (see
-   * separate_coarse_restriction); -1 none or not yet on the device */
+  /* the level above the coarsest one of a Jacobi hierarchy when its
+   * pre-sweeps and restriction are one product: with F (see
+   * separate_coarse_restriction), or inside the dense operator when
+   * cfdla_amg_dense_level reports a level; -1 three products, or not yet on
+   * the device */
   int32_t fused_level;
   int64_t level_rows[CFDLA_MAX_LEVELS];
   int64_t level_nnz[CFDLA_MAX_LEVELS];
@@ -317,6 +322,11 @@ cfdla_status cfdla_amg_set_gather(cfdla_precond p, int32_t layout);
  * refresh (crates/cfd-2d/src/pressure_velocity/correction.rs:56-89). */
 cfdla_status cfdla_amg_update_values_device(cfdla_precond p, cfdla_matrix m);
 cfdla_status cfdla_amg_stats(cfdla_precond p, cfdla_amg_statistics *out);
+/* The first of the last levels that run as one dense operator x = C b, formed
+ * from the level values on the device whenever they change (Jacobi and
+ * Gauss-Seidel hierarchies); -1 none or not yet on the device.  No level from
+ * it on runs sweeps of its own.  No reference counterpart. */
+cfdla_status cfdla_amg_dense_level(cfdla_precond p, int32_t *level);
 /* Hierarchy export for structure checks.  which: 0 = A_l, 1 = R_l, 2 = P_l.
  * First call with arrays NULL to get sizes. */
 cfdla_status cfdla_amg_export_level(cfdla_precond p, int32_t level, int32_t which, int64_t *nrows,
