@@ -91,6 +91,7 @@ SIGNATURES = {
     "cfdla_matrix_storage": (C.c_int, [_VP, _I32P, _I64P, _I64P]),
     "cfdla_matrix_set_storage": (C.c_int, [_VP, C.c_int32]),
     "cfdla_matrix_set_gather": (C.c_int, [_VP, C.c_int32]),
+    "cfdla_matrix_set_resident_polls": (C.c_int, [_VP, C.c_int32]),
     "cfdla_matrix_gather": (C.c_int, [_VP, _I32P, _I32P]),
     "cfdla_matrix_destroy": (C.c_int, [_VP]),
     "cfdla_spmv": (C.c_int, [_VP, _VP, _VP]),

@@ -427,6 +427,15 @@ cfdla_status cfdla_matrix_set_gather(cfdla_matrix m, int32_t layout) {
   });
 }
 
+cfdla_status cfdla_matrix_set_resident_polls(cfdla_matrix m, int32_t polls) {
+  return guarded([&] {
+    require_ptr(m, "matrix");
+    CFDLA_REQUIRE(polls >= CFDLA_RESIDENT_POLLS_DEFAULT && polls <= kResidentPollsMax, CFDLA_ERR_INVALID_ARG,
+                  "polls must be between -1 and 2^20");
+    m->dev.resident_polls = polls == CFDLA_RESIDENT_POLLS_DEFAULT ? kResidentPolls : polls;
+  });
+}
+
 cfdla_status cfdla_matrix_gather(cfdla_matrix m, int32_t *layout_fp64, int32_t *layout_fp32) {
   return guarded([&] {
     require_ptr(m, "matrix");

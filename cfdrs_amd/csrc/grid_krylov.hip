@@ -14,10 +14,11 @@
 // 12.1.  Bound by the two (CG) or three exchanges of an iteration.  Larger
 // systems would need every CU or rows that no longer fit the registers.
 //
-// Every wait is bounded: a block that does not see the others' sums in time
-// reports it in Scal::pad.  The new iterate and scalars replace the old ones in
-// a launch of their own (k_grid_commit), if no block did: a solve whose blocks
-// did not meet goes on with a launch per phase from where it was.
+// Every wait is bounded: a block that does not see the others' sums within
+// DevCsr::resident_polls polls reports it in Scal::pad.  The new iterate and
+// scalars replace the old ones in a launch of their own (k_grid_commit), if no
+// block did: a solve whose blocks did not meet goes on with a launch per phase
+// from where it was.
 #include "finalize.hpp"
 #include "internal.hpp"
 #include "solver.hpp"
@@ -30,7 +31,6 @@ constexpr int kGridWaves = kGridThreads / 64;
 constexpr int kGridBlocks = 128;
 constexpr int kGridHalo = 1024;   // largest |offset|: 2 halo entries per thread
 constexpr int kGridSums = 3;      // sums per exchange
-constexpr int kGridSpin = 1 << 17;  // polls (about 0.7 us each) before a block gives up
 constexpr int kGridSet = kGridSums * kGridBlocks;
 constexpr unsigned long long kEmpty = 0x7ff8dead0000beefull;  // a NaN that no sum is stored as
 constexpr int kScalWords = (int)(sizeof(Scal) / sizeof(int));
@@ -62,7 +62,7 @@ __device__ __forceinline__ T fetch(const T *p) {
 // 16 / 32 / 64 / 128 blocks: 1.2 / 1.8 / 2.2 / 3.0 us, two trips to the memory
 // side of the eight L2s and the polls that queue there.
 template <int NV, bool EDGES, typename Fin>
-__device__ __forceinline__ bool exchange(GridShared &sh, unsigned long long *slots, int &phase,
+__device__ __forceinline__ bool exchange(GridShared &sh, unsigned long long *slots, int &phase, int polls,
                                          const double (&v)[NV], Fin &&fin) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nb = gridDim.x;
 #pragma unroll
@@ -89,7 +89,7 @@ __device__ __forceinline__ bool exchange(GridShared &sh, unsigned long long *slo
         for (int i = 0; i < kGridSums; ++i) publish(old + i * kGridBlocks + blockIdx.x, kEmpty);
       }
       unsigned long long got[NV][2];
-      int left = kGridSpin;
+      int left = polls;
       do {
         ok = true;
 #pragma unroll
@@ -196,7 +196,7 @@ template <typename T, int NS, int RPT>
 __global__ __launch_bounds__(kGridThreads) void k_grid_cg(DiaRows g, const T *__restrict__ dv,
                                                           const T *__restrict__ jd, const T *__restrict__ x,
                                                           T *xn, T *r, T *p, T *edge, Scal *s, Scal *sn,
-                                                          unsigned long long *slots, int steps) {
+                                                          unsigned long long *slots, int steps, int polls) {
   extern __shared__ char grid_lds[];
   __shared__ GridShared sh;
   GridRows<T, NS, RPT> A(g, dv);
@@ -231,7 +231,7 @@ __global__ __launch_bounds__(kGridThreads) void k_grid_cg(DiaRows g, const T *__
       A.publish_edge(out, u, q[u]);
       pq[0] += (double)pl[A.slot(u)] * (double)q[u];
     }
-    if (!exchange<1, true>(sh, slots, phase, pq, [](Scal &sc, const double(&t)[1]) {
+    if (!exchange<1, true>(sh, slots, phase, polls, pq, [](Scal &sc, const double(&t)[1]) {
           sc.red[0] = t[0];
           finalize(&sc, OP_CG_ALPHA);
         })) {
@@ -251,7 +251,7 @@ __global__ __launch_bounds__(kGridThreads) void k_grid_cg(DiaRows g, const T *__
       rr[0] += (double)rv[u] * (double)rv[u];
       rr[1] += (double)rv[u] * (double)(jv[u] * rv[u]);
     }
-    if (!exchange<2, false>(sh, slots, phase, rr, [](Scal &sc, const double(&t)[2]) {
+    if (!exchange<2, false>(sh, slots, phase, polls, rr, [](Scal &sc, const double(&t)[2]) {
           sc.red[0] = t[0];
           sc.red[1] = t[1];
           finalize(&sc, OP_CG_RR_RZ);
@@ -288,7 +288,7 @@ __global__ __launch_bounds__(kGridThreads) void k_grid_bicg(DiaRows g, const T *
                                                             const T *__restrict__ jd, const T *__restrict__ x,
                                                             T *xn, T *r, const T *__restrict__ rhat, T *p, T *v,
                                                             T *ph, T *edge, Scal *s, Scal *sn,
-                                                            unsigned long long *slots, int steps) {
+                                                            unsigned long long *slots, int steps, int polls) {
   extern __shared__ char grid_lds[];
   __shared__ GridShared sh;
   GridRows<T, NS, RPT> A(g, dv);
@@ -343,7 +343,7 @@ __global__ __launch_bounds__(kGridThreads) void k_grid_bicg(DiaRows g, const T *
       A.publish_edge(vout, u, vv[u]);
       rhv[0] += (double)hv[u] * (double)vv[u];
     }
-    failed = !exchange<1, true>(sh, slots, phase, rhv, [](Scal &sc, const double(&t)[1]) {
+    failed = !exchange<1, true>(sh, slots, phase, polls, rhv, [](Scal &sc, const double(&t)[1]) {
       sc.red[0] = t[0];
       finalize(&sc, OP_BI_ALPHA);
     });
@@ -374,7 +374,7 @@ __global__ __launch_bounds__(kGridThreads) void k_grid_bicg(DiaRows g, const T *
       sums[1] += (double)t[u] * (double)sv[u];
       sums[2] += (double)t[u] * (double)t[u];
     }
-    failed = !exchange<3, true>(sh, slots, phase, sums, [](Scal &sc, const double(&w)[3]) {
+    failed = !exchange<3, true>(sh, slots, phase, polls, sums, [](Scal &sc, const double(&w)[3]) {
       sc.red[0] = w[0];
       finalize(&sc, OP_BI_SNORM);
       if (!sc.done) {
@@ -396,7 +396,7 @@ __global__ __launch_bounds__(kGridThreads) void k_grid_bicg(DiaRows g, const T *
       rr[0] += (double)rv[u] * (double)rv[u];
       rr[1] += (double)hv[u] * (double)rv[u];
     }
-    failed = !exchange<2, false>(sh, slots, phase, rr, [](Scal &sc, const double(&w)[2]) {
+    failed = !exchange<2, false>(sh, slots, phase, polls, rr, [](Scal &sc, const double(&w)[2]) {
       sc.red[0] = w[0];
       sc.red[1] = w[1];
       finalize(&sc, OP_BI_RR_RHO);
@@ -469,7 +469,7 @@ template <typename T>
 bool grid_krylov_takes(const DevCsr &A, bool bicg) {
   const DiaRows g = dia_rows<T>(A);
   const int ns = g.count;
-  if (ns < 1 || A.n < 1 || g.halo > kGridHalo) return false;
+  if (A.resident_polls < 1 || ns < 1 || A.n < 1 || g.halo > kGridHalo) return false;
   // one block per CU, and no more than half of the CUs
   const int rows = kGridThreads * rows_per_thread(A.n, ns, bicg);
   return (A.n + rows - 1) / rows <= std::min(kGridBlocks, num_cus() / 2);
@@ -487,7 +487,8 @@ void grid_cg(const DevCsr &A, const T *jd, T *x, T *r, T *p, T *edge, Scal *s, i
   const auto go = [&](auto *kernel) {
     const int lds = (rows + 2 * g.halo) * (int)sizeof(T);
     hipLaunchKernelGGL(kernel, dim3((A.n + rows - 1) / rows), dim3(kGridThreads), lds, stream(), g,
-                       A.dia_vals<T>(), jd, x, edge + 2 * (size_t)A.n, r, p, edge, s, sn, c.grid_slots.p, steps);
+                       A.dia_vals<T>(), jd, x, edge + 2 * (size_t)A.n, r, p, edge, s, sn, c.grid_slots.p, steps,
+                       A.resident_polls);
   };
 #define CFDLA_GRID(RPT)                     \
   if (ns <= 3) go(k_grid_cg<T, 3, RPT>);    \
@@ -511,7 +512,8 @@ void grid_bicgstab(const DevCsr &A, const T *jd, T *x, T *r, const T *rhat, T *p
   const auto go = [&](auto *kernel) {
     const int lds = (rows + 2 * g.halo) * (int)sizeof(T);
     hipLaunchKernelGGL(kernel, dim3((A.n + rows - 1) / rows), dim3(kGridThreads), lds, stream(), g,
-                       A.dia_vals<T>(), jd, x, edge + 3 * (size_t)A.n, r, rhat, p, v, ph, edge, s, sn, c.grid_slots.p, steps);
+                       A.dia_vals<T>(), jd, x, edge + 3 * (size_t)A.n, r, rhat, p, v, ph, edge, s, sn, c.grid_slots.p, steps,
+                       A.resident_polls);
   };
 #define CFDLA_GRID(RPT)                       \
   if (ns <= 3) go(k_grid_bicg<T, 3, RPT>);    \

@@ -170,6 +170,9 @@ struct DiaDesc {
   int off[kDiaMax] = {};
 };
 
+constexpr int kResidentPolls = 1 << 17;     // about 0.7 us each
+constexpr int kResidentPollsMax = 1 << 20;  // no wait is longer than a second
+
 struct DevCsr {
   int n = 0, m = 0;
   int64_t nnz = 0;
@@ -222,6 +225,9 @@ struct DevCsr {
   // format from the matrix (diagonal, then sliced ELL, then row-block CSR);
   // a fixed one skips the others, for measuring one product kernel.
   int fmt_request = -1;
+  // Polls before a block of a resident solve (grid_krylov.hip) gives up
+  // waiting for the others (0: no such solves).
+  int resident_polls = kResidentPolls;
   void upload(const HostCsr &h, bool want_fp32, bool want_dinv, bool allow_sell = true, bool allow_ell = false);
   // Device value refresh.  v64 (CSR order) is the truth; build_maps (once,
   // from the host pattern) records for every CSR slot its position in the

@@ -222,6 +222,14 @@ class CsrMatrix:
         names = {0: "quad", 1: "rows", 2: "strided", 3: "sorted"}
         return {"fp64": names[g64.value], "fp32": names[g32.value]}
 
+    def set_resident_polls(self, polls: int = -1) -> None:
+        """How often a workgroup of a solve with many iterations per launch
+        (CG and BiCGSTAB, Jacobi or no preconditioner, diagonal storage) polls
+        for the others before the solve goes on with a launch per phase: -1
+        the default (2^17, about 0.1 s), 0 a launch per phase from the start
+        (for a program that keeps the device full with other work)."""
+        N.call("cfdla_matrix_set_resident_polls", self.handle, int(polls))
+
     def diagonal(self):
         d = np.zeros(self.nrows)
         for i in range(self.nrows):

@@ -262,6 +262,16 @@ cfdla_status cfdla_matrix_set_storage(cfdla_matrix m, int32_t format);
  * 32-bit columns. */
 #define CFDLA_GATHER_SORTED 3
 cfdla_status cfdla_matrix_set_gather(cfdla_matrix m, int32_t layout);
+/* CG and BiCGSTAB with a Jacobi (or no) preconditioner on diagonal storage run
+ * many iterations per launch where the rows fit at most half of the device.
+ * The launch's workgroups wait for each other; one that has polled `polls`
+ * times (about 0.7 us each) without the others being there gives up, and the
+ * solve goes on with a launch per phase.  CFDLA_RESIDENT_POLLS_DEFAULT: 2^17,
+ * about 0.1 s.  0: a launch per phase from the start, for a program that keeps
+ * the device full with other work for longer than that, so that every solve
+ * would wait in vain.  At most 2^20.  No reference counterpart. */
+#define CFDLA_RESIDENT_POLLS_DEFAULT (-1)
+cfdla_status cfdla_matrix_set_resident_polls(cfdla_matrix m, int32_t polls);
 /* Layout in use for FP64 and FP32 products (uploads the matrix if needed);
  * CFDLA_GATHER_QUAD for matrices not stored as row-block CSR. */
 cfdla_status cfdla_matrix_gather(cfdla_matrix m, int32_t *layout_fp64, int32_t *layout_fp32);
