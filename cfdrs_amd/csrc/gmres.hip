@@ -23,12 +23,13 @@
 namespace cfdla {
 namespace {
 
-constexpr int kMdotBlocks = 512;
+constexpr int kGramBlocks = 512;  // partials per vector of k_gram
+constexpr int kMdotBlocks = 256;  // and of k_mdot
 
 struct GmLayout {
   int m;
   double *H, *cs, *sn, *g, *y, *hc, *hp, *part;
-  static size_t doubles(int m) { return (size_t)(m + 1) * m + 2 * m + (m + 1) + m + 2 * (m + 1) + (size_t)(m + 1) * kMdotBlocks; }
+  static size_t doubles(int m) { return (size_t)(m + 1) * m + 2 * m + (m + 1) + m + 2 * (m + 1) + (size_t)(m + 1) * kGramBlocks; }
   GmLayout(double *base, int m_) : m(m_) {
     H = base;
     cs = H + (size_t)(m + 1) * m;
@@ -563,28 +564,33 @@ SolveOut gmres(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int64_
     return o;
   }
   const int eb = blocks_for(n, kBlock * 4);
-  const int nb = std::min(kMdotBlocks, blocks_for(n, kBlock));
+  const int gb = std::min(kGramBlocks, blocks_for(n, kBlock));
+  // k_mdot runs this many blocks for every vector, so each takes several rows
+  // per lane: with gb of them a cycle of 256 vectors on 147,456 rows, of which
+  // 87 steps run and the others find the solve done, takes 15.3 ms, with these
+  // 10.5 (262,144 rows: 21.1 and 17.9; FP32 33.0 and 26.3)
+  const int mb = std::min(kMdotBlocks, blocks_for(n, kBlock * 4));
   // Gram-Schmidt over basis vectors 0..j of w.  Up to 32 vectors fit the
   // registers of k_gram (384 x 384 momentum matrix, m = 32: 16.7 us per step on
   // average against 21.6 us in the separate multi-dots and multi-axpys); a
   // longer basis takes those.
   auto gram = [&](int j, T *w, Scal *sc) {
     const int jp1 = j + 1;
-    auto fin = [&](int pass) {
+    auto fin = [&](int pass, int nb) {
       hipLaunchKernelGGL(k_mdot_fin, dim3(jp1), dim3(kBlock), 0, stream(), nb, L.part, L.hp, L.hc, pass == 0 ? 1 : 0,
                          sc);
     };
 #define CFDLA_GRAM(JB)                                                                                                \
   do {                                                                                                                \
-    hipLaunchKernelGGL((k_gram<T, JB, false, true, false>), dim3(nb), dim3(kBlock), 0, stream(), n, jp1, V, ld, L.hp, \
+    hipLaunchKernelGGL((k_gram<T, JB, false, true, false>), dim3(gb), dim3(kBlock), 0, stream(), n, jp1, V, ld, L.hp, \
                        w, sc, L.part);                                                                                \
-    fin(0);                                                                                                           \
-    hipLaunchKernelGGL((k_gram<T, JB, true, true, false>), dim3(nb), dim3(kBlock), 0, stream(), n, jp1, V, ld, L.hp,  \
+    fin(0, gb);                                                                                                       \
+    hipLaunchKernelGGL((k_gram<T, JB, true, true, false>), dim3(gb), dim3(kBlock), 0, stream(), n, jp1, V, ld, L.hp,  \
                        w, sc, L.part);                                                                                \
-    fin(1);                                                                                                           \
-    hipLaunchKernelGGL((k_gram<T, JB, true, false, true>), dim3(nb), dim3(kBlock), 0, stream(), n, jp1, V, ld, L.hp,  \
+    fin(1, gb);                                                                                                       \
+    hipLaunchKernelGGL((k_gram<T, JB, true, false, true>), dim3(gb), dim3(kBlock), 0, stream(), n, jp1, V, ld, L.hp,  \
                        w, sc, ws.current());                                                                          \
-    return nb;                                                                                                        \
+    return gb;                                                                                                        \
   } while (0)
     if (jp1 <= 4) CFDLA_GRAM(4);
     if (jp1 <= 8) CFDLA_GRAM(8);
@@ -593,8 +599,8 @@ SolveOut gmres(const DevCsr &A, Precond *M, const T *b, T *x, double thr, int64_
     if (jp1 <= 32) CFDLA_GRAM(32);
 #undef CFDLA_GRAM
     for (int pass = 0; pass < 2; ++pass) {
-      hipLaunchKernelGGL((k_mdot<T>), dim3(nb, jp1), dim3(kBlock), 0, stream(), n, V, ld, w, L.part, sc);
-      fin(pass);
+      hipLaunchKernelGGL((k_mdot<T>), dim3(mb, jp1), dim3(kBlock), 0, stream(), n, V, ld, w, L.part, sc);
+      fin(pass, mb);
       if (pass == 0)
         hipLaunchKernelGGL((k_maxpy<T, false>), dim3(eb), dim3(kBlock), 0, stream(), n, jp1, V, ld, L.hp, w, sc,
                            nullptr);
