@@ -486,14 +486,33 @@ __global__ __launch_bounds__(kBlock) void k_batch(BArgs A) {
 // a chain of L2 round trips per product: 8.8 us per iteration of a 2,000-row
 // system with two such systems per CU.  A lane's 8 rows of at most 4
 // off-diagonal entries are 64 + 16 VGPRs of FP64 values and 16 of packed LDS
-// offsets; with x, r, p and the Jacobi factors they fit the 256 VGPRs of two
-// wavefronts per SIMD, the residency k_batch had.  The row count per lane R is
-// a template argument picked per system, so a small system neither loops
-// over nor holds rows it does not have, and all gathers of a product are
+// offsets; with x, r, p, z and the Jacobi factors they are 176 of the 256 VGPRs
+// of two wavefronts per SIMD, the residency k_batch had.  The row count per
+// lane R is a template argument picked per system, so a small system neither
+// loops over nor holds rows it does not have, and all gathers of a product are
 // issued together.  Whole calls, against k_batch on the same systems: 4,096
 // networks of 50-2,000 nodes 26.4 -> 8.0 ms, forward and adjoint of 600
-// networks of 30-700 nodes 6.35 -> 2.58 ms.
+// networks of 30-700 nodes 6.35 -> 2.58 ms (one native call each 23.1 -> 3.41
+// and 1.97 -> 0.34 ms).
+//
+// No scratch memory: the runtime allocates it when a queue first runs a kernel
+// that needs some (160 MB for the 304 bytes per lane this kernel once spilled),
+// and cfdla_batch_solve_device_noalloc must not allocate.  Left alone, the
+// compiler forms every row's addresses and unpacked offsets once, ahead of the
+// work queue's and the iterations' loops, and runs out of registers.  pin() has
+// it form them where they are used, at the row counts and precisions that need
+// it, and the scalars that outlive a loop go to scalar registers (scalar()).
+// With scratch and without, one call: the 4,096 networks 3.39 and 3.41 ms (FP32
+// 4.71 and 4.69), 600 of 1,600-2,000 nodes 1.24 and 1.29 (1.81 and 1.74), 600 of
+// 30-700 nodes 0.36 and 0.34 ms (0.52 and 0.46).
 constexpr int kRegOff = 4;  // off-diagonal entries per row
+
+// v, the same in every lane, in scalar registers
+__device__ __forceinline__ double scalar(double v) {
+  const long long b = __builtin_bit_cast(long long, v);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
 
 // Team sums with one barrier each: the two reductions of an iteration use
 // different LDS slots, and at least one other barrier lies between two uses
@@ -534,6 +553,7 @@ struct RegRows {
   __device__ __forceinline__ void load(const BArgs &A, const T *vals, const T *jdv, int r0, int n, int tl) {
 #pragma unroll
     for (int j = 0; j < R; ++j) {
+      if constexpr (sizeof(T) == 8 || R == kRowsPerLane) pin(tl);
       const int i = tl + j * Team::size;
       const bool own = i < n;
       const int row = r0 + (own ? i : 0);
@@ -573,8 +593,12 @@ struct RegRows {
     for (int j = 0; j < R; ++j) {
       T g[kRegOff];
 #pragma unroll
-      for (int k = 0; k < kRegOff; ++k)
-        g[k] = *reinterpret_cast<const T *>(base + ((k & 1) ? c[j][k / 2] >> 16 : c[j][k / 2] & 0xffffu));
+      for (int k = 0; k < kRegOff; k += 2) {
+        unsigned o = c[j][k / 2];
+        if constexpr (sizeof(T) == 8 && R == kRowsPerLane) pin(o);
+        g[k] = *reinterpret_cast<const T *>(base + (o & 0xffffu));
+        g[k + 1] = *reinterpret_cast<const T *>(base + (o >> 16));
+      }
       T s = d[j] * own[j];
 #pragma unroll
       for (int k = 0; k < kRegOff; ++k) s += a[j][k] * g[k];
@@ -604,6 +628,7 @@ __device__ __forceinline__ void reg_solve64(const BArgs &A, int r0, int n, int t
   else same = __all(same ? 1 : 0) != 0;
   iters = 0;
   for (bool first = true;; first = false) {
+    pin(tl);
     // r = b - A x and its equilibrated norm, x gathered through ps
     Team::sync();  // every lane is done with the previous contents of ps
 #pragma unroll
@@ -618,9 +643,9 @@ __device__ __forceinline__ void reg_solve64(const BArgs &A, int r0, int n, int t
       const double e = (i < n ? A.eq[r0 + i] : 0.0) * r[j];
       acc += e * e;
     }
-    rr = reg_sum<Team>(acc, sh);
+    rr = scalar(reg_sum<Team>(acc, sh));
     if (first) {
-      rn0 = sqrt(rr);
+      rn0 = scalar(sqrt(rr));
       term = CFDLA_TERM_INITIAL_RESIDUAL;
       if (rr <= thr2) break;
     } else {
@@ -643,7 +668,7 @@ __device__ __forceinline__ void reg_solve64(const BArgs &A, int r0, int n, int t
       ps[tl + j * Team::size] = p[j];
       rz += r[j] * p[j];
     }
-    rz = reg_sum<Team>(rz, sh);
+    rz = scalar(reg_sum<Team>(rz, sh));
     Team::sync();
     term = CFDLA_TERM_MAX_ITERATIONS;
     while (iters < A.max_it) {
@@ -686,7 +711,7 @@ __device__ __forceinline__ void reg_solve64(const BArgs &A, int r0, int n, int t
         break;
       }
       const double beta = rzn / rz;
-      rz = rzn;
+      rz = scalar(rzn);
 #pragma unroll
       for (int j = 0; j < R; ++j) {
         p[j] = q[j] + beta * p[j];
@@ -749,11 +774,11 @@ __device__ __forceinline__ void reg_solve32(const BArgs &A, int r0, int n, int t
       const double e = eq[j] * r64[j];
       acc += e * e;
     }
-    rr = reg_sum<Team>(acc, sh);
+    rr = scalar(reg_sum<Team>(acc, sh));
     ++nrep;
     bool restart = false;
     if (why == kStart) {
-      rn0 = sqrt(rr);
+      rn0 = scalar(sqrt(rr));
       term = CFDLA_TERM_INITIAL_RESIDUAL;
       if (rr <= thr2) break;
       sc = 1.0 / sqrt(rr);
@@ -851,6 +876,7 @@ __device__ __forceinline__ void reg_solve32(const BArgs &A, int r0, int n, int t
 template <class Team, bool F32>
 __device__ __forceinline__ void solve_system_reg(const BArgs &A, int sys, int tl, double *ps, double *sh) {
   const int r0 = A.sys_row[sys], n = A.sys_row[sys + 1] - r0;
+  if constexpr (!F32) pin(tl);
   double bb = 0.0;
   for (int i = tl; i < n; i += Team::size) {
     const double e = A.eq[r0 + i] * A.b[r0 + i];
@@ -858,7 +884,9 @@ __device__ __forceinline__ void solve_system_reg(const BArgs &A, int sys, int tl
   }
   bb = reg_sum<Team>(bb, sh);
   const double thr = fmax(A.tol_abs, A.tol_rel * sqrt(bb));
-  const double thr2 = thr * thr;
+  const double thr2 = scalar(thr * thr);
+  BatchReport *rep = A.rep + sys;
+  if (tl == 0) rep->thr = thr;
   double rn0 = 0.0, rr = 0.0;
   int iters = 0, outer = 0, term = 0;
   // rows per lane: the same for the whole team
@@ -875,15 +903,12 @@ __device__ __forceinline__ void solve_system_reg(const BArgs &A, int sys, int tl
   else CFDLA_REG(kRowsPerLane);
 #undef CFDLA_REG
   if (tl == 0) {
-    BatchReport rep;
-    rep.iterations = iters;
-    rep.outer = outer;
-    rep.rn0 = rn0;
-    rep.rn = sqrt(rr);
-    rep.thr = thr;
-    rep.term = term;
-    rep.pad = F32 ? 1 : 0;  // the report's precision: 0 FP64, 1 FP32-refined
-    A.rep[sys] = rep;
+    rep->iterations = iters;
+    rep->outer = outer;
+    rep->rn0 = rn0;
+    rep->rn = sqrt(rr);
+    rep->term = term;
+    rep->pad = F32 ? 1 : 0;  // the report's precision: 0 FP64, 1 FP32-refined
   }
 }
 
