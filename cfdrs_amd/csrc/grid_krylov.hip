@@ -12,7 +12,10 @@
 // 262,144 / 524,176 rows 8.6 / 8.8 / 9.5 / 12.5 / 17.3 -> 3.4 / 4.1 / 4.8 / 7.1 /
 // 8.1; BiCGSTAB up to 262,144 rows 18.7 / 19.2 / 20.2 / 27.6 -> 6.5 / 7.3 / 9.5 /
 // 12.1.  Bound by the two (CG) or three exchanges of an iteration.  Larger
-// systems would need every CU or rows that no longer fit the registers.
+// systems would need every CU or rows that no longer fit the registers: the
+// 128 of 1,024 threads hold all of a thread's rows but in FP64 CG with 4 rows
+// (10 spilled with 5 entries per row, 34 with 7) and FP64 BiCGSTAB with 2 rows of
+// 7 entries (8 spilled).
 //
 // Every wait is bounded: a block that does not see the others' sums within
 // DevCsr::resident_polls polls reports it in Scal::pad.  The new iterate and
@@ -425,7 +428,10 @@ __global__ __launch_bounds__(kGridThreads) void k_grid_bicg(DiaRows g, const T *
 // / 131,044 rows, us per iteration with 1, 2 and 4 rows: 4.1, 4.3, 4.3 / 5.4,
 // 4.6, 4.7 / 6.0, 5.7, 4.8 / 6.8, 6.5, 6.1; BiCGSTAB with 1 and 2: 7.3, 7.5 / 9.3,
 // 7.9 / 10.1, 9.5 / 11.7, 11.0.  7 entries in 4 rows no longer fit the registers
-// (32,768 rows: 5.5, 4.6, 7.5), nor do BiCGSTAB's vectors.
+// in FP64 (32,768 rows: 5.5, 4.6, 7.5), nor do BiCGSTAB's vectors, so CG takes 2
+// such rows as long as 128 blocks hold them.  Above, 4 rows still beat a launch
+// per phase: 263,168 / 409,600 / 524,288 rows 10.6 / 10.9 / 11.2 us against 14.2 /
+// 16.0 / 18.4, FP32, where they fit, 7.5 / 7.9 / 8.1 against 15.9 / 18.1 / 17.9.
 int rows_per_thread(int n, int ns, bool bicg) {
   const int most = bicg || (ns > 5 && n <= 2 * kGridThreads * kGridBlocks) ? 2 : 4;
   int rpt = 1;

@@ -118,7 +118,7 @@ typedef struct {
  * interpolation 0 = Classical, 1 = Direct, 2 = SmoothedDirect (prolongator
  * smoothing P = (I - smoothing_omega D^-1 A) P_direct, no reference
  * counterpart); smoother 0 = GaussSeidel, 1 = SymmetricGaussSeidel,
- * 2 = Jacobi (the device V-cycle runs Jacobi only);
+ * 2 = Jacobi (the device V-cycle runs all three, Gauss-Seidel colour by colour);
  * coarse_solver 0 = reference sweeps (pre + 10 smoother sweeps, amg.rs:501),
  * 1 = FP64 dense direct solve. */
 typedef struct {
